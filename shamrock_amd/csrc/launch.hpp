@@ -108,7 +108,9 @@ namespace shamx {
         DevArray<u32> cnt, offset, ids;
         DevArray<u32> lpos;                             // sorted layout: local rows in order
         DevArray<u32> fcnt, fids;                       // force-interacting subsequences
-        DevArray<u32> lflag, lscan, psum;
+        DevArray<u32> lflag, lscan;
+        DevArray<f64> tiers; // 8-ary hierarchy over the leaves (stage 1)
+        DevArray<u32> lap;   // per leaf: a later leaf's box meets its box
         // sorted layout: one pass per stage into rows of fixed capacity; leaf l's list at
         // leaf_ids[l * leaf_stride], row r at ids[r * row_stride] (0: packed layout).  The
         // capacities persist from build to build and grow on overflow.
@@ -124,7 +126,6 @@ namespace shamx {
         u32 n_mismatch = 0;
         DevArray<u32> counters;
         PinnedWords<u32, 16> host; // host copies of counters
-        DevArray<u32> wide_cnt;    // per-thread list counts of the overflow walk
         DevArray<unsigned char> scratch;
     };
     // NeighbourCache::start_neighbors_cache_2stages (NeighbourCache.cpp:222-604).

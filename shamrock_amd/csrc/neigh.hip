@@ -21,22 +21,6 @@
 namespace shamx {
 
     namespace {
-        struct Box {
-            f64 lo[3], hi[3];
-        };
-        __device__ inline Box node_box(const f64 *__restrict rec) {
-            return Box{{rec[0], rec[1], rec[2]}, {rec[3], rec[4], rec[5]}};
-        }
-        // BBAA::cella_neigh_b<f64_3> (geometry_utils.hpp:125-135).  The three comparisons are
-        // combined with & rather than &&: the same value (they have no side effects), without
-        // the branch and exec-mask updates the short-circuit form compiles to in a walk loop.
-        __device__ inline bool cella_neigh_b(const f64 *alo, const f64 *ahi, const f64 *blo,
-                                             const f64 *bhi) {
-            return (fmax(alo[0], blo[0]) <= fmin(ahi[0], bhi[0])) &
-                   (fmax(alo[1], blo[1]) <= fmin(ahi[1], bhi[1])) &
-                   (fmax(alo[2], blo[2]) <= fmin(ahi[2], bhi[2]));
-        }
-
         // orders the LDS accesses of one wave's lanes around this point (LDS executes a wave's
         // operations in issue order; the fences keep the compiler from moving them across)
         __device__ inline void wave_lds_sync() {
@@ -45,317 +29,271 @@ namespace shamx {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
 
-        // Depth-first traversal shared by the 64 lanes of a wave.  The stack lives in lanes
-        // (entry i in lane i: node id, the mask of lanes whose walk reaches it, its two child
-        // ids).  A node is tested before it is pushed, by the lanes of its parent's mask, so
-        // only nodes that some lane enters are pushed, and the two children of a popped node
-        // are loaded and tested together (one dependent load per tree level).  Each lane still
-        // visits exactly the nodes of its own depth-first walk (KarrasTreeTraverser.hpp:69-118,
-        // left child first), in the same order.  crit(rec) is evaluated per lane; found(node)
-        // is called in the lanes whose walk reaches leaf node.  Returns false on stack overflow
-        // or a child id out of range (wave-uniform).
-        template<class Crit, class Found>
-        __device__ inline bool wave_traverse(const f64 *__restrict nodes, u32 I, u32 ncell,
-                                             u64 live, Crit &&crit, Found &&found) {
-            const int lane = __lane_id();
-            u32 st_node = 0, st_lo = 0, st_hi = 0, st_l = 0, st_r = 0; // lane i: entry i
-            int sp      = 0;
-            auto push   = [&](u32 node, u64 mask, u32 cl, u32 cr) { // sp is wave-uniform
-                if (lane == sp) {
-                    st_node = node;
-                    st_lo   = (u32) mask;
-                    st_hi   = (u32) (mask >> 32);
-                    st_l    = cl;
-                    st_r    = cr;
-                }
-                sp++;
-            };
-            // a node record (box, rint, child ids), loaded whole so that the two children's
-            // loads are in flight together
-            struct Rec {
-                f64 v[7];
-                u32 c0, c1;
-            };
-            auto load = [&](u32 node) {
-                const f64 *p = nodes + (u64) node * NODE_F64;
-                Rec r;
-                for (int i = 0; i < 7; i++) r.v[i] = p[i];
-                node_children(nodes, node, r.c0, r.c1);
-                return r;
-            };
-            // lanes of mask that enter the node
-            auto test = [&](const Rec &r, u64 mask) -> u64 {
-                bool pass = ((mask >> lane) & 1ull) && crit(r.v);
-                return __ballot(pass);
-            };
-            {
-                Rec r0 = load(0);
-                u64 pm = test(r0, live);
-                if (pm) push(0, pm, r0.c0, r0.c1);
-            }
-            auto entry_mask = [&](int e) {
-                return (u64) (u32) __builtin_amdgcn_readlane((int) st_lo, e) |
-                       ((u64) (u32) __builtin_amdgcn_readlane((int) st_hi, e) << 32);
-            };
-            while (sp > 0) {
-                u32 node = (u32) __builtin_amdgcn_readlane((int) st_node, sp - 1);
-                u64 mask = entry_mask(sp - 1);
-                if (node >= I) { // a leaf on top: this is its turn in every lane's walk
-                    sp--;
-                    if ((mask >> lane) & 1ull) found(node);
-                    continue;
-                }
-                u32 l = (u32) __builtin_amdgcn_readlane((int) st_l, sp - 1);
-                u32 r = (u32) __builtin_amdgcn_readlane((int) st_r, sp - 1);
-                if (l >= ncell || r >= ncell) return false;
-                // the entry below is expanded in the same step when it is internal too: its
-                // children go under the top entry's, so every walk keeps its order, and four
-                // child records are in flight at once
-                u32 node2 = sp >= 2 ? (u32) __builtin_amdgcn_readlane((int) st_node, sp - 2) : I;
-                if (node2 < I && sp + 2 <= WAVE - 8) {
-                    u64 mask2 = entry_mask(sp - 2);
-                    u32 l2    = (u32) __builtin_amdgcn_readlane((int) st_l, sp - 2);
-                    u32 r2    = (u32) __builtin_amdgcn_readlane((int) st_r, sp - 2);
-                    if (l2 >= ncell || r2 >= ncell) return false;
-                    sp -= 2;
-                    const Rec nl = load(l), nr = load(r), nl2 = load(l2), nr2 = load(r2);
-                    u64 pl = test(nl, mask), pr = test(nr, mask);
-                    u64 pl2 = test(nl2, mask2), pr2 = test(nr2, mask2);
-                    if (pr2) push(r2, pr2, nr2.c0, nr2.c1);
-                    if (pl2) push(l2, pl2, nl2.c0, nl2.c1);
-                    if (pr) push(r, pr, nr.c0, nr.c1);
-                    if (pl) push(l, pl, nl.c0, nl.c1);
-                    continue;
-                }
-                sp--;
-                if (sp + 2 > WAVE) return false;
-                const Rec nl = load(l), nr = load(r);
-                u64 pl = test(nl, mask);
-                u64 pr = test(nr, mask);
-                if (pr) push(r, pr, nr.c0, nr.c1);
-                if (pl) push(l, pl, nl.c0, nl.c1);
-            }
-            return true;
+        // ------------------------------------------------------------- stage 1
+        // A leaf's list (:276-404) holds the leaves n whose box meets its box widened by its
+        // reach, or whose widened box meets its box; the reference finds them by a depth-first
+        // walk of the Karras tree with the same criterion on every cell.  A cell's box and reach
+        // hold those of all leaves below it and the criterion is monotone in both (rounding
+        // included), so a leaf is reached exactly when it passes itself, and left-first order is
+        // the order of the leaf index.  Any search that tests every leaf that can pass, in index
+        // order, therefore gives the reference's list.
+        //
+        // The search runs over tiers: tier 0 are the leaves, cell j of tier t holds the cells
+        // [8 j, 8 j + 8) of tier t - 1 (box and largest rint; same 64-byte records as the tree),
+        // up to a tier of at most 64 cells.  The leaves are in Morton order, so eight of a run
+        // are about one octant, the children of a cell are one contiguous read, and the number of
+        // dependent steps is log8 of the leaf count.
+        constexpr u32 TIER_MAX = 10; // 64 * 8^10 leaves
+        struct Tiers {
+            u32 top;              // index of the top tier
+            u32 n[TIER_MAX + 1];   // cells per tier; n[0] leaves
+            u32 off[TIER_MAX + 1]; // first record of a tier (tier 0: the tree's leaves)
+        };
+        struct Cell {
+            f64 lo[3], hi[3], r;
+        };
+        __device__ inline Cell cell_load(const f64 *__restrict rec) {
+            return Cell{{rec[0], rec[1], rec[2]}, {rec[3], rec[4], rec[5]}, rec[6]};
         }
-
-        // stage 1 count / fill, one lane per leaf, 64 consecutive leaves per wave.
-        // STRIDE: single pass, leaf g owns ids[g * cap, (g + 1) * cap); the count goes on past
-        // cap (entries beyond it are dropped) so the caller can detect the overflow.
-        // LIST: fill only the n_list leaves of list (overflowed ones), each at its offset[g].
-        template<bool FILL, bool STRIDE, bool LIST = false>
-        __global__ void __launch_bounds__(256)
-            k_leaf_neigh_w(u32 L, u32 I, const f64 *__restrict nodes, f64 Rkern,
-                           u32 *__restrict cnt, u32 *__restrict offset, u32 *__restrict ids,
-                           u32 cap, u32 *__restrict err, u32 lpw,
-                           const u32 *__restrict list = nullptr, u32 n_list = 0) {
-            // lpw leaves per wave (64, 32 or 16): fewer leaves give more, shorter walks
-            const u32 lane = (u32) __lane_id();
-            const u32 j = (blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE) * lpw + lane;
-            bool valid  = lane < lpw && j < (LIST ? n_list : L);
-            u32 g       = LIST ? (valid ? list[j] : 0u) : j;
-            u64 live    = __ballot(valid);
-            if (!live) return;
-            const f64 *ra = nodes + (u64) (I + (valid ? g : 0u)) * NODE_F64;
-            f64 rint_a    = ra[6] * Rkern;
-            f64 alo[3] = {ra[0], ra[1], ra[2]}, ahi[3] = {ra[3], ra[4], ra[5]};
-            f64 elo[3] = {alo[0] - rint_a, alo[1] - rint_a, alo[2] - rint_a};
-            f64 ehi[3] = {ahi[0] + rint_a, ahi[1] + rint_a, ahi[2] + rint_a};
-            const u32 c0 = STRIDE ? (valid ? g : 0u) * cap : (FILL && valid ? offset[g] : 0u);
-            const u32 ce = c0 + cap;
-            u32 c        = c0;
-            bool ok      = wave_traverse(
-                nodes, I, I + L, live,
-                [&](const f64 *rec) -> bool {
-                    // STRIDE: a lane whose list is past its capacity stops entering cells (its
-                    // count, then above cap, only flags the overflow; the true count comes
-                    // from the overflow walk), so its wave is not held for the whole list
-                    if (STRIDE && c - c0 > cap) return false;
-                    f64 r      = rec[6] * Rkern;
-                    f64 nlo[3] = {rec[0], rec[1], rec[2]}, nhi[3] = {rec[3], rec[4], rec[5]};
-                    f64 xlo[3] = {nlo[0] - r, nlo[1] - r, nlo[2] - r};
-                    f64 xhi[3] = {nhi[0] + r, nhi[1] + r, nhi[2] + r};
-                    return cella_neigh_b(alo, ahi, xlo, xhi) | cella_neigh_b(elo, ehi, nlo, nhi);
-                },
-                [&](u32 node) {
-                    if (FILL && (!STRIDE || c < ce)) ids[c] = node;
-                    c++;
-                });
-            if (!ok && __lane_id() == __builtin_ctzll(live)) atomicOr(err, 1u);
-            if ((!FILL || STRIDE) && valid) cnt[g] = c - c0;
-            if (STRIDE && valid) offset[g] = c0;
+        constexpr f64 F64_BIG = 1.7976931348623157e308;
+        __device__ inline Cell cell_none() {
+            return Cell{{F64_BIG, F64_BIG, F64_BIG}, {-F64_BIG, -F64_BIG, -F64_BIG}, 0.};
         }
-
-        // The lists longer than their fixed capacity, one listed leaf per block of WIDE_W
-        // waves, its walk spread over the block's threads: the first wave expands the tree
-        // breadth first into an ordered frontier of at least one subtree per thread (or of all
-        // its accepted leaves), then each thread walks a contiguous run of frontier entries
-        // depth first, left child first, with its own stack.  The frontier stays in
-        // left-to-right order and every thread's walk is left-first, so the threads' outputs
-        // in thread order are the leaf's list in the order of the reference's walk.
-        // COUNT pass: each thread's count to tcnt[j * WIDE_T + thread] and the block's total to
-        // cnt[g] (the fixed-capacity pass stops counting past the capacity).  FILL pass: the
-        // same frontier again, the threads' write positions from those counts, each list
-        // walked once more and written at offset[g]; the block's total must equal cnt[g]
-        // (err bit 4 otherwise).  The kernel lasts as long as its longest walk, so a block per
-        // leaf spreads that walk over several waves: 8 for the few long lists of a settled
-        // build, 1 when many leaves pass a capacity set too low (the first build), whose lists
-        // are only a little longer.
-        constexpr int WIDE_ST = 40;
-        template<int WIDE_W, bool COUNT, int WIDE_T = WIDE_W * WAVE, int WIDE_FR = 4 * WIDE_T>
-        __global__ void __launch_bounds__(WIDE_T)
-            k_leaf_walk_wide(u32 L, u32 I, const f64 *__restrict nodes, f64 Rkern,
-                             const u32 *__restrict list, u32 n_list, u32 *__restrict cnt,
-                             u32 *__restrict tcnt, const u32 *__restrict offset,
-                             u32 *__restrict ids, u32 *__restrict err) {
-            __shared__ u32 fr[2][WIDE_FR];
-            __shared__ u32 stk[WIDE_ST][WIDE_T]; // [depth][thread]
-            __shared__ u32 wsum[WIDE_W];
-            __shared__ u32 sh_F, sh_cur;
-            const u32 tid  = threadIdx.x;
-            const u32 lane = (u32) __lane_id();
-            const u32 wv   = tid / WAVE;
-            const u32 j    = blockIdx.x;
-            if (j >= n_list) return; // block-uniform
-            const u32 g     = list[j];
-            const f64 *ra   = nodes + (u64) (I + g) * NODE_F64;
-            const f64 rint_a = ra[6] * Rkern;
-            const f64 alo[3] = {ra[0], ra[1], ra[2]}, ahi[3] = {ra[3], ra[4], ra[5]};
-            const f64 elo[3] = {alo[0] - rint_a, alo[1] - rint_a, alo[2] - rint_a};
-            const f64 ehi[3] = {ahi[0] + rint_a, ahi[1] + rint_a, ahi[2] + rint_a};
-            auto crit = [&](u32 node) {
-                const f64 *rec = nodes + (u64) node * NODE_F64;
-                f64 r      = rec[6] * Rkern;
-                f64 nlo[3] = {rec[0], rec[1], rec[2]}, nhi[3] = {rec[3], rec[4], rec[5]};
-                f64 xlo[3] = {nlo[0] - r, nlo[1] - r, nlo[2] - r};
-                f64 xhi[3] = {nhi[0] + r, nhi[1] + r, nhi[2] + r};
-                return cella_neigh_b(alo, ahi, xlo, xhi) | cella_neigh_b(elo, ehi, nlo, nhi);
-            };
-            const u32 ncell = I + L;
-            constexpr u32 ACC = 0x80000000u; // frontier entry: a leaf already accepted
-            bool bad = false;
-            if (wv == 0) {
-                // breadth-first expansion (wave-uniform control)
-                u32 F = 1, cur = 0;
-                if (lane == 0) fr[0][0] = 0; // the root
-                wave_lds_sync();
-                for (int round = 0;; round++) {
-                    if (round == 128) { // deeper than any tree of these codes: a broken tree
-                        bad = true;
-                        break;
-                    }
-                    u32 total = 0;
-                    bool internal = false, full = false;
-                    for (u32 b = 0; b < F; b += WAVE) {
-                        const u32 e = b + lane;
-                        u32 no = 0, o0 = 0, o1 = 0;
-                        if (e < F) {
-                            const u32 node = fr[cur][e];
-                            if (node & ACC) {
-                                no = 1;
-                                o0 = node;
-                            } else if (node < ncell && crit(node)) {
-                                if (node >= I) {
-                                    no = 1;
-                                    o0 = node | ACC;
-                                } else {
-                                    node_children(nodes, node, o0, o1);
-                                    no = (o0 < ncell && o1 < ncell) ? 2u : 0u;
-                                    bad |= no == 0;
-                                }
-                            }
-                        }
-                        u32 inc = no;
-                        for (int o = 1; o < WAVE; o <<= 1) {
-                            u32 t = __shfl_up(inc, o, WAVE);
-                            if ((int) lane >= o) inc += t;
-                        }
-                        const u32 ct = __shfl(inc, WAVE - 1, WAVE);
-                        if (total + ct > WIDE_FR) {
-                            full = true;
-                            break;
-                        }
-                        const u32 pos = total + inc - no;
-                        if (no >= 1) fr[cur ^ 1][pos] = o0;
-                        if (no == 2) fr[cur ^ 1][pos + 1] = o1;
-                        internal |= __ballot(no == 2) != 0;
-                        total += ct;
-                    }
-                    wave_lds_sync();
-                    if (full) break; // keep the current frontier
-                    cur ^= 1;
-                    F = total;
-                    if (!internal || F >= WIDE_T) break;
-                }
-                if (lane == 0) {
-                    sh_F   = F;
-                    sh_cur = cur;
-                }
+        // union over the lanes whose index differs in the bits o
+        __device__ inline void cell_merge_xor(Cell &c, int o) {
+            for (int k = 0; k < 3; k++) {
+                c.lo[k] = fmin(c.lo[k], __shfl_xor(c.lo[k], o, WAVE));
+                c.hi[k] = fmax(c.hi[k], __shfl_xor(c.hi[k], o, WAVE));
             }
+            c.r = fmax(c.r, __shfl_xor(c.r, o, WAVE));
+        }
+        __device__ inline void cell_store(f64 *__restrict rec, const Cell &c) {
+            for (int k = 0; k < 3; k++) {
+                rec[k]     = c.lo[k];
+                rec[3 + k] = c.hi[k];
+            }
+            rec[6] = c.r;
+            rec[7] = 0.;
+        }
+        // three tiers over the n cells of src in one launch, 512 cells per block (d2, d3: null
+        // when the tiers end below them)
+        constexpr int TIER_BLK = 512;
+        __global__ void __launch_bounds__(TIER_BLK)
+            k_leaf_tiers(u32 n, const f64 *__restrict src, f64 *__restrict d1,
+                         f64 *__restrict d2, f64 *__restrict d3) {
+            __shared__ Cell part[TIER_BLK / WAVE];
+            const u32 i    = blockIdx.x * TIER_BLK + threadIdx.x;
+            const u32 lane = (u32) __lane_id();
+            Cell c         = i < n ? cell_load(src + (u64) i * NODE_F64) : cell_none();
+            for (int o = 1; o < 8; o <<= 1) cell_merge_xor(c, o);
+            if (i < n && i % 8 == 0) cell_store(d1 + (u64) (i / 8) * NODE_F64, c);
+            for (int o = 8; o < WAVE; o <<= 1) cell_merge_xor(c, o);
+            if (d2 && i < n && lane == 0) cell_store(d2 + (u64) (i / 64) * NODE_F64, c);
+            if (!d3) return; // the same for the whole grid
+            if (lane == 0) part[threadIdx.x / WAVE] = c;
             __syncthreads();
-            const u32 F = sh_F, cur = sh_cur;
-            // thread t: entries [t F / WIDE_T, (t + 1) F / WIDE_T) in order, each walked depth
-            // first
-            const u32 b0 = (tid * F) / WIDE_T, b1 = ((tid + 1) * F) / WIDE_T;
-            auto walk = [&](auto emit) {
-                for (u32 e = b0; e < b1; e++) {
-                    const u32 node = fr[cur][e];
-                    if (node & ACC) {
-                        emit(node & ~ACC);
-                        continue;
+            if (threadIdx.x < WAVE) {
+                c = lane < TIER_BLK / WAVE ? part[lane] : cell_none();
+                for (int o = 1; o < TIER_BLK / WAVE; o <<= 1) cell_merge_xor(c, o);
+                if (lane == 0) cell_store(d3 + (u64) blockIdx.x * NODE_F64, c);
+            }
+        }
+
+        // boxes [alo, ahi] and [blo, bhi] meet (BBAA::cella_neigh_b, geometry_utils.hpp:125-135:
+        // max of the lower bounds <= min of the upper ones; a NaN bound never separates, there
+        // as here)
+        __device__ inline bool boxes_meet(const f64 *alo, const f64 *ahi, const f64 *blo,
+                                          const f64 *bhi) {
+            return !((alo[0] > bhi[0]) | (blo[0] > ahi[0]) | (alo[1] > bhi[1]) |
+                     (blo[1] > ahi[1]) | (alo[2] > bhi[2]) | (blo[2] > ahi[2]));
+        }
+
+        // One wave finds the lists of eight consecutive leaves (the targets).  Per tier it keeps a
+        // first-in first-out queue in LDS of the cells that pass the criterion of the targets'
+        // common box, and takes eight cells of one tier at a time, their 64 children in the
+        // lanes; it takes from the lowest tier that has eight, else from the highest that has
+        // any, so a queue never holds more than 8 + 64 entries (tier 0: 64 + 64) and every queue
+        // stays in index order.  Leaves leave tier 0 64 at a time: a lane holds a leaf, the
+        // targets are tested one after the other with the reference's criterion, and a target's
+        // list grows by the lanes of its ballot, in order.
+        //
+        // Eight targets share the search while their common box is tight.  A run of leaves that
+        // crosses a boundary of the Morton curve, or holds one leaf of large reach, has a common
+        // box that meets far more leaves than its members do, so a group is halved while the
+        // halves are cheaper: per leaf met the search costs about 80 lane instructions and each
+        // target 30, so a group of T with box volume V against V1 and V2 of its halves splits
+        // when (80 + 30 T) V > (80 + 15 T) (V1 + V2).
+        //
+        // Bound by instruction issue (Sedov 128^3: 4280 VALU and 2720 scalar instructions per
+        // wave, 54 % of the VALU issue peak, 13 % of wave time waiting).  It replaces a
+        // depth-first walk of the binary tree shared by 64 leaves per wave, a chain of about
+        // 1000 dependent record loads.  Per build: Sedov 128^3 (391 k leaves) 1.39 -> 0.60 ms,
+        // disc of 1 M particles 4.05 -> 0.78 ms, Plummer sphere of 4.2 M 1.53 -> 0.66 ms,
+        // M8 box of 39 k 1.20 -> 0.09 ms, 1,728 particles 0.39 -> 0.04 ms; without the
+        // halving of loose groups the first three take 1.87, 5.8 and 9.4 ms.
+        //
+        // COUNT: list lengths only.  ROWS: leaf g's list at ids[g * cap], at most cap entries
+        // written, the count going on past it.  FILL: at ids[offset[g]].  LIST: the targets
+        // are the leaves of `list`, one per wave.  lap[g] (COUNT and ROWS) says whether a later
+        // leaf's box meets leaf g's box, which is what can make that leaf own one of its
+        // particles.
+        enum LeafOut { LEAF_COUNT, LEAF_ROWS, LEAF_FILL };
+        constexpr int LW_WAVES = 4, LQ_CAP = 128;
+        constexpr u32 LEAF_TGT = 8;
+        template<int OUT, bool LIST>
+        __global__ void __launch_bounds__(LW_WAVES *WAVE)
+            k_leaf_lists(u32 L, u32 I, const f64 *__restrict nodes, const f64 *__restrict tiers,
+                         Tiers tt, f64 Rkern, u32 *__restrict cnt, u32 *__restrict offset,
+                         u32 *__restrict ids, u32 cap, u32 *__restrict lap,
+                         const u32 *__restrict list, u32 n_list) {
+            constexpr u32 T = LIST ? 1 : LEAF_TGT;
+            __shared__ u32 queue[LW_WAVES][TIER_MAX + 1][LQ_CAP];
+            __shared__ f64 tgt[LW_WAVES][T][12]; // box and widened box of every target
+            const u32 lane = (u32) __lane_id();
+            const u32 wid  = (u32) __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
+            const u32 item = blockIdx.x * LW_WAVES + wid;
+            if (item >= (LIST ? n_list : (L + T - 1) / T)) return;
+            const u32 g0 =
+                LIST ? (u32) __builtin_amdgcn_readfirstlane((int) list[item]) : item * T;
+            const u32 nt = LIST ? 1u : min(T, L - g0);
+            const u64 lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+            u32(*q)[LQ_CAP] = queue[wid];
+            auto at = [](u32 v, u32 l) { return (u32) __builtin_amdgcn_readlane((int) v, (int) l); };
+            // lane t (< nt): target t, its list's length and first entry, the size of the group
+            // that it is searched in
+            u32 len = 0, base = 0, laps = 0, size = T;
+            {
+                Cell wide = cell_none();
+                if (lane < nt) {
+                    const Cell c = cell_load(nodes + (u64) (I + g0 + lane) * NODE_F64);
+                    const f64 r  = c.r * Rkern;
+                    f64 *m       = tgt[wid][lane];
+                    for (int k = 0; k < 3; k++) {
+                        wide.lo[k] = c.lo[k] - r;
+                        wide.hi[k] = c.hi[k] + r;
+                        m[k]       = c.lo[k];
+                        m[3 + k]   = c.hi[k];
+                        m[6 + k]   = wide.lo[k];
+                        m[9 + k]   = wide.hi[k];
                     }
-                    int sp            = 0;
-                    stk[sp++][tid]    = node;
-                    while (sp > 0) {
-                        const u32 nd = stk[--sp][tid];
-                        if (nd >= ncell || !crit(nd)) continue;
-                        if (nd >= I) {
-                            emit(nd);
-                            continue;
-                        }
-                        u32 cl, cr;
-                        node_children(nodes, nd, cl, cr);
-                        if (sp + 2 > WIDE_ST) {
-                            bad = true;
-                            break;
-                        }
-                        stk[sp++][tid] = cr; // the left child is popped first
-                        stk[sp++][tid] = cl;
+                    if (OUT == LEAF_ROWS) base = (g0 + lane) * cap;
+                    if (OUT == LEAF_FILL) base = offset[g0 + lane];
+                }
+                if (!LIST) {
+                    auto vol = [](const Cell &c) {
+                        f64 v = 1;
+                        for (int k = 0; k < 3; k++) v *= fmax(c.hi[k] - c.lo[k], 0.);
+                        return v;
+                    };
+                    f64 v = vol(wide);
+                    bool split[3];
+#pragma unroll
+                    for (int b = 0; b < 3; b++) { // groups of 2, 4, 8
+                        const f64 parts = v + __shfl_xor(v, 1 << b, WAVE);
+                        cell_merge_xor(wide, 1 << b);
+                        v           = vol(wide);
+                        const f64 t = (f64) (2 << b);
+                        split[b]    = (80. + 30. * t) * v > (80. + 15. * t) * parts;
                     }
+                    for (int b = 2; b >= 0 && split[b]; b--) size = 1u << b;
+                }
+            }
+            // queue state of tier t in lane t: entries and position of the first
+            u32 qn = 0, qh = 0;
+            f64 ulo[3], uhi[3], elo[3], ehi[3]; // the group's common box and widened box
+            // the cells of tier t in the lanes (on: this lane has one) that pass for the group
+            // go to the tier's queue
+            auto sift = [&](u32 t, u32 cell, bool on) {
+                bool pass = false;
+                if (on) {
+                    const f64 *rec = t ? tiers + (u64) (tt.off[t] + cell) * NODE_F64
+                                       : nodes + (u64) (I + cell) * NODE_F64;
+                    const Cell b   = cell_load(rec);
+                    const f64 r    = b.r * Rkern;
+                    const f64 xlo[3] = {b.lo[0] - r, b.lo[1] - r, b.lo[2] - r};
+                    const f64 xhi[3] = {b.hi[0] + r, b.hi[1] + r, b.hi[2] + r};
+                    pass = boxes_meet(ulo, uhi, xlo, xhi) | boxes_meet(elo, ehi, b.lo, b.hi);
+                }
+                const u64 m = __ballot(pass);
+                const u32 p = at(qh + qn, t);
+                if (pass) q[t][(p + (u32) __popcll(m & lt)) % LQ_CAP] = cell;
+                if (lane == t) qn += (u32) __popcll(m);
+                wave_lds_sync();
+            };
+            // up to 64 leaves of tier 0 against the targets [t0, t1)
+            auto leaves = [&](u32 t0, u32 t1) {
+                const u32 n   = min(at(qn, 0), (u32) WAVE);
+                const u32 h0  = at(qh, 0);
+                const bool on = lane < n;
+                const u32 g   = on ? q[0][(h0 + lane) % LQ_CAP] : 0u;
+                if (lane == 0) qh += n, qn -= n;
+                const Cell b = cell_load(nodes + (u64) (I + g) * NODE_F64);
+                const f64 r  = b.r * Rkern;
+                const f64 xlo[3] = {b.lo[0] - r, b.lo[1] - r, b.lo[2] - r};
+                const f64 xhi[3] = {b.hi[0] + r, b.hi[1] + r, b.hi[2] + r};
+                const bool later =
+                    OUT != LEAF_FILL &&
+                    __ballot(on & (g > g0 + t0) & boxes_meet(ulo, uhi, b.lo, b.hi)) != 0;
+                for (u32 t = t0; t < t1; t++) {
+                    const f64 *a = tgt[wid][t];
+                    const bool pass =
+                        on & (boxes_meet(a, a + 3, xlo, xhi) | boxes_meet(a + 6, a + 9, b.lo, b.hi));
+                    const u64 m = __ballot(pass);
+                    if (OUT != LEAF_COUNT && pass) {
+                        const u32 p = at(len, t) + (u32) __popcll(m & lt);
+                        if (OUT == LEAF_FILL || p < cap) ids[at(base, t) + p] = I + g;
+                    }
+                    if (lane == t) len += (u32) __popcll(m);
+                    if (later && __ballot(on & (g > g0 + t) & boxes_meet(a, a + 3, b.lo, b.hi)))
+                        laps |= 1u << t;
                 }
             };
-            u32 c = 0;
-            if constexpr (COUNT) {
-                walk([&](u32) { c++; });
-                tcnt[(u64) j * WIDE_T + tid] = c;
-            } else {
-                c = tcnt[(u64) j * WIDE_T + tid];
-            }
-            // block-wide exclusive scan of the counts
-            u32 inc = c;
-            for (int o = 1; o < WAVE; o <<= 1) {
-                u32 t = __shfl_up(inc, o, WAVE);
-                if ((int) lane >= o) inc += t;
-            }
-            if (lane == WAVE - 1) wsum[wv] = inc;
-            const bool block_bad = __syncthreads_or(bad);
-            u32 before = 0, tot = 0;
-            for (u32 w = 0; w < (u32) WIDE_W; w++) {
-                if (w < wv) before += wsum[w];
-                tot += wsum[w];
-            }
-            if (COUNT) {
-                if (tid == 0) {
-                    if (block_bad) atomicOr(err, 1u);
-                    else cnt[g] = tot;
+            wave_lds_sync();
+            for (u32 t0 = 0, t1; t0 < nt; t0 = t1) {
+                const u32 sz = at(size, t0);
+                t1           = min(t0 + sz, nt);
+                for (int k = 0; k < 3; k++) {
+                    ulo[k] = elo[k] = F64_BIG;
+                    uhi[k] = ehi[k] = -F64_BIG;
                 }
-                return;
+                for (u32 t = t0; t < t1; t++) {
+                    const f64 *m = tgt[wid][t];
+                    for (int k = 0; k < 3; k++) {
+                        ulo[k] = fmin(ulo[k], m[k]);
+                        uhi[k] = fmax(uhi[k], m[3 + k]);
+                        elo[k] = fmin(elo[k], m[6 + k]);
+                        ehi[k] = fmax(ehi[k], m[9 + k]);
+                    }
+                }
+                u32 t = tt.top, cell = lane;
+                bool on = lane < tt.n[tt.top];
+                for (;;) {
+                    sift(t, cell, on);
+                    u64 some;
+                    for (;;) {
+                        some = __ballot(qn > 0);
+                        // 64 leaves, or the last ones
+                        if (at(qn, 0) < (u32) WAVE && some != 1ull) break;
+                        leaves(t0, t1);
+                    }
+                    if (!some) break;
+                    const u64 eight = __ballot(qn >= 8) & ~1ull;
+                    const u32 f     = eight ? (u32) __builtin_ctzll(eight)
+                                            : 63u - (u32) __builtin_clzll(some);
+                    const u32 k     = min(at(qn, f), 8u);
+                    const u32 h0    = at(qh, f);
+                    if (lane == f) qh += k, qn -= k;
+                    const u32 slot = lane / 8;
+                    cell           = q[f][(h0 + slot) % LQ_CAP] * 8 + lane % 8;
+                    t              = f - 1;
+                    on             = (slot < k) & (cell < tt.n[t]);
+                }
             }
-            if (block_bad || tot != cnt[g]) {
-                if (tid == 0) atomicOr(err, block_bad ? 1u : 4u);
-                return;
+            if (OUT != LEAF_FILL && lane < nt) {
+                cnt[g0 + lane] = len;
+                lap[g0 + lane] = (laps >> lane) & 1u;
+                if (OUT == LEAF_ROWS) offset[g0 + lane] = base;
             }
-            u32 pos = offset[g] + before + inc - c;
-            walk([&](u32 nd) { ids[pos++] = nd; });
         }
 
         // rows (leaf lists or particle rows) longer than their fixed capacity: flag and count
@@ -379,30 +317,52 @@ namespace shamx {
             offset[i]     = base + opos[i];
         }
 
-        // owner leaf, lanes over sorted positions (spatially coherent waves)
+        // Owner leaf (:406-451) of every local particle, OWN_LANES lanes per member batch (64
+        // sorted positions of a leaf).  The particle's own leaf contains it, so its owner is the
+        // last leaf of the own leaf's list whose box contains it (a leaf that contains a
+        // particle of this one meets its box and is in its list); leaves whose box no later leaf
+        // meets (lap) own all their particles.  Particles owned by another leaf go to mism, and
+        // lflag (sorted layout) marks the local ones.  leaf_cap: as in stage 2.
+        constexpr u32 OWN_LANES = 16;
         __global__ void __launch_bounds__(256)
-            k_owner_w(u32 nm, u32 n, u32 I, const f64 *__restrict nodes,
-                      const u32 *__restrict sort_index, const double4 *__restrict ps, u32 L,
-                      u32 *__restrict owner, u32 *__restrict err) {
-            u32 s      = blockIdx.x * blockDim.x + threadIdx.x;
-            u32 a      = s < nm ? sort_index[s] : 0xffffffffu;
-            bool valid = a < n;
-            u64 live   = __ballot(valid);
-            if (!live) return;
-            double4 q = ps[valid ? s : 0u];
-            f64 p[3]  = {q.x, q.y, q.z};
-            u32 found = 0x7fffffffu;
-            bool ok   = wave_traverse(
-                nodes, I, I + L, live,
-                [&](const f64 *rec) { // is_coord_in_range_incl_max (geometry_utils.hpp:74-81)
-                    return (rec[0] <= p[0]) & (p[0] <= rec[3]) & (rec[1] <= p[1]) &
-                           (p[1] <= rec[4]) & (rec[2] <= p[2]) & (p[2] <= rec[5]);
-                },
-                [&](u32 node) { found = node - I; });
-            if (!ok && __lane_id() == __builtin_ctzll(live)) atomicOr(err, 1u);
-            if (valid) {
-                if (found >= L) atomicOr(err, 2u);
-                owner[a] = (found < L) ? found : 0u;
+            k_owner(u32 n, u32 I, const f64 *__restrict nodes, const u32 *__restrict item_leaf,
+                    const u32 *__restrict bstart, const u32 *__restrict n_items,
+                    const u32 *__restrict sort_index, const double4 *__restrict ps,
+                    const u32 *__restrict lap, const u32 *__restrict leaf_cnt,
+                    const u32 *__restrict leaf_offset, const u32 *__restrict leaf_ids,
+                    u32 leaf_cap, u32 *__restrict owner, u32 *__restrict lflag,
+                    u32 *__restrict mism, u32 *__restrict mism_len) {
+            const u32 item = (blockIdx.x * 256 + threadIdx.x) / OWN_LANES;
+            if (item >= *n_items) return;
+            const u32 l = item_leaf[item];
+            u32 m0, m1;
+            node_children(nodes, I + l, m0, m1);
+            m0 += (item - bstart[l]) * WAVE;
+            m1 = min(m1, m0 + WAVE);
+            const bool over = lap[l] != 0;
+            for (u32 s = m0 + threadIdx.x % OWN_LANES; s < m1; s += OWN_LANES) {
+                const u32 a = sort_index[s];
+                if (lflag) lflag[s] = a < n ? 1u : 0u;
+                if (a >= n) continue;
+                u32 own = l;
+                if (over) {
+                    const double4 p = ps[s];
+                    const u32 k0    = leaf_offset[l];
+                    u32 k = k0 + (leaf_cap ? min(leaf_cnt[l], leaf_cap) : leaf_cnt[l]);
+                    while (k > k0) {
+                        const u32 nd = leaf_ids[--k];
+                        if (nd <= I + l) break;
+                        const f64 *rec = nodes + (u64) nd * NODE_F64;
+                        // is_coord_in_range_incl_max (geometry_utils.hpp:74-81)
+                        if ((rec[0] <= p.x) & (p.x <= rec[3]) & (rec[1] <= p.y) &
+                            (p.y <= rec[4]) & (rec[2] <= p.z) & (p.z <= rec[5])) {
+                            own = nd - I;
+                            break;
+                        }
+                    }
+                }
+                owner[a] = own;
+                if (own != l) mism[atomicAdd(mism_len, 1u)] = a;
             }
         }
 
@@ -456,48 +416,28 @@ namespace shamx {
         }
 
         // sorted copy of positions and h (AoS, 32 B per object) + inverse permutation
-        __global__ void k_sorted_copy(u32 nm, const u32 *__restrict sort_index,
+        // (a local particle with a NaN coordinate is inside no leaf box: err bit 2)
+        __global__ void k_sorted_copy(u32 nm, u32 n, const u32 *__restrict sort_index,
                                       const f64 *__restrict x, const f64 *__restrict y,
                                       const f64 *__restrict z, const f64 *__restrict h,
-                                      double4 *__restrict ps, u32 *__restrict inv) {
+                                      double4 *__restrict ps, u32 *__restrict inv,
+                                      u32 *__restrict err) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
             if (s >= nm) return;
-            u32 b  = sort_index[s];
-            ps[s]  = make_double4(x[b], y[b], z[b], h[b]);
-            inv[b] = s;
+            u32 b           = sort_index[s];
+            const double4 q = make_double4(x[b], y[b], z[b], h[b]);
+            ps[s]           = q;
+            inv[b]          = s;
+            if ((b < n) & ((q.x != q.x) | (q.y != q.y) | (q.z != q.z))) atomicOr(err, 2u);
         }
 
-        // particles whose owner leaf is not the leaf holding them go to the per-particle path
-        __global__ void k_mismatch(u32 n, u32 I, const f64 *__restrict nodes,
-                                   const u32 *__restrict owner, const u32 *__restrict inv,
-                                   u32 *__restrict list, u32 *__restrict list_len) {
-            u32 a = blockIdx.x * blockDim.x + threadIdx.x;
-            if (a >= n) return;
-            u32 s0, s1;
-            node_children(nodes, I + owner[a], s0, s1);
-            u32 sa = inv[a];
-            if (!(s0 <= sa && sa < s1)) list[atomicAdd(list_len, 1u)] = a;
-        }
-
-        // local particles in sorted order: flag, then scatter after the scan
-        __global__ void k_local_flag(u32 nm, u32 n, const u32 *__restrict sort_index,
-                                     u32 *__restrict flag) {
-            u32 s = blockIdx.x * blockDim.x + threadIdx.x;
-            if (s < nm) flag[s] = sort_index[s] < n ? 1u : 0u;
-        }
+        // local particles in sorted order, scattered after the scan of their flags
         __global__ void k_local_scatter(u32 nm, const u32 *__restrict flag,
                                         const u32 *__restrict pos, u32 *__restrict lpos) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
             if (s < nm && flag[s]) lpos[pos[s]] = s;
         }
 
-
-        __device__ inline f64 wave_bcast(f64 v, int lane) {
-            i64 b  = __double_as_longlong(v);
-            int lo = __builtin_amdgcn_readlane((int) (b & 0xffffffff), lane);
-            int hi = __builtin_amdgcn_readlane((int) (b >> 32), lane);
-            return __longlong_as_double(((i64) hi << 32) | (u32) lo);
-        }
 
         constexpr int GRP_WAVES = 4;
 
@@ -829,6 +769,78 @@ namespace shamx {
             if (n) k_max_u32<<<std::min<u32>(div_up(n, 256), 256), 256, 0, s>>>(n, v, out);
         }
 
+        // out += {max of cnt[0, n), sum, number of rows longer than cap, their entries} (device;
+        // the four words must start at 0)
+        __global__ void __launch_bounds__(256)
+            k_row_stats(u32 n, const u32 *__restrict cnt, u32 cap, u32 *__restrict mx,
+                        u32 *__restrict tot, u32 *__restrict over) {
+            __shared__ u32 lds[4][256 / WAVE];
+            u32 v[4] = {0, 0, 0, 0};
+            for (u32 i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+                const u32 c = cnt[i];
+                const bool o = c > cap;
+                v[0]         = max(v[0], c);
+                v[1] += c;
+                v[2] += o ? 1u : 0u;
+                v[3] += o ? c : 0u;
+            }
+            v[0] = wave_reduce(v[0], [](u32 p, u32 q) { return p > q ? p : q; });
+            for (int k = 1; k < 4; k++) v[k] = wave_reduce(v[k], [](u32 p, u32 q) { return p + q; });
+            if (__lane_id() == 0)
+                for (int k = 0; k < 4; k++) lds[k][threadIdx.x / WAVE] = v[k];
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                for (int w = 1; w < 256 / WAVE; w++) {
+                    v[0] = max(v[0], lds[0][w]);
+                    for (int k = 1; k < 4; k++) v[k] += lds[k][w];
+                }
+                atomicMax(mx, v[0]);
+                if (v[1]) atomicAdd(tot, v[1]);
+                if (v[2]) {
+                    atomicAdd(over, v[2]);
+                    atomicAdd(over + 1, v[3]);
+                }
+            }
+        }
+        void row_stats(hipStream_t s, u32 n, const u32 *cnt, u32 cap, u32 *mx, u32 *tot,
+                       u32 *over) {
+            if (n)
+                k_row_stats<<<std::min<u32>(div_up(n, 1024), 512), 256, 0, s>>>(n, cnt, cap, mx,
+                                                                                tot, over);
+        }
+
+        // the tiers over the leaves for the searches of stage 1
+        Tiers build_tiers(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t) {
+            Tiers tt{};
+            tt.n[0] = t.L;
+            u32 at  = 0;
+            while (tt.n[tt.top] > (u32) WAVE) {
+                const u32 k = tt.top + 1; // at most 10 for a u32 leaf count
+                tt.n[k]     = div_up(tt.n[k - 1], 8);
+                tt.off[k]   = at;
+                at += tt.n[k];
+                tt.top = k;
+            }
+            nb.tiers.resize(std::max<size_t>((size_t) at * NODE_F64, 1));
+            auto rec = [&](u32 k) -> f64 * {
+                return k <= tt.top ? nb.tiers.data() + (size_t) tt.off[k] * NODE_F64 : nullptr;
+            };
+            for (u32 k = 0; k < tt.top; k += 3)
+                k_leaf_tiers<<<div_up(tt.n[k], TIER_BLK), TIER_BLK, 0, s>>>(
+                    tt.n[k], k ? rec(k) : t.nodes.data() + (size_t) t.I * NODE_F64, rec(k + 1),
+                    rec(k + 2), rec(k + 3));
+            return tt;
+        }
+        // lists of all leaves, eight per wave
+        template<int OUT>
+        void leaf_lists(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, const Tiers &tt,
+                        f64 Rkern, u32 cap) {
+            k_leaf_lists<OUT, false>
+                <<<div_up(div_up(t.L, LEAF_TGT), LW_WAVES), LW_WAVES * WAVE, 0, s>>>(
+                    t.L, t.I, t.nodes.data(), nb.tiers.data(), tt, Rkern, nb.leaf_cnt.data(),
+                    nb.leaf_offset.data(), nb.leaf_ids.data(), cap, nb.lap.data(), nullptr, 0);
+        }
+
         // the stage-2 wave items (one per 64 sorted positions of every leaf): item -> leaf map,
         // first item of every leaf, item count at counters[7]; returns the launch's block
         // count, sized for the bound L + nm / 64 (waves past the count return at once)
@@ -846,13 +858,19 @@ namespace shamx {
             return div_up(bound, (u32) GRP_WAVES);
         }
 
-        // error flags of the walks (counters[4]) into exceptions
-        void check_walk_flags(u32 f) {
-            if (f & 1u) throw std::runtime_error("neighbour cache: tree traversal stack overflow");
+        // error flags (counters[4]) into exceptions
+        void check_flags(u32 f) {
             if (f & 2u)
                 throw std::runtime_error("neighbour cache: a particle is outside every leaf box");
-            if (f & 4u)
-                throw std::runtime_error("neighbour cache: a leaf walk disagrees with its count");
+        }
+        // owner leaves, mismatch list and (sorted layout) local flags, on complete leaf lists
+        void owners(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, u32 n_local,
+                    u32 gblocks, u32 leaf_cap, u32 *lflag) {
+            k_owner<<<div_up((u64) gblocks * GRP_WAVES * OWN_LANES, 256), 256, 0, s>>>(
+                n_local, t.I, t.nodes.data(), nb.item_leaf.data(), nb.bstart.data(),
+                nb.counters.data() + 7, t.sort_index.data(), nb.ps.data(), nb.lap.data(),
+                nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(), leaf_cap,
+                nb.owner.data(), lflag, nb.mism.data(), nb.counters.data() + 5);
         }
 
         // boxes of the member batches for the batch-level cull of stage 2, on sets whose tree
@@ -883,12 +901,11 @@ namespace shamx {
         // (leaf_cap: capacity of fixed-capacity leaf lists, 0 for packed ones)
         template<bool SORTED>
         void stage2_packed(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, u32 n_local,
-                           const f64 *x, const f64 *y, const f64 *z, const f64 *h, f64 htol,
-                           f64 Rker2, u32 *hc, u32 leaf_cap = 0) {
+                           u32 gblocks, const f64 *x, const f64 *y, const f64 *z, const f64 *h,
+                           f64 htol, f64 Rker2, u32 *hc, u32 leaf_cap = 0) {
             u32 L = t.L, I = t.I;
             u32 rows      = SORTED ? t.n_obj : n_local;
-            u32 *mism_len = nb.counters.data() + 5;
-            u32 gblocks   = batch_items(s, nb, t);
+            u32 *mism_len      = nb.counters.data() + 5;
             const u32 *n_items = nb.counters.data() + 7;
             if (SORTED) fill_u32(s, nb.cnt.data(), 0, rows); // ghost rows stay empty
             const f64 *bb = batch_boxes(s, nb, t, gblocks, htol, Rker2);
@@ -911,7 +928,7 @@ namespace shamx {
             SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
                                      hipMemcpyDeviceToHost, s));
             SHAMX_HIP(hipStreamSynchronize(s));
-            check_walk_flags(hc[4]);
+            check_flags(hc[4]);
             nb.n_pairs    = hc[1];
             nb.n_mismatch = hc[5];
             nb.ids.resize(std::max<u64>(nb.n_pairs, 1));
@@ -925,16 +942,6 @@ namespace shamx {
                 nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(), x,
                 y, z, h, nb.inv.data(), htol, Rker2, nullptr, nb.offset.data(), nb.ids.data(), 0,
                 leaf_cap);
-        }
-
-        // leaves per wave in the stage-1 walk (SHAMX_LEAF_LANES: 64, 32 or 16)
-        u32 leaf_lanes() {
-            static const u32 v = [] {
-                const char *e = std::getenv("SHAMX_LEAF_LANES");
-                int x         = e ? std::atoi(e) : 64;
-                return (u32) ((x == 16 || x == 32) ? x : 64);
-            }();
-            return v;
         }
 
         // SHAMX_NEIGH_ROWS=packed (read at every build) takes packed particle rows even where
@@ -961,72 +968,64 @@ namespace shamx {
                                     scan_scratch_bytes(nm)}));
         nb.leaf_cnt.resize(L);
         nb.leaf_offset.resize(L);
+        nb.lap.resize(L);
         nb.owner.resize(std::max<u32>(n_local, 1));
         nb.cnt.resize(std::max<u32>(rows, 1));
         nb.offset.resize(std::max<u32>(rows, 1));
-        nb.psum.resize(std::max<u32>(std::max(rows, L), 1));
         u32 *err = nb.counters.data() + 4;
         fill_u32(s, nb.counters.data(), 0, 16);
         f64 Rker2 = Rkern * Rkern;
         u32 *hc = nb.host.data(); // 16 pinned words: the reads queue on the stream
 
-        // sorted copy and inverse permutation (independent of the leaf lists)
+        // sorted copy and inverse permutation, member batches, tiers over the leaves
         nb.ps.resize(nm);
         nb.inv.resize(nm);
         nb.mism.resize(std::max<u32>(n_local, 1));
-        k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, t.sort_index.data(), x, y, z, h,
-                                                      nb.ps.data(), nb.inv.data());
+        k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, t.sort_index.data(), x, y, z,
+                                                      h, nb.ps.data(), nb.inv.data(), err);
+        const u32 gblocks = batch_items(s, nb, t);
+        const Tiers tt    = build_tiers(s, nb, t);
 
-        if (!sorted_layout) {
-            // reference layout: stage 1 in two passes
-            k_leaf_neigh_w<false, false><<<div_up(L, 256), 256, 0, s>>>(
-                L, I, t.nodes.data(), Rkern, nb.leaf_cnt.data(), nullptr, nullptr, 0, err, 64);
+        // leaf lists in two passes (count, scan, fill); returns once their length is known
+        auto packed_leaves = [&] {
+            leaf_lists<LEAF_COUNT>(s, nb, t, tt, Rkern, 0);
             exclusive_scan_u32(s, nb.leaf_cnt.data(), nb.leaf_offset.data(), L,
                                nb.counters.data(), nb.scratch.data());
             SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 8 * sizeof(u32),
                                      hipMemcpyDeviceToHost, s));
             SHAMX_HIP(hipStreamSynchronize(s));
             tree_check(t);
-            if (hc[4]) throw std::runtime_error("neighbour cache: tree traversal stack overflow");
             nb.n_leaf_pairs = hc[0];
-            nb.leaf_stride  = 0;
             nb.leaf_ids.resize(std::max<u64>(nb.n_leaf_pairs, 1));
-            k_leaf_neigh_w<true, false><<<div_up(L, 256), 256, 0, s>>>(
-                L, I, t.nodes.data(), Rkern, nullptr, nb.leaf_offset.data(), nb.leaf_ids.data(),
-                0, err, 64);
+            leaf_lists<LEAF_FILL>(s, nb, t, tt, Rkern, 0);
+        };
+
+        if (!sorted_layout) {
+            // reference layout
+            packed_leaves();
+            nb.leaf_stride = 0;
             if (n_local == 0) {
                 nb.n_pairs = 0;
                 return;
             }
-            k_owner_w<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, I, t.nodes.data(),
-                                                      t.sort_index.data(), nb.ps.data(), L,
-                                                      nb.owner.data(), err);
-            k_mismatch<<<div_up(n_local, 256), 256, 0, s>>>(n_local, I, t.nodes.data(),
-                                                            nb.owner.data(), nb.inv.data(),
-                                                            nb.mism.data(),
-                                                            nb.counters.data() + 5);
-            stage2_packed<false>(s, nb, t, n_local, x, y, z, h, htol, Rker2, hc);
+            owners(s, nb, t, n_local, gblocks, 0, nullptr);
+            stage2_packed<false>(s, nb, t, n_local, gblocks, x, y, z, h, htol, Rker2, hc);
             nb.row_stride = 0;
             SHAMX_HIP(hipGetLastError());
             return;
         }
 
-        // sorted layout: owner leaves, mismatch list, local rows in sorted order
-        k_owner_w<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, I, t.nodes.data(),
-                                                  t.sort_index.data(), nb.ps.data(), L,
-                                                  nb.owner.data(), err);
-        k_mismatch<<<div_up(n_local, 256), 256, 0, s>>>(n_local, I, t.nodes.data(),
-                                                        nb.owner.data(), nb.inv.data(),
-                                                        nb.mism.data(), nb.counters.data() + 5);
+        // sorted layout: with the owners, the local rows in sorted order
         nb.lflag.resize(nm);
         nb.lscan.resize(nm);
         nb.lpos.resize(std::max<u32>(n_local, 1));
-        k_local_flag<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, t.sort_index.data(),
-                                                     nb.lflag.data());
-        exclusive_scan_u32(s, nb.lflag.data(), nb.lscan.data(), nm, nb.counters.data() + 6,
-                           nb.scratch.data());
-        k_local_scatter<<<div_up(nm, 256), 256, 0, s>>>(nm, nb.lflag.data(), nb.lscan.data(),
-                                                        nb.lpos.data());
+        auto own_leaves = [&](u32 leaf_cap) {
+            owners(s, nb, t, n_local, gblocks, leaf_cap, nb.lflag.data());
+            exclusive_scan_u32(s, nb.lflag.data(), nb.lscan.data(), nm, nb.counters.data() + 6,
+                               nb.scratch.data());
+            k_local_scatter<<<div_up(nm, 256), 256, 0, s>>>(nm, nb.lflag.data(),
+                                                            nb.lscan.data(), nb.lpos.data());
+        };
 
         // Both stages in one pass each, rows of fixed capacity, chosen from the previous build
         // (about four times the mean length, at most the longest row plus headroom).  Rows
@@ -1036,7 +1035,6 @@ namespace shamx {
         // must be complete before stage 2 reads them: once a build has seen leaf overflow,
         // the next ones resolve it between the stages (one more host sync); the first time, the
         // build is repeated.
-        const u32 gblocks = batch_items(s, nb, t);
         // capacity for rows of measured longest `mx` and total `tot` over `rows_` rows, at most
         // what u32 entry indices address for rows_ rows (a multiple of 16: 64-byte rows)
         auto fit = [](u32 rows_, u32 cap) {
@@ -1055,82 +1053,45 @@ namespace shamx {
         u32 *mism_len = nb.counters.data() + 5;
         const u32 big = std::max(L, nm);
         for (auto *a_ : {&nb.oflag, &nb.ocnt, &nb.ofpos, &nb.opos, &nb.olist}) a_->resize(big);
-        // list the rows of cnt[0, n) longer than cap: count at counters[c], total at c + 1
-        auto mark = [&](u32 n, const u32 *cnt, u32 cap, int c) {
+        // list the rows of cnt[0, n) longer than cap (map: their labels) with their offsets
+        // from `base` on, where the host knows that there are some
+        auto list_over = [&](u32 n, const u32 *cnt, u32 cap, u64 base, const u32 *map,
+                             u32 *offset) {
             k_over_mark<<<div_up(n, 256), 256, 0, s>>>(n, cnt, cap, nb.oflag.data(),
                                                         nb.ocnt.data());
-            exclusive_scan_u32(s, nb.oflag.data(), nb.ofpos.data(), n, nb.counters.data() + c,
+            exclusive_scan_u32(s, nb.oflag.data(), nb.ofpos.data(), n, nullptr,
                                nb.scratch.data());
-            exclusive_scan_u32(s, nb.ocnt.data(), nb.opos.data(), n, nb.counters.data() + c + 1,
-                               nb.scratch.data());
+            exclusive_scan_u32(s, nb.ocnt.data(), nb.opos.data(), n, nullptr, nb.scratch.data());
+            k_over_list<<<div_up(n, 256), 256, 0, s>>>(n, nb.oflag.data(), nb.ofpos.data(),
+                                                        nb.opos.data(), (u32) base, map,
+                                                        nb.olist.data(), offset);
         };
-        // blocks of 8 waves per listed leaf while there are few of them, 1 wave beyond
-        constexpr u32 WIDE_FEW = 8192;
-        // the listed leaves (n_over, from the fixed-capacity pass's counts: above the capacity
-        // for exactly these) walked again into the overflow region of leaf_ids: their true
-        // list lengths first (one leaf per block, its walk spread over the threads: the listed
-        // leaves are far apart, and a wave walks the union of its lanes' walks), then the
-        // maximum, the total and the overflow offsets over the true lengths (counters 8, 10,
-        // 12, 13, read back into hc: one more host read), then the lists
-        auto resolve_leaves = [&](u32 cl, u32 n_over) {
+        // the n_over leaves whose lists (of `tot` entries in all) are longer than cl, one per
+        // wave, into the overflow region of leaf_ids
+        auto resolve_leaves = [&](u32 cl, u32 n_over, u32 tot) {
             const u64 base = (u64) L * cl;
-            k_over_list<<<div_up(L, 256), 256, 0, s>>>(L, nb.oflag.data(), nb.ofpos.data(),
-                                                        nb.opos.data(), (u32) base, nullptr,
-                                                        nb.olist.data(), nb.leaf_offset.data());
-            const bool few = n_over <= WIDE_FEW;
-            nb.wide_cnt.resize((size_t) n_over * (few ? 8 : 1) * WAVE);
-            auto walk_wide = [&](auto count, u32 *offset, u32 *ids_) {
-                constexpr bool C = decltype(count)::value;
-                if (few)
-                    k_leaf_walk_wide<8, C><<<n_over, 8 * WAVE, 0, s>>>(
-                        L, I, t.nodes.data(), Rkern, nb.olist.data(), n_over, nb.leaf_cnt.data(),
-                        nb.wide_cnt.data(), offset, ids_, err);
-                else
-                    k_leaf_walk_wide<1, C><<<n_over, WAVE, 0, s>>>(
-                        L, I, t.nodes.data(), Rkern, nb.olist.data(), n_over, nb.leaf_cnt.data(),
-                        nb.wide_cnt.data(), offset, ids_, err);
-            };
-            walk_wide(std::true_type{}, nullptr, nullptr);
-            fill_u32(s, nb.counters.data() + 8, 0, 1);
-            max_u32(s, L, nb.leaf_cnt.data(), nb.counters.data() + 8);
-            exclusive_scan_u32(s, nb.leaf_cnt.data(), nb.psum.data(), L, nb.counters.data() + 10,
-                               nb.scratch.data());
-            mark(L, nb.leaf_cnt.data(), cl, 12);
-            SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
-                                     hipMemcpyDeviceToHost, s));
-            SHAMX_HIP(hipStreamSynchronize(s));
-            check_walk_flags(hc[4]);
-            const u32 tot = hc[13];
-            if (hc[12] != n_over)
-                throw std::runtime_error("neighbour cache: overflowing leaf lists changed");
             if (base + tot > 0xffffffffull)
                 throw std::runtime_error("neighbour cache: leaf lists exceed u32 entry indices");
             nb.leaf_ids.resize_keep(std::max<u64>(base + tot, 1), s);
-            k_over_list<<<div_up(L, 256), 256, 0, s>>>(L, nb.oflag.data(), nb.ofpos.data(),
-                                                        nb.opos.data(), (u32) base, nullptr,
-                                                        nb.olist.data(), nb.leaf_offset.data());
-            walk_wide(std::false_type{}, nb.leaf_offset.data(), nb.leaf_ids.data());
+            list_over(L, nb.leaf_cnt.data(), cl, base, nullptr, nb.leaf_offset.data());
+            k_leaf_lists<LEAF_FILL, true>
+                <<<div_up(n_over, (u32) LW_WAVES), LW_WAVES * WAVE, 0, s>>>(
+                    L, I, t.nodes.data(), nb.tiers.data(), tt, Rkern, nb.leaf_cnt.data(),
+                    nb.leaf_offset.data(), nb.leaf_ids.data(), 0, nb.lap.data(),
+                    nb.olist.data(), n_over);
         };
         for (int attempt = 0;; attempt++) {
             if (attempt == 4) throw std::runtime_error("neighbour cache: capacities do not settle");
             u32 cl = nb.cap_leaf, cp = nb.cap_part;
+            if (attempt) {
+                fill_u32(s, mism_len, 0, 1);
+                fill_u32(s, nb.counters.data() + 8, 0, 8);
+            }
             if ((u64) L * cl > 0xffffffffull) {
                 // u32 entry indices cannot address fixed-capacity leaf lists: two passes each
-                k_leaf_neigh_w<false, false><<<div_up(L, 256), 256, 0, s>>>(
-                    L, I, t.nodes.data(), Rkern, nb.leaf_cnt.data(), nullptr, nullptr, 0, err, 64);
-                exclusive_scan_u32(s, nb.leaf_cnt.data(), nb.leaf_offset.data(), L,
-                                   nb.counters.data(), nb.scratch.data());
-                SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 8 * sizeof(u32),
-                                         hipMemcpyDeviceToHost, s));
-                SHAMX_HIP(hipStreamSynchronize(s));
-                tree_check(t);
-                if (hc[4]) throw std::runtime_error("neighbour cache: tree traversal stack overflow");
-                nb.n_leaf_pairs = hc[0];
-                nb.leaf_ids.resize(std::max<u64>(nb.n_leaf_pairs, 1));
-                k_leaf_neigh_w<true, false><<<div_up(L, 256), 256, 0, s>>>(
-                    L, I, t.nodes.data(), Rkern, nullptr, nb.leaf_offset.data(),
-                    nb.leaf_ids.data(), 0, err, 64);
-                stage2_packed<true>(s, nb, t, n_local, x, y, z, h, htol, Rker2, hc);
+                packed_leaves();
+                own_leaves(0);
+                stage2_packed<true>(s, nb, t, n_local, gblocks, x, y, z, h, htol, Rker2, hc);
                 nb.leaf_stride = 0;
                 nb.row_stride  = 0;
                 nb.cap_leaf    = choose(hc[8], nb.n_leaf_pairs, L, L);
@@ -1139,40 +1100,26 @@ namespace shamx {
             }
             // stage 1: fixed-capacity leaf lists
             nb.leaf_ids.resize(std::max<u64>((u64) L * cl, 1));
-            fill_u32(s, nb.counters.data() + 8, 0, 8);
-            const u32 lpw = leaf_lanes();
-            k_leaf_neigh_w<true, true><<<div_up(div_up(L, lpw), 256 / WAVE), 256, 0, s>>>(
-                L, I, t.nodes.data(), Rkern, nb.leaf_cnt.data(), nb.leaf_offset.data(),
-                nb.leaf_ids.data(), cl, err, lpw);
-            max_u32(s, L, nb.leaf_cnt.data(), nb.counters.data() + 8);
-            exclusive_scan_u32(s, nb.leaf_cnt.data(), nb.psum.data(), L, nb.counters.data() + 10,
-                               nb.scratch.data());
-            mark(L, nb.leaf_cnt.data(), cl, 12);
-            const bool resolve_first = nb.leaf_overflowed;
+            leaf_lists<LEAF_ROWS>(s, nb, t, tt, Rkern, cl);
+            row_stats(s, L, nb.leaf_cnt.data(), cl, nb.counters.data() + 8,
+                      nb.counters.data() + 10, nb.counters.data() + 12);
+            const bool packed        = (u64) nm * cp > 0xffffffffull || packed_rows_forced();
+            const bool resolve_first = nb.leaf_overflowed || packed;
             if (resolve_first) {
                 SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
                                          hipMemcpyDeviceToHost, s));
                 SHAMX_HIP(hipStreamSynchronize(s));
                 tree_check(t);
-                if (hc[4]) throw std::runtime_error("neighbour cache: tree traversal stack overflow");
-                if (hc[12]) resolve_leaves(cl, hc[12]);
+                if (hc[12]) resolve_leaves(cl, hc[12], hc[13]);
             }
             const u32 leaf_cap = resolve_first ? 0u : cl; // lists past cl are truncated
-            if ((u64) nm * cp > 0xffffffffull || packed_rows_forced()) {
+            own_leaves(leaf_cap);
+            if (packed) {
                 // particle rows packed (count, scan, fill)
-                if (!resolve_first) {
-                    SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
-                                             hipMemcpyDeviceToHost, s));
-                    SHAMX_HIP(hipStreamSynchronize(s));
-                    tree_check(t);
-                    if (hc[4])
-                        throw std::runtime_error("neighbour cache: tree traversal stack overflow");
-                    if (hc[12]) resolve_leaves(cl, hc[12]);
-                }
                 const u32 n_leaf_pairs = hc[10];
                 nb.leaf_overflowed     = hc[12] > 0;
                 const u32 mxl          = hc[8];
-                stage2_packed<true>(s, nb, t, n_local, x, y, z, h, htol, Rker2, hc, 0);
+                stage2_packed<true>(s, nb, t, n_local, gblocks, x, y, z, h, htol, Rker2, hc, 0);
                 nb.n_leaf_pairs = n_leaf_pairs;
                 nb.leaf_stride  = cl;
                 nb.row_stride   = 0;
@@ -1193,14 +1140,13 @@ namespace shamx {
                 nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(), x,
                 y, z, h, nb.inv.data(), htol, Rker2, nb.cnt.data(), nb.offset.data(),
                 nb.ids.data(), cp, leaf_cap);
-            max_u32(s, nm, nb.cnt.data(), nb.counters.data() + 9);
-            exclusive_scan_u32(s, nb.cnt.data(), nb.psum.data(), nm, nb.counters.data() + 11,
-                               nb.scratch.data());
+            row_stats(s, nm, nb.cnt.data(), cp, nb.counters.data() + 9, nb.counters.data() + 11,
+                      nb.counters.data() + 14);
             SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
                                      hipMemcpyDeviceToHost, s));
             SHAMX_HIP(hipStreamSynchronize(s));
             tree_check(t);
-            check_walk_flags(hc[4]);
+            check_flags(hc[4]);
             if (!resolve_first && hc[12]) {
                 // leaf lists overflowed for the first time: stage 2 read truncated lists
                 nb.leaf_overflowed = true;
@@ -1215,20 +1161,12 @@ namespace shamx {
             const u32 mxl = hc[8], mxp = hc[9];
             // particle rows past cp: list them (sorted positions -> particle ids) and fill each
             // again, one wave per row, into the overflow region of ids
-            fill_u32(s, nb.counters.data() + 14, 0, 2);
-            mark(nm, nb.cnt.data(), cp, 14);
-            SHAMX_HIP(hipMemcpyAsync(hc + 14, nb.counters.data() + 14, 2 * sizeof(u32),
-                                     hipMemcpyDeviceToHost, s));
-            SHAMX_HIP(hipStreamSynchronize(s));
             if (hc[14]) {
                 const u64 base = (u64) nm * cp;
                 if (base + hc[15] > 0xffffffffull)
                     throw std::runtime_error("neighbour cache: rows exceed u32 entry indices");
                 nb.ids.resize_keep(base + hc[15], s);
-                k_over_list<<<div_up(nm, 256), 256, 0, s>>>(nm, nb.oflag.data(), nb.ofpos.data(),
-                                                             nb.opos.data(), (u32) base,
-                                                             t.sort_index.data(), nb.olist.data(),
-                                                             nb.offset.data());
+                list_over(nm, nb.cnt.data(), cp, base, t.sort_index.data(), nb.offset.data());
                 k_group_neigh<true, true, false, true>
                     <<<div_up(hc[14], (u32) GRP_WAVES), GRP_WAVES * WAVE, 0, s>>>(
                         n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
