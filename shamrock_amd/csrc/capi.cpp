@@ -134,7 +134,8 @@ struct shamx_solver {
     DevArray<f64> ax, ay, az, du, ax_old, ay_old, az_old, du_old, eps, h_old, vsig, dtc;
     // varying AV (Cullen & Dehnen 2010): alpha and the sound speed saved at the end of the
     // previous step (local), the updated alpha, 5 operator arrays (local), sorted accelerations
-    DevArray<f64> alpha_av, soundspeed, alpha_new, sacc;
+    DevArray<f64> alpha_av, soundspeed, alpha_new;
+    DevArray<double4> sacc;
     DevArray<f64> divv, curlx, curly, curlz, dtdivv; // the operators of the last force pass
     // sinks (sink_edges_helper.hpp:234-248), host-side like the reference's synchronized data,
     // and the particles' external acceleration (axyz_ext, 3 N)
@@ -609,17 +610,14 @@ struct shamx_solver {
                 // accelerations, alpha update over this dt, alpha into the records
                 b = timer.begin(stream);
                 u32 Nm = N + G;
-                sacc.resize(3 * (size_t) std::max<u32>(Nm, 1));
-                const f64 *acc_in[3] = {ax.data(), ay.data(), az.data()};
-                f64 *acc_out[3] = {sacc.data(), sacc.data() + Nm, sacc.data() + 2 * (size_t) Nm};
-                adjoint_gather_sorted(stream, Nm, N, tree.sort_index.data(), ghost_src.data(), 3,
-                                      acc_in, acc_out);
+                sacc.resize(std::max<u32>(Nm, 1));
                 f64 *w5[5] = {divv.data(), curlx.data(), curly.data(), curlz.data(),
                               dtdivv.data()};
                 cd10_alpha(stream, cfg.kernel, N, Nm, csr_force(), frec.data(),
-                           tree.sort_index.data(), ghost_src.data(), acc_out, soundspeed.data(),
-                           h.data(), alpha_av.data(), dtc_, cfg.gpart_mass, cfg.alpha_min,
-                           cfg.alpha_max, cfg.sigma_decay, w5, alpha_new.data());
+                           tree.sort_index.data(), ghost_src.data(), ax.data(), ay.data(),
+                           az.data(), sacc.data(), soundspeed.data(), h.data(), alpha_av.data(),
+                           dtc_, cfg.gpart_mass, cfg.alpha_min, cfg.alpha_max, cfg.sigma_decay,
+                           w5, alpha_new.data());
                 timer.end(stream, PH_EOS, b);
             }
             b = timer.begin(stream);

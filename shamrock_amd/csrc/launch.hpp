@@ -236,12 +236,13 @@ namespace shamx {
     // varying AV (Cullen & Dehnen 2010): div v, curl v, d(div v)/dt over the force rows of the
     // n local particles (sorted layout), the alpha update from the saved sound speed into
     // alpha_new (local), and alpha of every merged particle into the FP64 records.
-    // sorted_acc: merged accelerations in sorted order; work6: 5 local scratch arrays.
+    // ax, ay, az: local accelerations; sacc: nm entries of work space; work6: 5 local scratch
+    // arrays.
     void cd10_alpha(hipStream_t s, int kernel, u32 n, u32 nm, Csr c, const void *rec,
-                    const u32 *sort_index, const u32 *ghost_src, const f64 *const *sorted_acc,
-                    const f64 *cs_saved, const f64 *h, const f64 *alpha, f64 dt, f64 mass,
-                    f64 alpha_min, f64 alpha_max, f64 sigma_decay, f64 *const *work6,
-                    f64 *alpha_new);
+                    const u32 *sort_index, const u32 *ghost_src, const f64 *ax, const f64 *ay,
+                    const f64 *az, double4 *sacc, const f64 *cs_saved, const f64 *h,
+                    const f64 *alpha, f64 dt, f64 mass, f64 alpha_min, f64 alpha_max,
+                    f64 sigma_decay, f64 *const *work6, f64 *alpha_new);
     // one sink's gravity on n particles (SinkParticlesUpdate.cpp:69-150): ext += -G M d/|d|^3
     // (ext starts from 0 when first), zero inside the accretion radius, with an optional
     // Plummer softening (0 = the reference's force); sum_out (device, 3 f64 as u64 words)

@@ -1011,82 +1011,13 @@ namespace shamx {
             c[2] = a[0] * b[1] - a[1] * b[0];
         }
 
-        // div v and curl v (DiffOperator.cpp:24-268) over the force rows (their criterion is the
-        // operators' own), one lane per particle, sums in row order
-        template<class K>
-        __global__ void __launch_bounds__(BLK)
-            k_divv_curlv(u32 n, Rows r, const FRec *__restrict rec, f64 mass,
-                         f64 *__restrict divv, f64 *__restrict curlx, f64 *__restrict curly,
-                         f64 *__restrict curlz) {
-            using KK = Kern<K, f64>;
-            u32 j    = xcd_block(blockIdx.x, gridDim.x) * BLK + threadIdx.x;
-            if (j >= n) return;
-            u32 row = r.sel[j], a = r.outi[row];
-            const FRec A = rec[row];
-            f64 inv_rho_omega_a = 1. / A.romega; // 1 / (omega_a rho_a)
-            f64 sum_nabla_v = 0, sc[3] = {0, 0, 0};
-            u32 k0 = r.off[row], k1 = k0 + r.cnt[row];
-            for (u32 k = k0; k < k1; k++) {
-                const FRec B = rec[r.ids[k]];
-                f64 dr[3] = {A.x - B.x, A.y - B.y, A.z - B.z};
-                f64 rab2  = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
-                if (rab2 > rec_hR2<K>(A) && rab2 > rec_hR2<K>(B)) continue;
-                f64 rab     = sqrt(rab2);
-                f64 v_ab[3] = {A.vx - B.vx, A.vy - B.vy, A.vz - B.vz};
-                f64 ru[3]   = {dr[0] / rab, dr[1] / rab, dr[2] / rab};
-                if (rab < 1e-9) ru[0] = ru[1] = ru[2] = 0;
-                f64 dW      = KK::dW(rab, A.h);
-                f64 dWa[3]  = {dW * ru[0], dW * ru[1], dW * ru[2]};
-                sum_nabla_v += mass * (v_ab[0] * dWa[0] + v_ab[1] * dWa[1] + v_ab[2] * dWa[2]);
-                f64 c[3];
-                cross3(v_ab, dWa, c);
-                for (int t = 0; t < 3; t++) sc[t] = sc[t] + mass * c[t];
-            }
-            divv[a]  = -inv_rho_omega_a * sum_nabla_v;
-            curlx[a] = -inv_rho_omega_a * sc[0];
-            curly[a] = -inv_rho_omega_a * sc[1];
-            curlz[a] = -inv_rho_omega_a * sc[2];
-        }
-
-        // d(div v)/dt (DiffOperatorDtDivv.cpp:89-175) with the merged accelerations in sorted
-        // order; 3x3 inverse and products as in matrix_legacy.hpp:25-95 (rows stored)
-        template<class K>
-        __global__ void __launch_bounds__(BLK)
-            k_dtdivv(u32 n, Rows r, const FRec *__restrict rec, const f64 *__restrict sax,
-                     const f64 *__restrict say, const f64 *__restrict saz, f64 mass,
-                     f64 *__restrict dtdivv) {
-            using KK = Kern<K, f64>;
-            u32 j    = xcd_block(blockIdx.x, gridDim.x) * BLK + threadIdx.x;
-            if (j >= n) return;
-            u32 row = r.sel[j], a = r.outi[row];
-            const FRec A = rec[row];
-            const f64 aa[3] = {sax[row], say[row], saz[row]};
-            f64 R[3][3] = {}, Rv[3][3] = {}, Ra[3][3] = {};
-            u32 k0 = r.off[row], k1 = k0 + r.cnt[row];
-            for (u32 k = k0; k < k1; k++) {
-                u32 b        = r.ids[k];
-                const FRec B = rec[b];
-                f64 rr[3] = {A.x - B.x, A.y - B.y, A.z - B.z};
-                f64 rab2  = rr[0] * rr[0] + rr[1] * rr[1] + rr[2] * rr[2];
-                if (rab2 > rec_hR2<K>(A) && rab2 > rec_hR2<K>(B)) continue;
-                f64 rab     = sqrt(rab2);
-                f64 v_ab[3] = {A.vx - B.vx, A.vy - B.vy, A.vz - B.vz};
-                f64 a_ab[3] = {aa[0] - sax[b], aa[1] - say[b], aa[2] - saz[b]};
-                f64 ru[3]   = {rr[0] / rab, rr[1] / rab, rr[2] / rab};
-                if (rab < 1e-9) ru[0] = ru[1] = ru[2] = 0;
-                f64 dW = KK::dW(rab, A.h);
-                f64 m[3] = {dW * ru[0] * mass, dW * ru[1] * mass, dW * ru[2] * mass};
-                for (int i = 0; i < 3; i++)
-                    for (int c = 0; c < 3; c++) {
-                        R[i][c]  = R[i][c] - rr[i] * m[c];
-                        Rv[i][c] = Rv[i][c] - v_ab[c] * m[i];
-                        Ra[i][c] = Ra[i][c] - a_ab[c] * m[i];
-                    }
-            }
+        // 3x3 inverse and products as in matrix_legacy.hpp:25-95 (rows stored), and the trace
+        // terms of d(div v)/dt (DiffOperatorDtDivv.cpp:89-175) from the three sums
+        __device__ inline f64 dtdivv_of(const f64 *R, const f64 *Rv, const f64 *Ra) {
             // inverse (matrix_legacy.hpp:25-50): aij = R[i][j] (element j of stored row i)
-            f64 a00 = R[0][0], a10 = R[1][0], a20 = R[2][0];
-            f64 a01 = R[0][1], a11 = R[1][1], a21 = R[2][1];
-            f64 a02 = R[0][2], a12 = R[1][2], a22 = R[2][2];
+            f64 a00 = R[0], a10 = R[3], a20 = R[6];
+            f64 a01 = R[1], a11 = R[4], a21 = R[7];
+            f64 a02 = R[2], a12 = R[5], a22 = R[8];
             f64 det = (-a02 * a11 * a20 + a01 * a12 * a20 + a02 * a10 * a21 - a00 * a12 * a21 -
                        a01 * a10 * a22 + a00 * a11 * a22);
             f64 iv[3][3] = {{(-a12 * a21 + a11 * a22) / det, (a02 * a21 - a01 * a22) / det,
@@ -1096,10 +1027,10 @@ namespace shamx {
                             {(-a11 * a20 + a10 * a21) / det, (a01 * a20 - a00 * a21) / det,
                              (-a01 * a10 + a00 * a11) / det}};
             // products (matrix_legacy.hpp:53-95): out[i][c] = sum_k iv[i][k] B[k][c], k order
-            auto prod = [&](const f64 B[3][3], f64 O[3][3]) {
+            auto prod = [&](const f64 *B, f64 O[3][3]) {
                 for (int i = 0; i < 3; i++)
                     for (int c = 0; c < 3; c++)
-                        O[i][c] = iv[i][0] * B[0][c] + iv[i][1] * B[1][c] + iv[i][2] * B[2][c];
+                        O[i][c] = iv[i][0] * B[c] + iv[i][1] * B[3 + c] + iv[i][2] * B[6 + c];
             };
             f64 dv[3][3], da[3][3];
             prod(Rv, dv);
@@ -1108,7 +1039,151 @@ namespace shamx {
             f64 tens  = dv[0][0] * dv[0][0] + dv[1][0] * dv[0][1] + dv[2][0] * dv[0][2] +
                        dv[0][1] * dv[1][0] + dv[1][1] * dv[1][1] + dv[2][1] * dv[1][2] +
                        dv[0][2] * dv[2][0] + dv[1][2] * dv[2][1] + dv[2][2] * dv[2][2];
-            dtdivv[a] = div_a - tens;
+            return div_a - tens;
+        }
+
+        // div v, curl v (DiffOperator.cpp:24-268) and d(div v)/dt (DiffOperatorDtDivv.cpp:89-175)
+        // in one loop over the force rows (their criterion is the operators' own, so the rows
+        // hold exactly the pairs that enter).  sacc: the merged accelerations in sorted order.
+        //
+        // Four lanes per particle, as in the force loop, and its record prefetch: one pair's
+        // geometry serves all three operators.  The 31 sums (1 divergence, 3 curl, 3 matrices)
+        // would take 62 registers in every lane if each folded them all; instead the lanes
+        // write their terms to LDS, 16 sums at a time, and lane c folds sums 4 c .. 4 c + 3 of the
+        // sixteen over the four lanes' terms in lane order: the sums still take their terms in
+        // row order, one IEEE add each (X - p is X + (-p)).  Rows of 18 doubles keep the 16-byte
+        // accesses of eight neighbouring lanes on different banks.  Entries past the row's end
+        // and terms of a particle with itself are zeros, which leave a sum that started at +0.0
+        // as it is.
+        //
+        // Bound by its LDS traffic (32 16-byte accesses per lane and pass: 256 of the about 350
+        // cycles that 64 pairs take on a CU) beside about 190 VALU instructions per pair.  HCP
+        // lattice of 1.09 M particles (M4, 62 M pairs): 0.69 ms, against 1.97 + 2.31 ms for one
+        // lane per particle with all sums in registers and plain divisions, one kernel for the
+        // first-order operators and one for d(div v)/dt; Sod tube (M6, 11 M pairs) 0.19 against
+        // 0.37 + 0.49 ms.
+        constexpr int CD_SUMS = 16, CD_ROW = CD_SUMS + 2;
+        template<class K>
+        __global__ void __launch_bounds__(BLK)
+            k_cd10_operators(u32 n, Rows r, const FRec *__restrict rec,
+                             const double4 *__restrict sacc, f64 mass, f64 *__restrict divv,
+                             f64 *__restrict curlx, f64 *__restrict curly,
+                             f64 *__restrict curlz, f64 *__restrict dtdivv) {
+            using KK        = Kern<K, f64>;
+            constexpr int G = 4;
+            __shared__ __attribute__((aligned(16))) f64 fold[BLK][CD_ROW];
+            const u32 j  = (xcd_block(blockIdx.x, gridDim.x) * BLK + threadIdx.x) / G;
+            const u32 lg = threadIdx.x % G;
+            if (j >= n) return; // whole groups: no barrier below spans waves
+            const u32 row = r.sel[j];
+            // what the loop reads of a record: position, velocity; acceleration from sacc
+            struct Nb {
+                f64 x, y, z, vx, vy, vz, ax, ay, az;
+            };
+            auto load = [&](u32 b) {
+                const FRec &q   = rec[b];
+                const double4 a = sacc[b];
+                return Nb{q.x, q.y, q.z, q.vx, q.vy, q.vz, a.x, a.y, a.z};
+            };
+            const Nb A        = load(row);
+            const f64 h_a     = rec[row].h, rh = rec[row].rh, rh4 = rec[row].rh4;
+            const f64 h4_a    = h_a * h_a * h_a * h_a;
+            const bool fast   = rh != 0;
+            const u32 k0 = r.off[row], k1 = k0 + r.cnt[row];
+            f64 acc[2][4] = {};
+            f64 *mine     = fold[threadIdx.x];
+            const f64(*grp)[CD_ROW] = fold + (threadIdx.x & ~3u);
+            // folds the 16 terms per lane in LDS into the sums of this half
+            auto share = [&](int half) {
+                wave_lds_sync();
+#pragma unroll
+                for (int L = 0; L < G; L++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        acc[half][c] = acc[half][c] + grp[L][4 * lg + c];
+                wave_lds_sync();
+            };
+            auto step = [&](const Nb &B, u32 k) {
+                f64 v[3] = {}, a[3] = {}, m[3] = {};
+                if (k < k1) {
+                    const f64 dr[3] = {A.x - B.x, A.y - B.y, A.z - B.z};
+                    const f64 rab   = sqrt(dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2]);
+                    v[0] = A.vx - B.vx, v[1] = A.vy - B.vy, v[2] = A.vz - B.vz;
+                    a[0] = A.ax - B.ax, a[1] = A.ay - B.ay, a[2] = A.az - B.az;
+                    // r_ab / |r_ab|, 0 below 1e-9 (inv is 0 there)
+                    const f64 inv   = inv_sat_positive(rab);
+                    const f64 ru[3] = {div_rcp(dr[0], rab, inv), div_rcp(dr[1], rab, inv),
+                                       div_rcp(dr[2], rab, inv)};
+                    f64 dW;
+                    if (fast) dW = div_rcp(KK::norm * K::df(div_rcp(rab, h_a, rh)), h4_a, rh4);
+                    else dW = KK::dW(rab, h_a);
+                    const f64 g[3] = {dW * ru[0], dW * ru[1], dW * ru[2]};
+                    f64 c[3];
+                    cross3(v, g, c);
+                    mine[0] = mass * (v[0] * g[0] + v[1] * g[1] + v[2] * g[2]);
+                    for (int i = 0; i < 3; i++) {
+                        mine[1 + i] = mass * c[i];
+                        m[i]        = g[i] * mass;
+                    }
+                    for (int i = 0; i < 3; i++)
+                        for (int e = 0; e < 3; e++) mine[4 + 3 * i + e] = -(dr[i] * m[e]);
+                    for (int e = 0; e < 3; e++) mine[13 + e] = -(v[e] * m[0]);
+                } else {
+                    for (int c = 0; c < CD_SUMS; c++) mine[c] = 0.;
+                }
+                share(0);
+                // (v, a, m of an entry past the row's end are zeros)
+                for (int i = 1; i < 3; i++)
+                    for (int e = 0; e < 3; e++) mine[3 * (i - 1) + e] = -(v[e] * m[i]);
+                for (int i = 0; i < 3; i++)
+                    for (int e = 0; e < 3; e++) mine[6 + 3 * i + e] = -(a[e] * m[i]);
+                share(1);
+            };
+            // two records in flight, used in turn (k_force)
+            if (k0 < k1) {
+                const u32 last = k1 - 1;
+                u32 id1        = r.ids[min(k0 + lg + G, last)];
+                Nb B0          = load(r.ids[min(k0 + lg, last)]);
+                for (u32 base = k0; base < k1; base += 2 * G) {
+                    const u32 k   = base + lg;
+                    const Nb B1   = load(id1);
+                    const u32 id0 = r.ids[min(k + 2 * G, last)];
+                    id1           = r.ids[min(k + 3 * G, last)];
+                    step(B0, k);
+                    B0 = load(id0);
+                    if (base + G < k1) step(B1, k + G);
+                }
+            }
+            // the sums to the first lane
+            for (int half = 0; half < 2; half++)
+                for (int c = 0; c < 4; c++) mine[4 * half + c] = acc[half][c];
+            wave_lds_sync();
+            if (lg == 0) {
+                f64 s[2 * CD_SUMS];
+                for (int half = 0; half < 2; half++)
+                    for (int L = 0; L < G; L++)
+                        for (int c = 0; c < 4; c++)
+                            s[half * CD_SUMS + 4 * L + c] = grp[L][4 * half + c];
+                const u32 a = r.outi[row];
+                const f64 inv_rho_omega_a = 1. / rec[row].romega; // 1 / (omega_a rho_a)
+                divv[a]   = -inv_rho_omega_a * s[0];
+                curlx[a]  = -inv_rho_omega_a * s[1];
+                curly[a]  = -inv_rho_omega_a * s[2];
+                curlz[a]  = -inv_rho_omega_a * s[3];
+                dtdivv[a] = dtdivv_of(s + 4, s + 13, s + 22);
+            }
+        }
+
+        // merged accelerations in sorted order (images take their source's)
+        __global__ void k_sorted_acc(u32 nm, u32 N, const u32 *__restrict sort_index,
+                                     const u32 *__restrict ghost_src, const f64 *__restrict ax,
+                                     const f64 *__restrict ay, const f64 *__restrict az,
+                                     double4 *__restrict sacc) {
+            u32 s = blockIdx.x * blockDim.x + threadIdx.x;
+            if (s >= nm) return;
+            u32 b = sort_index[s];
+            if (b >= N) b = ghost_src[b - N];
+            sacc[s] = make_double4(ax[b], ay[b], az[b], 0.);
         }
 
         // alpha update (UpdateViscosity.cpp:120-219), local particles
@@ -1774,20 +1849,17 @@ namespace shamx {
     }
 
     void cd10_alpha(hipStream_t s, int kernel, u32 n, u32 nm, Csr c, const void *rec,
-                    const u32 *sort_index, const u32 *ghost_src, const f64 *const *sorted_acc,
-                    const f64 *cs_saved, const f64 *h, const f64 *alpha, f64 dt, f64 mass,
-                    f64 alpha_min, f64 alpha_max, f64 sigma_decay, f64 *const *work6,
-                    f64 *alpha_new) {
+                    const u32 *sort_index, const u32 *ghost_src, const f64 *ax, const f64 *ay,
+                    const f64 *az, double4 *sacc, const f64 *cs_saved, const f64 *h,
+                    const f64 *alpha, f64 dt, f64 mass, f64 alpha_min, f64 alpha_max,
+                    f64 sigma_decay, f64 *const *work6, f64 *alpha_new) {
         if (n == 0) return;
-        u32 nb = div_up(n, BLK);
-        Rows r = rows_of(c);
         const FRec *fr = (const FRec *) rec;
+        k_sorted_acc<<<div_up(nm, 256), 256, 0, s>>>(nm, n, sort_index, ghost_src, ax, ay, az,
+                                                     sacc);
         dispatch_kernel(kernel, [&](auto K) {
-            using KT = decltype(K);
-            k_divv_curlv<KT><<<nb, BLK, 0, s>>>(n, r, fr, mass, work6[0], work6[1], work6[2],
-                                                work6[3]);
-            k_dtdivv<KT><<<nb, BLK, 0, s>>>(n, r, fr, sorted_acc[0], sorted_acc[1],
-                                            sorted_acc[2], mass, work6[4]);
+            k_cd10_operators<decltype(K)><<<div_up((u64) n * 4, BLK), BLK, 0, s>>>(
+                n, rows_of(c), fr, sacc, mass, work6[0], work6[1], work6[2], work6[3], work6[4]);
         });
         k_alpha_cd10<<<div_up(n, 256), 256, 0, s>>>(n, dt, cs_saved, h, alpha, work6[0],
                                                     work6[1], work6[2], work6[3], work6[4],
