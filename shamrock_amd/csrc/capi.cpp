@@ -1208,7 +1208,6 @@ int shamx_tree_build(shamx_ctx *ctx, void *stream, uint32_t n, const double *x, 
         need(ctx != nullptr, "shamx_tree_build: null context");
         tree_build((hipStream_t) stream, ctx->tree, n, x, y, z, h, reduction_level, htol);
         SHAMX_HIP(hipStreamSynchronize((hipStream_t) stream));
-        tree_check(ctx->tree);
     });
 }
 
@@ -1229,7 +1228,6 @@ int shamx_tree_aabb_hmax(shamx_ctx *ctx, void *stream, const double *x, const do
         need(ctx && ctx->tree.L > 0, "shamx_tree_aabb_hmax: build the tree first");
         tree_stage_aabb((hipStream_t) stream, ctx->tree, x, y, z, h, htol);
         SHAMX_HIP(hipStreamSynchronize((hipStream_t) stream));
-        tree_check(ctx->tree);
     });
 }
 

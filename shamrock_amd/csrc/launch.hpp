@@ -9,6 +9,7 @@
 
 #include "common.hpp"
 #include "devbuf.hpp"
+#include "tree_layout.hpp"
 
 namespace shamx {
 
@@ -61,12 +62,12 @@ namespace shamx {
         DevArray<u32> leaf_codes;      // L
         DevArray<u32> lchild, rchild, endrange; // I
         DevArray<u8> lflag, rflag;     // I
-        DevArray<u32> parent;          // I + L
-        DevArray<u16> depth;           // I (root 0)
         DevArray<f64> nodes;           // (I + L) * NODE_F64 records (tree_layout.hpp)
+        DevArray<f64> tiers;           // 8-ary hierarchy over the leaves (tree_layout.hpp)
+        Tiers tt;
         DevArray<u32> counters;        // small device scalars
         PinnedWords<u32, 8> host;      // their host copies
-        bool err_pending = false;      // host[5] holds the last box pass's flags (tree_check)
+        bool big_listed = false;       // counters[7] counts listed leaves of an earlier box pass
         DevArray<unsigned char> scratch;
         // order runs of equal codes by the position inside the cell (set from the previous
         // build's distinct-code count when allow_fine_ties; the phase entries keep the plain
@@ -90,10 +91,6 @@ namespace shamx {
     void tree_stage_karras(hipStream_t s, TreeBuffers &t, u32 reduction_level);
     void tree_stage_aabb(hipStream_t s, TreeBuffers &t, const f64 *x, const f64 *y,
                          const f64 *z, const f64 *h, f64 htol);
-    // throws if the last box pass flagged the tree (broken parent links, a child index out of
-    // range, a cell deeper than the merge levels); valid once the stream has been synchronised
-    // after that pass (the neighbour build and the next tree build do it)
-    void tree_check(TreeBuffers &t);
 
     // ------------------------------------------------------------------ neigh.hip
     struct NeighBuffers {
@@ -109,7 +106,6 @@ namespace shamx {
         DevArray<u32> lpos;                             // sorted layout: local rows in order
         DevArray<u32> fcnt, fids;                       // force-interacting subsequences
         DevArray<u32> lflag, lscan;
-        DevArray<f64> tiers; // 8-ary hierarchy over the leaves (stage 1)
         DevArray<u32> lap;   // per leaf: a later leaf's box meets its box
         // sorted layout: one pass per stage into rows of fixed capacity; leaf l's list at
         // leaf_ids[l * leaf_stride], row r at ids[r * row_stride] (0: packed layout).  The

@@ -38,67 +38,8 @@ namespace shamx {
         // the order of the leaf index.  Any search that tests every leaf that can pass, in index
         // order, therefore gives the reference's list.
         //
-        // The search runs over tiers: tier 0 are the leaves, cell j of tier t holds the cells
-        // [8 j, 8 j + 8) of tier t - 1 (box and largest rint; same 64-byte records as the tree),
-        // up to a tier of at most 64 cells.  The leaves are in Morton order, so eight of a run
-        // are about one octant, the children of a cell are one contiguous read, and the number of
-        // dependent steps is log8 of the leaf count.
-        constexpr u32 TIER_MAX = 10; // 64 * 8^10 leaves
-        struct Tiers {
-            u32 top;              // index of the top tier
-            u32 n[TIER_MAX + 1];   // cells per tier; n[0] leaves
-            u32 off[TIER_MAX + 1]; // first record of a tier (tier 0: the tree's leaves)
-        };
-        struct Cell {
-            f64 lo[3], hi[3], r;
-        };
-        __device__ inline Cell cell_load(const f64 *__restrict rec) {
-            return Cell{{rec[0], rec[1], rec[2]}, {rec[3], rec[4], rec[5]}, rec[6]};
-        }
-        constexpr f64 F64_BIG = 1.7976931348623157e308;
-        __device__ inline Cell cell_none() {
-            return Cell{{F64_BIG, F64_BIG, F64_BIG}, {-F64_BIG, -F64_BIG, -F64_BIG}, 0.};
-        }
-        // union over the lanes whose index differs in the bits o
-        __device__ inline void cell_merge_xor(Cell &c, int o) {
-            for (int k = 0; k < 3; k++) {
-                c.lo[k] = fmin(c.lo[k], __shfl_xor(c.lo[k], o, WAVE));
-                c.hi[k] = fmax(c.hi[k], __shfl_xor(c.hi[k], o, WAVE));
-            }
-            c.r = fmax(c.r, __shfl_xor(c.r, o, WAVE));
-        }
-        __device__ inline void cell_store(f64 *__restrict rec, const Cell &c) {
-            for (int k = 0; k < 3; k++) {
-                rec[k]     = c.lo[k];
-                rec[3 + k] = c.hi[k];
-            }
-            rec[6] = c.r;
-            rec[7] = 0.;
-        }
-        // three tiers over the n cells of src in one launch, 512 cells per block (d2, d3: null
-        // when the tiers end below them)
-        constexpr int TIER_BLK = 512;
-        __global__ void __launch_bounds__(TIER_BLK)
-            k_leaf_tiers(u32 n, const f64 *__restrict src, f64 *__restrict d1,
-                         f64 *__restrict d2, f64 *__restrict d3) {
-            __shared__ Cell part[TIER_BLK / WAVE];
-            const u32 i    = blockIdx.x * TIER_BLK + threadIdx.x;
-            const u32 lane = (u32) __lane_id();
-            Cell c         = i < n ? cell_load(src + (u64) i * NODE_F64) : cell_none();
-            for (int o = 1; o < 8; o <<= 1) cell_merge_xor(c, o);
-            if (i < n && i % 8 == 0) cell_store(d1 + (u64) (i / 8) * NODE_F64, c);
-            for (int o = 8; o < WAVE; o <<= 1) cell_merge_xor(c, o);
-            if (d2 && i < n && lane == 0) cell_store(d2 + (u64) (i / 64) * NODE_F64, c);
-            if (!d3) return; // the same for the whole grid
-            if (lane == 0) part[threadIdx.x / WAVE] = c;
-            __syncthreads();
-            if (threadIdx.x < WAVE) {
-                c = lane < TIER_BLK / WAVE ? part[lane] : cell_none();
-                for (int o = 1; o < TIER_BLK / WAVE; o <<= 1) cell_merge_xor(c, o);
-                if (lane == 0) cell_store(d3 + (u64) blockIdx.x * NODE_F64, c);
-            }
-        }
-
+        // The search runs over the tiers of the tree (tree_layout.hpp): the number of dependent
+        // steps is log8 of the leaf count.
         // boxes [alo, ahi] and [blo, bhi] meet (BBAA::cella_neigh_b, geometry_utils.hpp:125-135:
         // max of the lower bounds <= min of the upper ones; a NaN bound never separates, there
         // as here)
@@ -809,35 +750,13 @@ namespace shamx {
                                                                                 tot, over);
         }
 
-        // the tiers over the leaves for the searches of stage 1
-        Tiers build_tiers(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t) {
-            Tiers tt{};
-            tt.n[0] = t.L;
-            u32 at  = 0;
-            while (tt.n[tt.top] > (u32) WAVE) {
-                const u32 k = tt.top + 1; // at most 10 for a u32 leaf count
-                tt.n[k]     = div_up(tt.n[k - 1], 8);
-                tt.off[k]   = at;
-                at += tt.n[k];
-                tt.top = k;
-            }
-            nb.tiers.resize(std::max<size_t>((size_t) at * NODE_F64, 1));
-            auto rec = [&](u32 k) -> f64 * {
-                return k <= tt.top ? nb.tiers.data() + (size_t) tt.off[k] * NODE_F64 : nullptr;
-            };
-            for (u32 k = 0; k < tt.top; k += 3)
-                k_leaf_tiers<<<div_up(tt.n[k], TIER_BLK), TIER_BLK, 0, s>>>(
-                    tt.n[k], k ? rec(k) : t.nodes.data() + (size_t) t.I * NODE_F64, rec(k + 1),
-                    rec(k + 2), rec(k + 3));
-            return tt;
-        }
         // lists of all leaves, eight per wave
         template<int OUT>
-        void leaf_lists(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, const Tiers &tt,
-                        f64 Rkern, u32 cap) {
+        void leaf_lists(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, f64 Rkern,
+                        u32 cap) {
             k_leaf_lists<OUT, false>
                 <<<div_up(div_up(t.L, LEAF_TGT), LW_WAVES), LW_WAVES * WAVE, 0, s>>>(
-                    t.L, t.I, t.nodes.data(), nb.tiers.data(), tt, Rkern, nb.leaf_cnt.data(),
+                    t.L, t.I, t.nodes.data(), t.tiers.data(), t.tt, Rkern, nb.leaf_cnt.data(),
                     nb.leaf_offset.data(), nb.leaf_ids.data(), cap, nb.lap.data(), nullptr, 0);
         }
 
@@ -977,27 +896,25 @@ namespace shamx {
         f64 Rker2 = Rkern * Rkern;
         u32 *hc = nb.host.data(); // 16 pinned words: the reads queue on the stream
 
-        // sorted copy and inverse permutation, member batches, tiers over the leaves
+        // sorted copy and inverse permutation, member batches
         nb.ps.resize(nm);
         nb.inv.resize(nm);
         nb.mism.resize(std::max<u32>(n_local, 1));
         k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, t.sort_index.data(), x, y, z,
                                                       h, nb.ps.data(), nb.inv.data(), err);
         const u32 gblocks = batch_items(s, nb, t);
-        const Tiers tt    = build_tiers(s, nb, t);
 
         // leaf lists in two passes (count, scan, fill); returns once their length is known
         auto packed_leaves = [&] {
-            leaf_lists<LEAF_COUNT>(s, nb, t, tt, Rkern, 0);
+            leaf_lists<LEAF_COUNT>(s, nb, t, Rkern, 0);
             exclusive_scan_u32(s, nb.leaf_cnt.data(), nb.leaf_offset.data(), L,
                                nb.counters.data(), nb.scratch.data());
             SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 8 * sizeof(u32),
                                      hipMemcpyDeviceToHost, s));
             SHAMX_HIP(hipStreamSynchronize(s));
-            tree_check(t);
             nb.n_leaf_pairs = hc[0];
             nb.leaf_ids.resize(std::max<u64>(nb.n_leaf_pairs, 1));
-            leaf_lists<LEAF_FILL>(s, nb, t, tt, Rkern, 0);
+            leaf_lists<LEAF_FILL>(s, nb, t, Rkern, 0);
         };
 
         if (!sorted_layout) {
@@ -1076,7 +993,7 @@ namespace shamx {
             list_over(L, nb.leaf_cnt.data(), cl, base, nullptr, nb.leaf_offset.data());
             k_leaf_lists<LEAF_FILL, true>
                 <<<div_up(n_over, (u32) LW_WAVES), LW_WAVES * WAVE, 0, s>>>(
-                    L, I, t.nodes.data(), nb.tiers.data(), tt, Rkern, nb.leaf_cnt.data(),
+                    L, I, t.nodes.data(), t.tiers.data(), t.tt, Rkern, nb.leaf_cnt.data(),
                     nb.leaf_offset.data(), nb.leaf_ids.data(), 0, nb.lap.data(),
                     nb.olist.data(), n_over);
         };
@@ -1100,7 +1017,7 @@ namespace shamx {
             }
             // stage 1: fixed-capacity leaf lists
             nb.leaf_ids.resize(std::max<u64>((u64) L * cl, 1));
-            leaf_lists<LEAF_ROWS>(s, nb, t, tt, Rkern, cl);
+            leaf_lists<LEAF_ROWS>(s, nb, t, Rkern, cl);
             row_stats(s, L, nb.leaf_cnt.data(), cl, nb.counters.data() + 8,
                       nb.counters.data() + 10, nb.counters.data() + 12);
             const bool packed        = (u64) nm * cp > 0xffffffffull || packed_rows_forced();
@@ -1109,7 +1026,6 @@ namespace shamx {
                 SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
                                          hipMemcpyDeviceToHost, s));
                 SHAMX_HIP(hipStreamSynchronize(s));
-                tree_check(t);
                 if (hc[12]) resolve_leaves(cl, hc[12], hc[13]);
             }
             const u32 leaf_cap = resolve_first ? 0u : cl; // lists past cl are truncated
@@ -1145,7 +1061,6 @@ namespace shamx {
             SHAMX_HIP(hipMemcpyAsync(hc, nb.counters.data(), 16 * sizeof(u32),
                                      hipMemcpyDeviceToHost, s));
             SHAMX_HIP(hipStreamSynchronize(s));
-            tree_check(t);
             check_flags(hc[4]);
             if (!resolve_first && hc[12]) {
                 // leaf lists overflowed for the first time: stage 2 read truncated lists

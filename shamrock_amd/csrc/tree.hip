@@ -6,11 +6,11 @@
 //   stable onesweep LSD radix sort        (replaces bitonicSort_updated_usm.cpp:284-396)
 //   leaf reduction                        (reduction_alg.cpp:62-585, MortonReducedSet.cpp:24-73)
 //   Karras 2012 radix tree                (KarrasRadixTree.cpp:45-180)
-//   leaf AABB + max-h field, then the internal cells level by level from the deepest up,
-//   one launch per depth (replaces the tree_depth = 32 full passes of
-//   KarrasRadixTreeAABB.cpp:32-74 and KarrasRadixTreeField.hpp:133-169; min / max are exact
-//   so the result is identical).  A bottom-up climb with arrival counters would need a
-//   device-scope fence per step, which on a multi-XCD GPU writes back and invalidates L2.
+//   leaf AABB + max-h field, tiers over the leaves, then every internal cell from its leaf range
+//   (replaces the tree_depth = 32 full passes of KarrasRadixTreeAABB.cpp:32-74 and
+//   KarrasRadixTreeField.hpp:133-169; min / max are exact so the result is identical).  A
+//   bottom-up climb with arrival counters would need a device-scope fence per step, which on a
+//   multi-XCD GPU writes back and invalidates L2.
 //
 // Node records: every cell (I internal cells then L leaves) owns one 64-byte record
 //   [0..2] aabb min, [3..5] aabb max, [6] rint = max h * htol,
@@ -481,7 +481,7 @@ namespace shamx {
         __global__ void k_karras(u32 L, const u32 *__restrict morton, u32 *__restrict lchild,
                                  u32 *__restrict rchild, u8 *__restrict lflag,
                                  u8 *__restrict rflag, u32 *__restrict endrange,
-                                 u32 *__restrict parent, f64 *__restrict nodes) {
+                                 f64 *__restrict nodes) {
             u32 I  = L - 1;
             u32 iu = blockIdx.x * blockDim.x + threadIdx.x;
             if (iu >= I) return;
@@ -519,10 +519,7 @@ namespace shamx {
             rflag[iu]  = rf;
             u32 lt     = (u32) gamma + (lf ? I : 0u);
             u32 rt     = (u32) (gamma + 1) + (rf ? I : 0u);
-            parent[lt] = iu;
-            parent[rt] = iu;
             node_set_children(nodes, iu, lt, rt);
-            if (iu == 0) parent[0] = NO_PARENT;
         }
 
         // leaf boxes + max h of the leaf's sorted range
@@ -650,95 +647,67 @@ namespace shamx {
             }
         }
 
-        // Internal cells are merged in bands of levels, deepest first, over MERGE_LEVELS levels
-        // with no host read of the actual depth: the leaf codes are distinct 32-bit codes (runs of
-        // equal codes are merged into one leaf), every child's range shares a strictly longer
-        // prefix than its parent's, so no internal cell lies deeper than 31.
-        constexpr u32 MERGE_LEVELS = 32;
-        // cycle guard of the parent walk
-        constexpr u32 DEPTH_MAX = 1024;
+        __device__ inline void cell_store(f64 *__restrict rec, const Cell &c) {
+            for (int k = 0; k < 3; k++) {
+                rec[k]     = c.lo[k];
+                rec[3 + k] = c.hi[k];
+            }
+            rec[6] = c.r;
+        }
+        // three tiers over the n cells of src in one launch, 512 cells per block (d2, d3: null
+        // when the tiers end below them)
+        constexpr int TIER_BLK = 512;
+        __global__ void __launch_bounds__(TIER_BLK)
+            k_leaf_tiers(u32 n, const f64 *__restrict src, f64 *__restrict d1,
+                         f64 *__restrict d2, f64 *__restrict d3) {
+            __shared__ Cell part[TIER_BLK / WAVE];
+            const u32 i    = blockIdx.x * TIER_BLK + threadIdx.x;
+            const u32 lane = (u32) __lane_id();
+            Cell c         = i < n ? cell_load(src + (u64) i * NODE_F64) : cell_none();
+            for (int o = 1; o < 8; o <<= 1) cell_merge_xor(c, o);
+            if (i < n && i % 8 == 0) cell_store(d1 + (u64) (i / 8) * NODE_F64, c);
+            for (int o = 8; o < WAVE; o <<= 1) cell_merge_xor(c, o);
+            if (d2 && i < n && lane == 0) cell_store(d2 + (u64) (i / 64) * NODE_F64, c);
+            if (!d3) return; // the same for the whole grid
+            if (lane == 0) part[threadIdx.x / WAVE] = c;
+            __syncthreads();
+            if (threadIdx.x < WAVE) {
+                c = lane < TIER_BLK / WAVE ? part[lane] : cell_none();
+                for (int o = 1; o < TIER_BLK / WAVE; o <<= 1) cell_merge_xor(c, o);
+                if (lane == 0) cell_store(d3 + (u64) blockIdx.x * NODE_F64, c);
+            }
+        }
 
-        // depth of every internal node (root 0) by walking the parent links; err bit 0: broken
-        // links, bit 2: a cell at depth >= MERGE_LEVELS
+        // Box and largest rint of every internal cell: the cell covers the leaves between its
+        // index and endrange, which are at most 14 cells per tier (the ragged ends of the range,
+        // then its whole cells one tier up).  min and max are exact, so any merge order gives the
+        // same doubles.  It replaces a merge up the binary tree, eight launches over bands of
+        // four levels after a depth pass: MEASURED_CELLS
         __global__ void __launch_bounds__(256)
-            k_node_depth(u32 I, const u32 *__restrict parent, u16 *__restrict depth,
-                         u32 *__restrict err) {
-            bool broken = false, deep = false;
-            for (u32 i = blockIdx.x * 256 + threadIdx.x; i < I; i += gridDim.x * 256) {
-                u32 d = 0, p = parent[i];
-                while (p < I && d < DEPTH_MAX) {
-                    d++;
-                    p = parent[p];
-                }
-                broken |= p != NO_PARENT;
-                deep |= d >= MERGE_LEVELS;
-                depth[i] = (u16) min(d, DEPTH_MAX - 1);
-            }
-            const bool any_broken = __ballot(broken) != 0, any_deep = __ballot(deep) != 0;
-            if (__lane_id() == 0 && (any_broken || any_deep))
-                atomicOr(err, (any_broken ? 1u : 0u) | (any_deep ? 4u : 0u));
-        }
-
-        // box and h max of a cell: [0..2] min, [3..5] max, [6] max rint
-        struct Rec7 {
-            f64 v[7];
-        };
-        __device__ inline Rec7 rec7_load(const f64 *__restrict nodes, u32 c) {
-            const f64 *p = nodes + (u64) c * NODE_F64;
-            Rec7 r;
-#pragma unroll
-            for (int k = 0; k < 7; k++) r.v[k] = p[k];
-            return r;
-        }
-        __device__ inline Rec7 rec7_merge(const Rec7 &a, const Rec7 &b) {
-            Rec7 r;
-#pragma unroll
-            for (int k = 0; k < 3; k++) r.v[k] = fmin(a.v[k], b.v[k]);
-#pragma unroll
-            for (int k = 3; k < 7; k++) r.v[k] = fmax(a.v[k], b.v[k]);
-            return r;
-        }
-        // the record of cell c as merged from the complete cells rem levels below it (or from
-        // leaves above that): cells at depth >= the band's end were merged by an earlier launch.
-        // Only the children links of the cells on the way are read; this kernel never writes
-        // them.  R bounds the recursion at compile time (rem <= R).
-        template<int R>
-        __device__ inline Rec7 band_subtree(const f64 *__restrict nodes, u32 I, u32 L, u32 c,
-                                            u32 rem, bool &bad) {
-            if constexpr (R == 0) {
-                return rec7_load(nodes, c);
-            } else {
-                if (c >= I || rem == 0) return rec7_load(nodes, c);
-                u32 lt, rt;
-                node_children(nodes, c, lt, rt);
-                if (lt >= I + L || rt >= I + L) {
-                    bad = true;
-                    return rec7_load(nodes, c);
-                }
-                return rec7_merge(band_subtree<R - 1>(nodes, I, L, lt, rem - 1, bad),
-                                  band_subtree<R - 1>(nodes, I, L, rt, rem - 1, bad));
-            }
-        }
-
-        // boxes and h max of the internal cells of depth [b0, b0 + BAND), each from its
-        // descendants of depth b0 + BAND (merged by the previous launch) and the leaves above
-        // them.  min / max are exact, so this equals any other merge order bit for bit.
-        constexpr u32 BAND = 4;
-        __global__ void k_merge_band(u32 I, u32 L, u32 b0, const u16 *__restrict depth,
-                                     f64 *__restrict nodes, u32 *__restrict err) {
-            u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+            k_cell_boxes(u32 L, const u32 *__restrict endrange, const f64 *__restrict tiers,
+                         Tiers tt, f64 *__restrict nodes) {
+            const u32 I = L - 1, i = blockIdx.x * 256 + threadIdx.x;
             if (i >= I) return;
-            const u32 d = depth[i];
-            if (d < b0 || d >= b0 + BAND) return;
-            bool bad        = false;
-            const Rec7 m    = band_subtree<BAND>(nodes, I, L, i, b0 + BAND - d, bad);
-            if (bad) {
-                atomicOr(err, 2u);
-                return;
+            const u32 j = endrange[i];
+            u32 lo = min(i, j), hi = min(max(i, j) + 1, L);
+            Cell c = cell_none();
+            for (u32 t = 0;; t++) {
+                const f64 *cells = t ? tiers + (u64) tt.off[t] * NODE_F64
+                                     : nodes + (u64) I * NODE_F64;
+                const bool last  = t == tt.top;
+                while (lo < hi && (last || lo % 8)) {
+                    cell_merge(c, cell_load(cells + (u64) lo * NODE_F64));
+                    lo++;
+                }
+                while (lo < hi && hi % 8) {
+                    hi--;
+                    cell_merge(c, cell_load(cells + (u64) hi * NODE_F64));
+                }
+                if (lo >= hi) break;
+                lo /= 8;
+                hi /= 8;
             }
-            f64 *P = nodes + (u64) i * NODE_F64;
-#pragma unroll
-            for (int k = 0; k < 7; k++) P[k] = m.v[k];
+            cell_store(nodes + (u64) i * NODE_F64, c); // the children's words stay
         }
     } // namespace
 
@@ -877,6 +846,7 @@ namespace shamx {
             a->resize(n);
         t.reduc_map.resize((size_t) n + 2);
         fill_u32(s, t.counters.data(), 0, 8);
+        t.big_listed = false;
         bbox_nextafter(s, n, x, y, z, t.bbox6.data(), t.scratch.data());
         morton_codes(s, n, x, y, z, t.bbox6.data(), t.codes.data());
         SHAMX_HIP(hipMemcpyAsync(t.sorted.data(), t.codes.data(), n * sizeof(u32),
@@ -944,7 +914,6 @@ namespace shamx {
         u32 *hc = t.host.data();
         t.host.read_async(s, t.counters.data(), 4);
         SHAMX_HIP(hipStreamSynchronize(s));
-        tree_check(t); // the previous build's, if nothing has read it since
         if (hc[2] | hc[3]) throw std::runtime_error("radix sort: look-back or scatter inconsistency");
         // the next builds order runs of equal codes spatially when codes repeat on average
         // more than 1.5 times (clustered sets whose cells hold many particles); unique codes
@@ -960,20 +929,14 @@ namespace shamx {
                                                    t.leaf_codes.data());
         u32 I = t.I;
         for (auto *a : {&t.lchild, &t.rchild, &t.endrange}) a->resize(std::max<u32>(I, 1));
-        t.depth.resize(std::max<u32>(I, 1));
         t.lflag.resize(std::max<u32>(I, 1));
         t.rflag.resize(std::max<u32>(I, 1));
-        t.parent.resize((size_t) I + L);
         t.nodes.resize((size_t) (I + L) * NODE_F64);
-        fill_u32(s, t.parent.data(), NO_PARENT, (size_t) I + L);
-        if (I > 0) {
+        if (I > 0)
             k_karras<<<div_up(I, 256), 256, 0, s>>>(L, t.leaf_codes.data(), t.lchild.data(),
                                                    t.rchild.data(), t.lflag.data(),
                                                    t.rflag.data(), t.endrange.data(),
-                                                   t.parent.data(), t.nodes.data());
-        } else {
-            fill_u32(s, t.parent.data(), NO_PARENT, 1);
-        }
+                                                   t.nodes.data());
         SHAMX_HIP(hipGetLastError());
     }
 
@@ -983,39 +946,38 @@ namespace shamx {
         if (L == 0) throw std::invalid_argument("tree_stage_aabb: build the tree first");
         t.big_leaves.resize(std::max<u32>(L, 1));
         u32 *n_big = t.counters.data() + 7;
-        fill_u32(s, n_big, 0, 1);
+        if (t.big_listed) fill_u32(s, n_big, 0, 1); // a second box pass on the same tree
+        t.big_listed = true;
         k_leaf_boxes<<<div_up((u64) L * LEAF_LANES, 256), 256, 0, s>>>(
             L, I, t.reduc_map.data(), t.sort_index.data(), x, y, z, h, htol, t.nodes.data(),
             t.big_leaves.data(), n_big);
         k_big_leaf_boxes<<<std::min<u32>(L, 1024), BIG_BLOCK, 0, s>>>(
             I, t.reduc_map.data(), t.sort_index.data(), x, y, z, h, htol, t.nodes.data(),
             t.big_leaves.data(), n_big);
-        if (I > 0) {
-            // internal boxes band by band, deepest first (the kernel boundary between two
-            // bands orders the writes of one band before the reads of the next)
-            u32 *err = t.counters.data() + 5;
-            k_node_depth<<<std::min<u32>(1024, div_up(I, 256)), 256, 0, s>>>(
-                I, t.parent.data(), t.depth.data(), err);
-            static_assert(MERGE_LEVELS % BAND == 0, "bands tile the merge levels");
-            for (u32 b0 = MERGE_LEVELS; b0 > 0;) {
-                b0 -= BAND;
-                k_merge_band<<<div_up(I, 256), 256, 0, s>>>(I, L, b0, t.depth.data(),
-                                                           t.nodes.data(), err);
-            }
+        // tiers over the leaves, three per launch
+        Tiers tt;
+        tt.n[0] = L;
+        u32 at  = 0;
+        while (tt.n[tt.top] > (u32) WAVE) {
+            const u32 k = tt.top + 1; // at most 10 for a u32 leaf count
+            tt.n[k]     = div_up(tt.n[k - 1], 8);
+            tt.off[k]   = at;
+            at += tt.n[k];
+            tt.top = k;
         }
-        // the flags reach the host with the next synchronisation of the stream (tree_check)
-        t.host.read_async(s, t.counters.data() + 5, 1, 5);
-        t.err_pending = true;
+        t.tt = tt;
+        t.tiers.resize(std::max<size_t>((size_t) at * NODE_F64, 1));
+        auto rec = [&](u32 k) -> f64 * {
+            return k <= tt.top ? t.tiers.data() + (size_t) tt.off[k] * NODE_F64 : nullptr;
+        };
+        for (u32 k = 0; k < tt.top; k += 3)
+            k_leaf_tiers<<<div_up(tt.n[k], TIER_BLK), TIER_BLK, 0, s>>>(
+                tt.n[k], k ? rec(k) : t.nodes.data() + (size_t) I * NODE_F64, rec(k + 1),
+                rec(k + 2), rec(k + 3));
+        if (I > 0)
+            k_cell_boxes<<<div_up(I, 256), 256, 0, s>>>(L, t.endrange.data(), t.tiers.data(), tt,
+                                                       t.nodes.data());
         SHAMX_HIP(hipGetLastError());
-    }
-
-    void tree_check(TreeBuffers &t) {
-        if (!t.err_pending) return;
-        t.err_pending = false;
-        const u32 e   = t.host[5];
-        if (e & 1u) throw std::runtime_error("tree build: broken parent links");
-        if (e & 2u) throw std::runtime_error("tree build: child index out of range");
-        if (e & 4u) throw std::runtime_error("tree build: internal cell deeper than 31");
     }
 
     void tree_stage_finish(hipStream_t s, TreeBuffers &t, const f64 *x, const f64 *y,

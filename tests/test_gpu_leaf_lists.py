@@ -88,6 +88,40 @@ def test_leaf_lists_and_owners(n, level, outliers):
         assert own[a] == inside[-1]
 
 
+@pytest.mark.parametrize("n,level", [(2, 0), (8, 0), (9, 0), (64, 0), (65, 0), (512, 0), (513, 0),
+                                     (4097, 0), (4608, 0), (33_000, 0), (20_000, 3)])
+def test_internal_boxes(n, level):
+    """Box and largest rint of every internal cell against the leaves of its range (from its
+    index to endrange): min and max, so exactly equal."""
+    say(f"[internal_boxes] n={n} level={level}")
+    rng = np.random.default_rng(n)
+    pos = rng.normal(0, 1, (n, 3))
+    h = rng.uniform(0.01, 0.1, n)
+    t = [dev(a) for a in (*pos.T, h)]
+    ctx = C.c_void_p()
+    check(lib().shamx_ctx_create(C.byref(ctx)))
+    s = torch.cuda.current_stream().cuda_stream
+    check(lib().shamx_tree_build(ctx, s, n, *[a.data_ptr() for a in t], level, 1.1))
+    sz = (C.c_uint32 * 4)()
+    check(lib().shamx_tree_sizes(ctx, sz))
+    L, I = sz[1], sz[2]
+    end = torch.zeros(max(I, 1), dtype=torch.int32, device="cuda")
+    box = [torch.zeros(3 * (I + L), dtype=torch.float64, device="cuda") for _ in range(2)]
+    rint = torch.zeros(I + L, dtype=torch.float64, device="cuda")
+    check(lib().shamx_tree_get(ctx, s, *[None] * 7, end.data_ptr(), box[0].data_ptr(),
+                               box[1].data_ptr(), rint.data_ptr()))
+    torch.cuda.synchronize()
+    lib().shamx_ctx_destroy(ctx)
+    lo, hi = (b.cpu().numpy().reshape(-1, 3) for b in box)
+    r, end = rint.cpu().numpy(), end.cpu().numpy()
+    assert r[0] == h.max() * 1.1
+    for i in range(I):
+        a, b = min(i, end[i]), max(i, end[i]) + 1
+        assert np.array_equal(lo[i], lo[I + a:I + b].min(0)), i
+        assert np.array_equal(hi[i], hi[I + a:I + b].max(0)), i
+        assert r[i] == r[I + a:I + b].max(), i
+
+
 def test_nan_position_is_refused():
     """A particle with a NaN coordinate lies in no leaf box: the build raises, as the reference's
     search finds no owner for it."""
