@@ -21,10 +21,6 @@ namespace shamx {
     size_t scan_scratch_bytes(u32 n);
     void exclusive_scan_u32(hipStream_t s, const u32 *in, u32 *out, u32 n, u32 *total,
                             void *scratch);
-    // the same over the first min(n_max, *n_dev) values, a length known on the device only
-    // (no synchronisation; scratch sized for n_max)
-    void exclusive_scan_u32_devn(hipStream_t s, const u32 *in, u32 *out, u32 n_max,
-                                 const u32 *n_dev, u32 *total, void *scratch);
 
     // ------------------------------------------------------------------ tree.hip
     // bounding box of n positions widened outward by one ulp (BuildTrees.cpp:38-55);
@@ -56,7 +52,7 @@ namespace shamx {
         DevArray<u32> sort_index;      // n_obj permutation (map_morton_id_to_obj_id)
         DevArray<u32> keys_alt, vals_alt;
         DevArray<u32> split_a, split_b;
-        DevArray<u32> red_cnt, red_pos; // leaf reduction: flags before i, flagged indices
+        DevArray<u32> red_cnt, red_pos; // leaf reduction: kept entries per tile, list
         DevArray<u32> big_leaves;       // leaves too large for the lane-group box kernel
         DevArray<u32> reduc_map;       // L + 2
         DevArray<u32> leaf_codes;      // L

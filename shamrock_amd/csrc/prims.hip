@@ -44,10 +44,8 @@ namespace shamx {
         }
 
         __global__ void __launch_bounds__(SCAN_BLOCK)
-            k_tile_sums(const u32 *__restrict in, u32 n, u32 *__restrict tile_sums,
-                        const u32 *__restrict n_dev) {
+            k_tile_sums(const u32 *__restrict in, u32 n, u32 *__restrict tile_sums) {
             __shared__ u32 lds_waves[SCAN_BLOCK / WAVE];
-            if (n_dev) n = min(n, *n_dev); // the length known on the device only
             u64 base = (u64) blockIdx.x * SCAN_TILE;
             u32 s = 0;
 #pragma unroll
@@ -78,10 +76,9 @@ namespace shamx {
 
         __global__ void __launch_bounds__(SCAN_BLOCK)
             k_scan_tiles_apply(const u32 *__restrict in, u32 *__restrict out, u32 n,
-                               const u32 *__restrict tile_base, const u32 *__restrict n_dev) {
+                               const u32 *__restrict tile_base) {
             __shared__ u32 tile[SCAN_TILE];
             __shared__ u32 lds_waves[SCAN_BLOCK / WAVE];
-            if (n_dev) n = min(n, *n_dev);
             u64 base = (u64) blockIdx.x * SCAN_TILE;
             if (base >= n) return; // block-uniform
 #pragma unroll
@@ -120,11 +117,9 @@ namespace shamx {
         constexpr u32 FUSED_TILES = 4096;
         __global__ void __launch_bounds__(SCAN_BLOCK)
             k_scan_apply_fused(const u32 *__restrict in, u32 *__restrict out, u32 n,
-                               const u32 *__restrict tile_sums, u32 nt, u32 *__restrict total,
-                               const u32 *__restrict n_dev) {
+                               const u32 *__restrict tile_sums, u32 nt, u32 *__restrict total) {
             __shared__ u32 tile[SCAN_TILE];
             __shared__ u32 lds_waves[SCAN_BLOCK / WAVE];
-            if (n_dev) n = min(n, *n_dev);
             u32 base = 0;
             if (tile_sums) {
                 const u32 lim = blockIdx.x == 0 ? nt : blockIdx.x;
@@ -173,26 +168,6 @@ namespace shamx {
             }
         }
 
-        // the scan of in[0, n) with n <= n_max, n read from n_dev when it is not null
-        void scan_impl(hipStream_t s, const u32 *in, u32 *out, u32 n_max, const u32 *n_dev,
-                       u32 *total, void *scratch) {
-            u32 nt         = div_up(n_max, SCAN_TILE);
-            u32 *tile_sums = (u32 *) scratch;
-            if (nt == 1) {
-                k_scan_apply_fused<<<1, SCAN_BLOCK, 0, s>>>(in, out, n_max, nullptr, 1, total,
-                                                            n_dev);
-            } else if (nt <= FUSED_TILES) {
-                k_tile_sums<<<nt, SCAN_BLOCK, 0, s>>>(in, n_max, tile_sums, n_dev);
-                k_scan_apply_fused<<<nt, SCAN_BLOCK, 0, s>>>(in, out, n_max, tile_sums, nt,
-                                                             total, n_dev);
-            } else {
-                k_tile_sums<<<nt, SCAN_BLOCK, 0, s>>>(in, n_max, tile_sums, n_dev);
-                k_scan_tiles<<<1, SCAN_BLOCK, 0, s>>>(tile_sums, nt, total);
-                k_scan_tiles_apply<<<nt, SCAN_BLOCK, 0, s>>>(in, out, n_max, tile_sums, n_dev);
-            }
-            SHAMX_HIP(hipGetLastError());
-        }
-
         template<class T>
         void fill_impl(hipStream_t s, T *p, T v, size_t n) {
             if (n == 0) return;
@@ -214,16 +189,19 @@ namespace shamx {
             if (total) fill_u32(s, total, 0, 1);
             return;
         }
-        scan_impl(s, in, out, n, nullptr, total, scratch);
-    }
-
-    void exclusive_scan_u32_devn(hipStream_t s, const u32 *in, u32 *out, u32 n_max,
-                                 const u32 *n_dev, u32 *total, void *scratch) {
-        if (n_max == 0) {
-            if (total) fill_u32(s, total, 0, 1);
-            return;
+        const u32 nt   = div_up(n, SCAN_TILE);
+        u32 *tile_sums = (u32 *) scratch;
+        if (nt == 1) {
+            k_scan_apply_fused<<<1, SCAN_BLOCK, 0, s>>>(in, out, n, nullptr, 1, total);
+        } else if (nt <= FUSED_TILES) {
+            k_tile_sums<<<nt, SCAN_BLOCK, 0, s>>>(in, n, tile_sums);
+            k_scan_apply_fused<<<nt, SCAN_BLOCK, 0, s>>>(in, out, n, tile_sums, nt, total);
+        } else {
+            k_tile_sums<<<nt, SCAN_BLOCK, 0, s>>>(in, n, tile_sums);
+            k_scan_tiles<<<1, SCAN_BLOCK, 0, s>>>(tile_sums, nt, total);
+            k_scan_tiles_apply<<<nt, SCAN_BLOCK, 0, s>>>(in, out, n, tile_sums);
         }
-        scan_impl(s, in, out, n_max, n_dev, total, scratch);
+        SHAMX_HIP(hipGetLastError());
     }
 
 } // namespace shamx

@@ -21,6 +21,7 @@
 
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 
 namespace shamx {
 
@@ -404,66 +405,131 @@ namespace shamx {
             return ((u32) y > len - 1 || y < 0) ? -1 : clz32(m[x] ^ m[y]);
         }
 
-        __global__ void k_split(u32 n, const u32 *__restrict m, u32 *__restrict s) {
-            u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-            if (i >= n) return;
-            s[i] = (i > 0) ? (m[i - 1] != m[i] ? 1u : 0u) : 1u;
-        }
-
-        // sycl_reduction_iteration (NEW_BEHAVIOR), reduction_alg.cpp:196-244.  The reference
-        // walks from i to the nearest set flags on either side, which is linear in the run
-        // length (runs of equal codes are long in clustered sets); here the flagged indices
-        // are compacted first (F, with cnt[i] = flags before i and *total flags in all), so
-        // the walks become lookups with the same results, including the wrapped u32 values
-        // (-1, -2) the walks stop at when no flag is left.
-        __global__ void k_reduc_iter(u32 n, const u32 *__restrict m, const u32 *__restrict s_in,
-                                     const u32 *__restrict cnt, const u32 *__restrict F,
-                                     const u32 *__restrict total, u32 *__restrict s_out) {
-            u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-            if (i >= n) return;
-            const u32 c = cnt[i], K = *total;
-            u32 before1 = c >= 1 ? F[c - 1] : 0xFFFFFFFFu;
-            u32 before2 = c >= 2 ? F[c - 2] : (c == 1 ? 0xFFFFFFFFu : 0xFFFFFFFEu);
-            const u32 ci = c + (s_in[i] ? 1u : 0u);
-            u32 next1    = ci < K ? F[ci] : n;
-            i32 d0  = kdelta((i32) i, (i32) next1, n, m);
-            i32 dm  = kdelta((i32) i, (i32) before1, n, m);
-            i32 dmm = kdelta((i32) before1, (i32) before2, n, m);
-            s_out[i] = (!(d0 < dm && dmm < dm) && s_in[i]) ? 1u : 0u;
-        }
-
-        // sycl_reduction_iteration on the compacted list of kept positions: F[0..K) are the
-        // positions whose split flag is set (K on the device); keep[j] is F[j]'s new flag.  The
-        // reference walks from F[j] to the nearest set flags on either side (reduction_alg.cpp:
-        // 196-244): those are F[j - 1], F[j - 2] and F[j + 1], with the wrapped u32 values
+        // The leaf reduction works on the compacted list of kept positions, F[0..K) (K on the
+        // device).  FIRST: the list is all n positions, and the kept ones are the split
+        // positions, where the code changes.  Else one sycl_reduction_iteration (NEW_BEHAVIOR,
+        // reduction_alg.cpp:196-244): the reference walks from F[j] to the nearest set flags on
+        // either side, which is linear in the run length (runs of equal codes are long in
+        // clustered sets); those are F[j - 1], F[j - 2] and F[j + 1], with the wrapped u32 values
         // (-1, -2) the walks stop at when no flag is left before, and n when none is after.
-        __global__ void k_reduc_keep(u32 n, const u32 *__restrict m, const u32 *__restrict F,
-                                     const u32 *__restrict K_dev, u32 *__restrict keep) {
-            const u32 j = blockIdx.x * blockDim.x + threadIdx.x;
-            const u32 K = *K_dev;
-            if (j >= K) return;
-            const u32 i       = F[j];
-            const u32 before1 = j >= 1 ? F[j - 1] : 0xFFFFFFFFu;
-            const u32 before2 = j >= 2 ? F[j - 2] : (j == 1 ? 0xFFFFFFFFu : 0xFFFFFFFEu);
-            const u32 next1   = j + 1 < K ? F[j + 1] : n;
-            i32 d0  = kdelta((i32) i, (i32) next1, n, m);
-            i32 dm  = kdelta((i32) i, (i32) before1, n, m);
-            i32 dmm = kdelta((i32) before1, (i32) before2, n, m);
-            keep[j] = !(d0 < dm && dmm < dm) ? 1u : 0u;
-        }
-        // F_out[off[j]] = F_in[j] for the kept j < K (K on the device)
-        __global__ void k_compact_list(const u32 *__restrict K_dev, const u32 *__restrict keep,
-                                       const u32 *__restrict off, const u32 *__restrict F_in,
-                                       u32 *__restrict F_out) {
-            const u32 j = blockIdx.x * blockDim.x + threadIdx.x;
-            if (j < *K_dev && keep[j]) F_out[off[j]] = F_in[j];
+        template<bool FIRST>
+        __device__ inline bool reduc_keep(u32 j, u32 n, u32 K, const u32 *__restrict m,
+                                          const u32 *__restrict F) {
+            if (j >= K) return false;
+            if constexpr (FIRST) {
+                return j == 0 || m[j - 1] != m[j];
+            } else {
+                const u32 i       = F[j];
+                const u32 before1 = j >= 1 ? F[j - 1] : 0xFFFFFFFFu;
+                const u32 before2 = j >= 2 ? F[j - 2] : (j == 1 ? 0xFFFFFFFFu : 0xFFFFFFFEu);
+                const u32 next1   = j + 1 < K ? F[j + 1] : n;
+                i32 d0  = kdelta((i32) i, (i32) next1, n, m);
+                i32 dm  = kdelta((i32) i, (i32) before1, n, m);
+                i32 dmm = kdelta((i32) before1, (i32) before2, n, m);
+                return !(d0 < dm && dmm < dm);
+            }
         }
 
-        __global__ void k_compact(u32 n, const u32 *__restrict flag, const u32 *__restrict off,
-                                  u32 *__restrict map) {
-            u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-            if (i >= n) return;
-            if (flag[i]) map[off[i]] = i;
+        // One iteration is two launches over tiles of the list: the kept entries
+        // of every tile, then their compaction, a block adding the counts of the tiles before
+        // its own (a few cached loads per thread) and testing its entries again, which is
+        // cheaper than a pass over stored flags.  (Flags, a two-launch scan and a compaction
+        // were four launches per iteration, each a few microseconds at any size below a few
+        // hundred thousand.)  A list of one tile needs the second launch only.
+        // Tiles of 1024 entries up to 2^23 (2.46 M positions: 67 us for the four iterations
+        // against 114 us with tiles of 4096, whose 600 blocks leave the chip half empty, and
+        // about 130 us for the sixteen launches before), 4096 beyond, where adding the counts of
+        // the earlier tiles, quadratic in their number, would weigh more.
+        constexpr int RED_BLK       = 256;
+        constexpr u32 RED_SMALL_MAX = 1u << 23;
+        template<bool FIRST, int RED_ITEMS>
+        __global__ void __launch_bounds__(RED_BLK)
+            k_reduc_count(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
+                          const u32 *__restrict F, u32 *__restrict tile_cnt) {
+            __shared__ u32 part[RED_BLK / WAVE];
+            const u32 K = FIRST ? n : min(*K_dev, n);
+            const u32 t0 = blockIdx.x * (RED_BLK * RED_ITEMS);
+            u32 c = 0;
+            if (t0 < K) {
+#pragma unroll 4
+                for (int k = 0; k < RED_ITEMS; k++)
+                    c += (u32) __popcll(__ballot(
+                        reduc_keep<FIRST>(t0 + k * RED_BLK + threadIdx.x, n, K, m, F)));
+            }
+            if (__lane_id() == 0) part[threadIdx.x / WAVE] = c;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                for (int w = 1; w < RED_BLK / WAVE; w++) c += part[w];
+                tile_cnt[blockIdx.x] = c;
+            }
+        }
+        template<bool FIRST, int RED_ITEMS>
+        __global__ void __launch_bounds__(RED_BLK)
+            k_reduc_compact(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
+                            const u32 *__restrict F, const u32 *__restrict tile_cnt, u32 nt,
+                            u32 *__restrict F_out, u32 *__restrict K_out,
+                            u32 *__restrict K_copy) {
+            constexpr int NW = RED_BLK / WAVE;
+            __shared__ u32 part[NW];
+            __shared__ u32 cnt[RED_ITEMS * NW]; // kept entries per 64 of the tile, then before it
+            const u32 K    = FIRST ? n : min(*K_dev, n);
+            const u32 t0   = blockIdx.x * (RED_BLK * RED_ITEMS);
+            const u32 lane = (u32) __lane_id(), wid = threadIdx.x / WAVE;
+            // kept entries of the earlier tiles; block 0 counts all of them for the total
+            u32 before = 0;
+            if (nt > 1) {
+                const u32 lim = blockIdx.x == 0 ? nt : blockIdx.x;
+#pragma unroll 4
+                for (u32 i = threadIdx.x; i < lim; i += RED_BLK) before += tile_cnt[i];
+                before = wave_reduce(before, [](u32 p, u32 q) { return p + q; });
+                if (lane == 0) part[wid] = before;
+                __syncthreads();
+                before = 0;
+                for (int w = 0; w < NW; w++) before += part[w];
+                if (blockIdx.x == 0) {
+                    if (threadIdx.x == 0) {
+                        *K_out = before;
+                        if (K_copy) *K_copy = before;
+                    }
+                    before = 0;
+                }
+            }
+            if (t0 >= K) { // block-uniform
+                if (nt == 1 && threadIdx.x == 0) {
+                    *K_out = 0;
+                    if (K_copy) *K_copy = 0;
+                }
+                return;
+            }
+            u64 bal[RED_ITEMS];
+#pragma unroll
+            for (int k = 0; k < RED_ITEMS; k++) {
+                bal[k] = __ballot(reduc_keep<FIRST>(t0 + k * RED_BLK + threadIdx.x, n, K, m, F));
+                if (lane == 0) cnt[k * NW + wid] = (u32) __popcll(bal[k]);
+            }
+            __syncthreads();
+            static_assert(RED_ITEMS * NW <= WAVE, "one wave scans the counts");
+            if (wid == 0) {
+                const u32 v = lane < RED_ITEMS * NW ? cnt[lane] : 0u;
+                u32 inc     = v;
+                for (int o = 1; o < WAVE; o <<= 1) {
+                    u32 t = __shfl_up(inc, o, WAVE);
+                    if ((int) lane >= o) inc += t;
+                }
+                if (lane < RED_ITEMS * NW) cnt[lane] = inc - v;
+                if (nt == 1 && lane == WAVE - 1) {
+                    *K_out = inc;
+                    if (K_copy) *K_copy = inc;
+                }
+            }
+            __syncthreads();
+            const u64 lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+            for (int k = 0; k < RED_ITEMS; k++) {
+                if (!((bal[k] >> lane) & 1ull)) continue;
+                const u32 j = t0 + k * RED_BLK + threadIdx.x;
+                F_out[before + cnt[k * NW + wid] + (u32) __popcll(bal[k] & lt)] = FIRST ? j : F[j];
+            }
         }
 
         // update_morton_buf tail (reduction_alg.cpp:274-295) + remap (:564-585)
@@ -885,29 +951,37 @@ namespace shamx {
         // leaf reduction (reduction_alg.cpp:413-456) on the compacted list of split positions:
         // each iteration tests the positions still kept and compacts them, so it costs the
         // number of kept positions, not n (the lengths stay on the device: no host round trip)
-        u32 g = div_up(n, 256);
-        k_split<<<g, 256, 0, s>>>(n, t.sorted.data(), t.split_a.data());
-        t.red_cnt.resize(std::max<u32>(n, 1));
+        const bool small = n <= RED_SMALL_MAX;
+        const u32 nt     = div_up(n, RED_BLK * (small ? 4 : 16));
+        t.red_cnt.resize(nt);
         t.red_pos.resize(std::max<u32>(n, 1));
         u32 *distinct = t.counters.data() + 1; // distinct codes (positions where codes change)
         u32 *L_dev    = t.counters.data() + 0;
         u32 *K_tmp[2] = {t.counters.data() + 8, t.counters.data() + 9};
-        exclusive_scan_u32(s, t.split_a.data(), t.red_cnt.data(), n, distinct, t.scratch.data());
+        auto iterate = [&](auto first, const u32 *K_in, const u32 *F_in, u32 *F_out, u32 *K_out,
+                           u32 *K_copy) {
+            constexpr bool FIRST = decltype(first)::value;
+            auto go              = [&](auto items) {
+                constexpr int IT = decltype(items)::value;
+                if (nt > 1)
+                    k_reduc_count<FIRST, IT><<<nt, RED_BLK, 0, s>>>(
+                        n, K_in, t.sorted.data(), F_in, t.red_cnt.data());
+                k_reduc_compact<FIRST, IT><<<nt, RED_BLK, 0, s>>>(
+                    n, K_in, t.sorted.data(), F_in, t.red_cnt.data(), nt, F_out, K_out, K_copy);
+            };
+            if (small) go(std::integral_constant<int, 4>{});
+            else go(std::integral_constant<int, 16>{});
+        };
         u32 *F_in = reduction_level > 0 ? t.red_pos.data() : t.reduc_map.data();
-        k_compact<<<g, 256, 0, s>>>(n, t.split_a.data(), t.red_cnt.data(), F_in);
+        iterate(std::true_type{}, nullptr, nullptr, F_in, distinct,
+                reduction_level == 0 ? L_dev : nullptr);
         const u32 *K_in = distinct;
-        if (reduction_level == 0)
-            SHAMX_HIP(hipMemcpyAsync(L_dev, distinct, sizeof(u32), hipMemcpyDeviceToDevice, s));
         for (u32 it = 1; it <= reduction_level; it++) {
             const bool last = it == reduction_level;
             u32 *F_out = last ? t.reduc_map.data()
                               : (F_in == t.red_pos.data() ? t.split_b.data() : t.red_pos.data());
             u32 *K_out = last ? L_dev : K_tmp[it % 2];
-            k_reduc_keep<<<g, 256, 0, s>>>(n, t.sorted.data(), F_in, K_in, t.split_a.data());
-            exclusive_scan_u32_devn(s, t.split_a.data(), t.red_cnt.data(), n, K_in, K_out,
-                                    t.scratch.data());
-            k_compact_list<<<g, 256, 0, s>>>(K_in, t.split_a.data(), t.red_cnt.data(), F_in,
-                                             F_out);
+            iterate(std::false_type{}, K_in, F_in, F_out, K_out, nullptr);
             F_in = F_out;
             K_in = K_out;
         }
