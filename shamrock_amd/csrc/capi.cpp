@@ -164,14 +164,12 @@ struct shamx_solver {
     // per-particle gathers of the tree, records and outputs read and write nearly contiguous
     // memory.  pid[j] = particle id (the caller's order) of storage slot j; field getters and
     // setters and the inspection getters translate, so every result keeps the caller's order.
-    DevArray<u32> pid, pid_tmp, reo_perm, reo_flag, reo_off, reo_count;
-    // the next step's reorder, prepared after the step's last tree build: reo_perm holds the
-    // permutation and reo_moved (read with the corrector's reductions, no sync of its own) how
-    // many particles it moves; reo_known says both describe the current storage and tree
-    u32 reo_moved  = 0;
+    DevArray<u32> pid, pid_tmp;
+    // the next step's reorder: the neighbour build leaves its permutation in nb.perm and the
+    // number of particles it moves in nb.moved; reo_known says both describe the current
+    // storage and tree
     bool reo_known = false;
-    DevArray<unsigned char> reo_scan;
-    DevArray<f64> tmp_f64;
+    DevArray<f64> tmp_f64, reo_tmp[GATHER_MAX];
     bool pid_identity = true; // pid[j] = j (nothing reordered yet)
     bool tree_valid   = false; // tree.sort_index describes the current storage
     DevArray<unsigned char> frec; // force records, sorted order
@@ -235,38 +233,24 @@ struct shamx_solver {
     }
 
     // the permutation from the storage to the last tree's sorted order of the local particles
-    // (in reo_perm), and whether the storage is far enough from it to reorder: the reorder
+    // (in nb.perm), and whether the storage is far enough from it to reorder: the reorder
     // moves every field (22 gathers, about 0.2 ms at 2.1 M particles), so it waits until at
     // least 1/32 of the particles have changed places since the last one
     bool pending_reorder() {
         if (cfg.keep_storage_order || !tree_valid || tree.n_obj != N + G || N == 0) return false;
-        if (reo_known) return (u64) reo_moved * 32 >= N;
-        const u32 Nm = N + G;
-        reo_perm.resize(N);
-        reo_flag.resize(Nm);
-        reo_off.resize(Nm);
-        reo_scan.resize(std::max(reo_scan.size(), scan_scratch_bytes(Nm)));
-        local_sorted_order(stream, Nm, N, tree.sort_index.data(), reo_perm.data(),
-                           reo_flag.data(), reo_off.data(), reo_scan.data());
-        const u32 moved = perm_moved(stream, N, reo_perm.data(), reo_flag.data(), hostc.data());
-        return (u64) moved * 32 >= N;
-    }
-
-    // after the step's last tree build: the permutation of the next reorder and its count of
-    // moved particles on the device (the count is read with the corrector's reductions)
-    bool prepare_reorder() {
-        reo_known = false;
-        if (cfg.keep_storage_order || !tree_valid || tree.n_obj != N + G || N == 0) return false;
-        const u32 Nm = N + G;
-        reo_perm.resize(N);
-        reo_flag.resize(Nm);
-        reo_off.resize(Nm);
-        reo_count.resize(1);
-        reo_scan.resize(std::max(reo_scan.size(), scan_scratch_bytes(Nm)));
-        local_sorted_order(stream, Nm, N, tree.sort_index.data(), reo_perm.data(),
-                           reo_flag.data(), reo_off.data(), reo_scan.data());
-        perm_moved_async(stream, N, reo_perm.data(), reo_count.data());
-        return true;
+        if (!reo_known) { // a step that ended with an error after its tree build
+            nb.lpos.resize(N);
+            nb.perm.resize(N);
+            nb.counters.resize(16);
+            fill_u32(stream, nb.counters.data() + 3, 0, 1);
+            local_rows(stream, N + G, N, tree.sort_index.data(), nb.lpos.data(), nb.perm.data(),
+                       nb.counters.data() + 3, nb.tile_cnt);
+            hostc.read_async(stream, nb.counters.data() + 3, 1);
+            SHAMX_HIP(hipStreamSynchronize(stream));
+            nb.moved  = hostc[0];
+            reo_known = true;
+        }
+        return (u64) nb.moved * 32 >= N;
     }
 
     // permute every per-particle field of the local particles into the sorted order of the
@@ -275,12 +259,23 @@ struct shamx_solver {
         const bool go = pending_reorder();
         reo_known     = false;
         if (!go) return;
-        const u32 *perm = reo_perm.data();
-        for (auto *f : {&x, &y, &z, &h, &vx, &vy, &vz, &u, &ax, &ay, &az, &du, &alpha_av,
-                        &soundspeed, &divv, &curlx, &curly, &curlz, &dtdivv, &axe, &aye, &aze}) {
-            tmp_f64.resize(f->size()); // same element count: no allocation once sizes settle
-            perm_gather_f64(stream, N, perm, f->data(), tmp_f64.data());
-            f->swap(tmp_f64);
+        const u32 *perm = nb.perm.data();
+        DevArray<f64> *fields[] = {&x,    &y,        &z,          &h,    &vx,    &vy,    &vz,    &u,
+                                   &ax,   &ay,       &az,         &du,   &alpha_av, &soundspeed,
+                                   &divv, &curlx,    &curly,      &curlz, &dtdivv, &axe,   &aye,
+                                   &aze};
+        constexpr int nf = (int) (sizeof(fields) / sizeof(fields[0]));
+        for (int f0 = 0; f0 < nf; f0 += GATHER_MAX) {
+            GatherPtrs g{};
+            g.n = std::min(GATHER_MAX, nf - f0);
+            for (int k = 0; k < g.n; k++) {
+                // same element count: no allocation once sizes settle
+                reo_tmp[k].resize(fields[f0 + k]->size());
+                g.src[k] = fields[f0 + k]->data();
+                g.dst[k] = reo_tmp[k].data();
+            }
+            perm_gather_fields(stream, N, perm, g);
+            for (int k = 0; k < g.n; k++) fields[f0 + k]->swap(reo_tmp[k]);
         }
         if (pid_identity) {
             std::vector<u32> iota(N);
@@ -302,7 +297,7 @@ struct shamx_solver {
     std::vector<u32> next_storage_order() {
         if (!pending_reorder()) return host_pid();
         std::vector<u32> perm(N), p = host_pid(), out(N);
-        SHAMX_HIP(hipMemcpyAsync(perm.data(), reo_perm.data(), N * sizeof(u32),
+        SHAMX_HIP(hipMemcpyAsync(perm.data(), nb.perm.data(), N * sizeof(u32),
                                  hipMemcpyDeviceToHost, stream));
         SHAMX_HIP(hipStreamSynchronize(stream));
         for (u32 j = 0; j < N; j++) out[j] = p[perm[j]];
@@ -439,7 +434,8 @@ struct shamx_solver {
     // require_converged false, a last subcycle that did not converge is kept as it is (h of
     // the unconverged particles clamped to the cache radius) instead of failing the step.
     void prestep(u32 max_sub, bool require_converged) {
-        reo_known = false; // the tree built here replaces the one a prepared reorder follows
+        reo_known    = false; // the tree built here replaces the one a prepared reorder follows
+        nb.want_perm = !cfg.keep_storage_order;
         u32 hstep = 0, hmax = max_sub;
         last.h_iterations = 0;
         for (; hstep < hmax; hstep++) {
@@ -484,6 +480,7 @@ struct shamx_solver {
             break;
         }
         last.subcycles = std::min(hstep + 1, hmax);
+        reo_known      = !cfg.keep_storage_order; // of the last subcycle's tree
         if (hstep == hmax) throw std::runtime_error("the h iterator is not converged");
         int b = timer.begin(stream);
         // final h of the images and in the sorted records, then Omega fused with the force
@@ -582,7 +579,6 @@ struct shamx_solver {
         }
         (void) box6;
         prestep((u32) cfg.h_max_subcycles, true);
-        const bool count_pending = prepare_reorder();
 
         f64 next_cfl = 0;
         u32 corr_iter = 0;
@@ -648,12 +644,7 @@ struct shamx_solver {
             timer.end(stream, PH_CORR, b);
             const u64 *k = hostw.data();
             hostw.read_async(stream, red.data() + 3, 5);
-            if (count_pending) hostc.read_async(stream, reo_count.data(), 1, 2);
             SHAMX_HIP(hipStreamSynchronize(stream));
-            if (count_pending) {
-                reo_moved = hostc[2];
-                reo_known = true;
-            }
             f64 dt_min         = ordered_to_f64(k[0]);
             last.n_interacting = k[4];
             f64 max_e2 = ordered_to_f64(k[1]);

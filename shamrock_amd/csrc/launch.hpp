@@ -101,7 +101,11 @@ namespace shamx {
         DevArray<u32> cnt, offset, ids;
         DevArray<u32> lpos;                             // sorted layout: local rows in order
         DevArray<u32> fcnt, fids;                       // force-interacting subsequences
-        DevArray<u32> lflag, lscan;
+        // sorted layout: the particles of the local rows in order (the permutation of a storage
+        // reorder; on request), and how many of them are not at their own index
+        DevArray<u32> perm, tile_cnt;
+        bool want_perm = false;
+        u32 moved      = 0;
         DevArray<u32> lap;   // per leaf: a later leaf's box meets its box
         // sorted layout: one pass per stage into rows of fixed capacity; leaf l's list at
         // leaf_ids[l * leaf_stride], row r at ids[r * row_stride] (0: packed layout).  The
@@ -110,7 +114,7 @@ namespace shamx {
         DevArray<double4> ps;                           // (x, y, z, h) in sorted order
         DevArray<u32> inv;                              // sorted position of each object
         DevArray<u32> mism;                             // owner leaf != own leaf
-        DevArray<u32> nbatch, bstart, item_leaf;        // stage-2 wave items (member batches)
+        DevArray<u32> xstart, item_leaf;                // stage-2 wave items (member batches)
         DevArray<f64> bbox; // member batch boxes (batch-level cull on clustered sets)
         // rows past their fixed capacity: flags, counts, positions, list (overflow region)
         DevArray<u32> oflag, ocnt, ofpos, opos, olist;
@@ -125,6 +129,11 @@ namespace shamx {
     void neigh_build(hipStream_t s, NeighBuffers &nb, TreeBuffers &t, u32 n_local,
                      const f64 *x, const f64 *y, const f64 *z, const f64 *h, f64 htol,
                      f64 Rkern, bool sorted_layout);
+
+    // the sorted positions of the local particles (< n) in order into lpos; with perm, those
+    // particles, and *moved += the ones that are not at their own index
+    void local_rows(hipStream_t s, u32 nm, u32 n, const u32 *sort_index, u32 *lpos, u32 *perm,
+                    u32 *moved, DevArray<u32> &tile_cnt);
 
     // ------------------------------------------------------------------ sph.hip
     // Neighbour CSR as the pair loops read it.  Particle j of a launch (j < n) reads row
@@ -265,16 +274,15 @@ namespace shamx {
         int n;
     };
     void gather_ghosts(hipStream_t s, u32 n, u32 G, const u32 *ghost_src, FieldPtrs fields);
-    // perm[j] = the j-th local index (< n) of the sorted order sort_index[0..nm) (flag, off:
-    // nm words of work space, scan_scratch: scan_scratch_bytes(nm))
-    void local_sorted_order(hipStream_t s, u32 nm, u32 n, const u32 *sort_index, u32 *perm,
-                            u32 *flag, u32 *off, void *scan_scratch);
     // dst[j] = src[perm[j]] (gather) and dst[perm[j]] = src[j] (scatter), j < n
-    // entries of perm[0..n) that differ from their index (synchronises to return the count;
-    // count_host: one pinned word)
-    u32 perm_moved(hipStream_t s, u32 n, const u32 *perm, u32 *count_dev, u32 *count_host);
-    // the same count left in *count_dev (no synchronisation)
-    void perm_moved_async(hipStream_t s, u32 n, const u32 *perm, u32 *count_dev);
+    // the same gather of up to GATHER_MAX fields in one launch
+    constexpr int GATHER_MAX = 8;
+    struct GatherPtrs {
+        const f64 *src[GATHER_MAX];
+        f64 *dst[GATHER_MAX];
+        int n;
+    };
+    void perm_gather_fields(hipStream_t s, u32 n, const u32 *perm, const GatherPtrs &g);
     void perm_gather_f64(hipStream_t s, u32 n, const u32 *perm, const f64 *src, f64 *dst);
     void perm_scatter_f64(hipStream_t s, u32 n, const u32 *perm, const f64 *src, f64 *dst);
     void perm_gather_u32(hipStream_t s, u32 n, const u32 *perm, const u32 *src, u32 *dst);

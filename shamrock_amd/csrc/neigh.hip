@@ -10,6 +10,7 @@
 // Each list is built with a count pass, an exclusive scan and a fill pass that walks the same
 // candidates in the same order, so lists (and their order) are deterministic and identical to
 // the reference algorithm.  Traversal: KarrasTreeTraverser.hpp:69-118 (left child first).
+#include "compact.hpp"
 #include "launch.hpp"
 #include "tree_layout.hpp"
 
@@ -258,32 +259,57 @@ namespace shamx {
             offset[i]     = base + opos[i];
         }
 
+        // Member batches: a batch is 64 consecutive sorted positions of a leaf.  Item l < L is the
+        // first batch of leaf l, the further ones of larger leaves follow after the L first ones,
+        // those of a leaf together (xstart: its first), in the order the leaves come by
+        __device__ inline u32 item_batch(u32 item, u32 l, u32 L, const u32 *__restrict xstart) {
+            return item < L ? 0u : item - xstart[l] + 1;
+        }
+        __device__ inline u32 batch_item(u32 b, u32 l, const u32 *__restrict xstart) {
+            return b == 0 ? l : xstart[l] + b - 1;
+        }
+        __global__ void k_items(u32 L, u32 I, const f64 *__restrict nodes,
+                                u32 *__restrict item_leaf, u32 *__restrict xstart,
+                                u32 *__restrict n_extra) {
+            u32 l = blockIdx.x * blockDim.x + threadIdx.x;
+            if (l >= L) return;
+            u32 m0, m1;
+            node_children(nodes, I + l, m0, m1);
+            item_leaf[l]  = l;
+            u32 x         = 0;
+            const u32 ext = m1 - m0 > WAVE ? (m1 - m0 - 1) / WAVE : 0u;
+            if (ext) {
+                x = L + atomicAdd(n_extra, ext);
+                for (u32 j = 0; j < ext; j++) item_leaf[x + j] = l;
+            }
+            xstart[l] = x;
+        }
+
         // Owner leaf (:406-451) of every local particle, OWN_LANES lanes per member batch (64
         // sorted positions of a leaf).  The particle's own leaf contains it, so its owner is the
         // last leaf of the own leaf's list whose box contains it (a leaf that contains a
         // particle of this one meets its box and is in its list); leaves whose box no later leaf
-        // meets (lap) own all their particles.  Particles owned by another leaf go to mism, and
-        // lflag (sorted layout) marks the local ones.  leaf_cap: as in stage 2.
+        // meets (lap) own all their particles.  Particles owned by another leaf go to mism.
+        // leaf_cap: as in stage 2.
         constexpr u32 OWN_LANES = 16;
         __global__ void __launch_bounds__(256)
-            k_owner(u32 n, u32 I, const f64 *__restrict nodes, const u32 *__restrict item_leaf,
-                    const u32 *__restrict bstart, const u32 *__restrict n_items,
+            k_owner(u32 n, u32 L, u32 I, const f64 *__restrict nodes,
+                    const u32 *__restrict item_leaf, const u32 *__restrict xstart,
+                    const u32 *__restrict n_extra,
                     const u32 *__restrict sort_index, const double4 *__restrict ps,
                     const u32 *__restrict lap, const u32 *__restrict leaf_cnt,
                     const u32 *__restrict leaf_offset, const u32 *__restrict leaf_ids,
-                    u32 leaf_cap, u32 *__restrict owner, u32 *__restrict lflag,
-                    u32 *__restrict mism, u32 *__restrict mism_len) {
+                    u32 leaf_cap, u32 *__restrict owner, u32 *__restrict mism, u32 *__restrict mism_len) {
             const u32 item = (blockIdx.x * 256 + threadIdx.x) / OWN_LANES;
-            if (item >= *n_items) return;
+            if (item >= L + *n_extra) return;
             const u32 l = item_leaf[item];
             u32 m0, m1;
             node_children(nodes, I + l, m0, m1);
-            m0 += (item - bstart[l]) * WAVE;
+            m0 += item_batch(item, l, L, xstart) * WAVE;
             m1 = min(m1, m0 + WAVE);
             const bool over = lap[l] != 0;
             for (u32 s = m0 + threadIdx.x % OWN_LANES; s < m1; s += OWN_LANES) {
                 const u32 a = sort_index[s];
-                if (lflag) lflag[s] = a < n ? 1u : 0u;
                 if (a >= n) continue;
                 u32 own = l;
                 if (over) {
@@ -357,33 +383,64 @@ namespace shamx {
         }
 
         // sorted copy of positions and h (AoS, 32 B per object) + inverse permutation
-        // (a local particle with a NaN coordinate is inside no leaf box: err bit 2)
+        // (sorted layout: with the row counts set to zero, the rows of images stay empty; a local
+        // particle with a NaN coordinate is inside no leaf box: err bit 2)
         __global__ void k_sorted_copy(u32 nm, u32 n, const u32 *__restrict sort_index,
                                       const f64 *__restrict x, const f64 *__restrict y,
                                       const f64 *__restrict z, const f64 *__restrict h,
                                       double4 *__restrict ps, u32 *__restrict inv,
-                                      u32 *__restrict err) {
+                                      u32 *__restrict cnt, u32 *__restrict err) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
             if (s >= nm) return;
             u32 b           = sort_index[s];
             const double4 q = make_double4(x[b], y[b], z[b], h[b]);
             ps[s]           = q;
             inv[b]          = s;
+            if (cnt) cnt[s] = 0;
             if ((b < n) & ((q.x != q.x) | (q.y != q.y) | (q.z != q.z))) atomicOr(err, 2u);
         }
 
-        // local particles in sorted order, scattered after the scan of their flags
-        __global__ void k_local_scatter(u32 nm, const u32 *__restrict flag,
-                                        const u32 *__restrict pos, u32 *__restrict lpos) {
-            u32 s = blockIdx.x * blockDim.x + threadIdx.x;
-            if (s < nm && flag[s]) lpos[pos[s]] = s;
+        // Sorted layout: the sorted positions of the local particles in order (lpos; perm: the
+        // particles there, moved: how many of them are not at their own index), compacted as in
+        // compact.hpp; without images every position is local
+        template<int ITEMS>
+        __global__ void __launch_bounds__(CT_BLK)
+            k_local_count(u32 nm, u32 n, const u32 *__restrict sort_index,
+                          u32 *__restrict tile_cnt) {
+            tile_count<ITEMS>(nm, tile_cnt, [&](u32 j) { return sort_index[j] < n; });
         }
-
+        template<int ITEMS>
+        __global__ void __launch_bounds__(CT_BLK)
+            k_local_rows(u32 nm, u32 n, const u32 *__restrict sort_index,
+                         const u32 *__restrict tile_cnt, u32 nt, u32 *__restrict lpos,
+                         u32 *__restrict perm, u32 *__restrict moved) {
+            __shared__ u32 part[CT_BLK / WAVE];
+            u32 mv = 0;
+            tile_compact<ITEMS>(
+                nm, tile_cnt, nt, nm == n, [&](u32 j) { return sort_index[j] < n; },
+                [&](u32 p, u32 j) {
+                    lpos[p] = j;
+                    if (perm) {
+                        const u32 a = sort_index[j];
+                        perm[p]     = a;
+                        mv += a != p ? 1u : 0u;
+                    }
+                },
+                [](u32) {});
+            if (!perm) return; // the same for the whole grid
+            mv = wave_reduce(mv, [](u32 a, u32 b) { return a + b; });
+            if (__lane_id() == 0) part[threadIdx.x / WAVE] = mv;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                for (int w = 1; w < CT_BLK / WAVE; w++) mv += part[w];
+                if (mv) atomicAdd(moved, mv);
+            }
+        }
 
         constexpr int GRP_WAVES = 4;
 
         // stage 2, one wave per member batch: a batch is 64 consecutive sorted positions of a
-        // leaf (item_leaf / bstart map the wave to its leaf and batch), its members the local
+        // leaf (item_leaf / xstart map the wave to its leaf and batch), its members the local
         // particles among them whose owner is this leaf; the candidates are the particles of
         // the neighbour leaves, in list order then sorted order.  Candidates are taken 64 at a
         // time; those farther from the members' bounding box than both the members' largest
@@ -393,6 +450,7 @@ namespace shamx {
         // index, position, cut radius).  The wave then tests P candidates x M members per
         // instruction, lane = candidate * M + member, so the kept lanes of one member are in
         // candidate order and its row is the compaction of a ballot restricted to its lanes.
+        // n_items: the batches beyond the leaves' first ones.
         // LIST: one wave per particle of list (item_leaf holds particle ids, n_items their
         // count): its whole row at offset[its sorted position], the path of rows longer than
         // their fixed capacity.
@@ -402,13 +460,13 @@ namespace shamx {
                           const u32 *__restrict sort_index, const double4 *__restrict ps,
                           const u32 *__restrict owner, const u32 *__restrict leaf_cnt,
                           const u32 *__restrict leaf_offset, const u32 *__restrict leaf_ids,
-                          const u32 *__restrict item_leaf, const u32 *__restrict bstart,
+                          const u32 *__restrict item_leaf, const u32 *__restrict xstart,
                           const u32 *__restrict n_items, f64 htol, f64 Rker2,
                           u32 *__restrict cnt, u32 *__restrict offset, u32 *__restrict ids,
                           u32 cap, u32 leaf_cap, const u32 *__restrict inv = nullptr,
                           const f64 *__restrict bbox = nullptr) {
             __shared__ u32 rstart[GRP_WAVES][WAVE], rexcl[GRP_WAVES][WAVE];
-            // BCULL: the neighbour leaves of one pass (range, first batch, batches before it)
+            // BCULL: the neighbour leaves of one pass (range, leaf, batches before it)
             __shared__ u32 lr0[GRP_WAVES][BCULL ? WAVE : 1], lr1[GRP_WAVES][BCULL ? WAVE : 1];
             __shared__ u32 lbs[GRP_WAVES][BCULL ? WAVE : 1], lbx[GRP_WAVES][BCULL ? WAVE : 1];
             __shared__ double4 cpos[GRP_WAVES][WAVE]; // candidate x, y, z, cut radius^2
@@ -417,7 +475,7 @@ namespace shamx {
             __shared__ u32 mrow[GRP_WAVES][WAVE];     // member row start
             const int lane = __lane_id(), wid = threadIdx.x / WAVE;
             const u32 item = blockIdx.x * GRP_WAVES + wid;
-            if (item >= *n_items) return;
+            if (item >= (LIST ? 0u : L) + *n_items) return;
             u32 l, mb, m1;
             if constexpr (LIST) { // the batch is the listed particle alone (lane 0)
                 const u32 a0 = item_leaf[item];
@@ -428,7 +486,7 @@ namespace shamx {
                 l = item_leaf[item];
                 u32 m0;
                 node_children(nodes, I + l, m0, m1);
-                mb = m0 + (item - bstart[l]) * WAVE;
+                mb = m0 + item_batch(item, l, L, xstart) * WAVE;
             }
             const u64 lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
             // leaf_cap (fixed-capacity leaf rows): a row that overflowed holds only leaf_cap
@@ -579,7 +637,6 @@ namespace shamx {
                     // radius^2), every batch dropped whole by the test above
                     const bool okl = nd >= I && nd - I < L;
                     const u32 nbl  = okl ? (r1 - r0 + WAVE - 1) / WAVE : 0u;
-                    const u32 bs0  = nbl ? bstart[nd - I] : 0u;
                     u32 binc       = nbl;
                     for (int o = 1; o < WAVE; o <<= 1) {
                         u32 t = __shfl_up(binc, o, WAVE);
@@ -589,7 +646,7 @@ namespace shamx {
                     wave_lds_sync();
                     lr0[wid][lane] = r0;
                     lr1[wid][lane] = r1;
-                    lbs[wid][lane] = bs0;
+                    lbs[wid][lane] = okl ? nd - I : 0u;
                     lbx[wid][lane] = binc - nbl;
                     wave_lds_sync();
                     for (u32 t0 = 0; t0 < totb; t0 += WAVE) {
@@ -605,7 +662,7 @@ namespace shamx {
                             const u32 bi = tb - lbx[wid][j];
                             s0           = lr0[wid][j] + bi * WAVE;
                             s1           = min(s0 + WAVE, lr1[wid][j]);
-                            const f64 *bx = bbox + (u64) (lbs[wid][j] + bi) * 8;
+                            const f64 *bx = bbox + (u64) batch_item(bi, lbs[wid][j], xstart) * 8;
                             const f64 ex  = fmax(fmax(bx[0] - bhx, blx - bx[3]), 0.);
                             const f64 ey  = fmax(fmax(bx[1] - bhy, bly - bx[4]), 0.);
                             const f64 ez  = fmax(fmax(bx[2] - bhz, blz - bx[5]), 0.);
@@ -638,38 +695,22 @@ namespace shamx {
             }
         }
 
-        // member batches: nb[l] = batches of 64 sorted positions in leaf l (>= 1)
-        __global__ void k_leaf_batches(u32 L, u32 I, const f64 *__restrict nodes,
-                                       u32 *__restrict nbatch) {
-            u32 l = blockIdx.x * blockDim.x + threadIdx.x;
-            if (l >= L) return;
-            u32 m0, m1;
-            node_children(nodes, I + l, m0, m1);
-            nbatch[l] = max(1u, (m1 - m0 + WAVE - 1) / WAVE);
-        }
-        // item -> leaf for the batches of every leaf (bstart: exclusive scan of nbatch)
-        __global__ void k_item_leaf(u32 L, const u32 *__restrict nbatch,
-                                    const u32 *__restrict bstart, u32 *__restrict item_leaf) {
-            u32 l = blockIdx.x * blockDim.x + threadIdx.x;
-            if (l >= L) return;
-            const u32 b0 = bstart[l], nbl = nbatch[l];
-            for (u32 j = 0; j < nbl; j++) item_leaf[b0 + j] = l;
-        }
         // box of every member batch (all its sorted positions, images included: they are
         // candidates too) and the largest cut radius^2 among them, 8 doubles per batch:
         // lo x, y, z, hi x, y, z, (h htol)^2 R^2, unused.  One wave per batch.
         __global__ void __launch_bounds__(GRP_WAVES * WAVE)
-            k_batch_boxes(u32 I, const f64 *__restrict nodes, const u32 *__restrict item_leaf,
-                          const u32 *__restrict bstart, const u32 *__restrict n_items,
+            k_batch_boxes(u32 L, u32 I, const f64 *__restrict nodes,
+                          const u32 *__restrict item_leaf, const u32 *__restrict xstart,
+                          const u32 *__restrict n_extra,
                           const double4 *__restrict ps, f64 htol, f64 Rker2,
                           f64 *__restrict bbox) {
             const int lane = __lane_id();
             const u32 item = blockIdx.x * GRP_WAVES + threadIdx.x / WAVE;
-            if (item >= *n_items) return;
+            if (item >= L + *n_extra) return;
             const u32 l = item_leaf[item];
             u32 m0, m1;
             node_children(nodes, I + l, m0, m1);
-            const u32 sm = m0 + (item - bstart[l]) * WAVE + lane;
+            const u32 sm = m0 + item_batch(item, l, L, xstart) * WAVE + lane;
             constexpr f64 BIG = 1.7976931348623157e308;
             f64 lx = BIG, ly = BIG, lz = BIG, hx = -BIG, hy = -BIG, hz = -BIG, r2 = 0;
             if (sm < m1) {
@@ -760,20 +801,15 @@ namespace shamx {
                     nb.leaf_offset.data(), nb.leaf_ids.data(), cap, nb.lap.data(), nullptr, 0);
         }
 
-        // the stage-2 wave items (one per 64 sorted positions of every leaf): item -> leaf map,
-        // first item of every leaf, item count at counters[7]; returns the launch's block
-        // count, sized for the bound L + nm / 64 (waves past the count return at once)
+        // the stage-2 wave items (one per 64 sorted positions of every leaf), those beyond the
+        // leaves' first ones counted at counters[7]; returns the launch's block count, sized for
+        // the bound L + nm / 64 (waves past the count return at once)
         u32 batch_items(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t) {
             const u32 L = t.L, bound = L + div_up(t.n_obj, (u32) WAVE);
-            nb.nbatch.resize(L);
-            nb.bstart.resize(L);
+            nb.xstart.resize(L);
             nb.item_leaf.resize(bound);
-            k_leaf_batches<<<div_up(L, 256), 256, 0, s>>>(L, t.I, t.nodes.data(),
-                                                           nb.nbatch.data());
-            exclusive_scan_u32(s, nb.nbatch.data(), nb.bstart.data(), L, nb.counters.data() + 7,
-                               nb.scratch.data());
-            k_item_leaf<<<div_up(L, 256), 256, 0, s>>>(L, nb.nbatch.data(), nb.bstart.data(),
-                                                        nb.item_leaf.data());
+            k_items<<<div_up(L, 256), 256, 0, s>>>(L, t.I, t.nodes.data(), nb.item_leaf.data(),
+                                                    nb.xstart.data(), nb.counters.data() + 7);
             return div_up(bound, (u32) GRP_WAVES);
         }
 
@@ -782,14 +818,14 @@ namespace shamx {
             if (f & 2u)
                 throw std::runtime_error("neighbour cache: a particle is outside every leaf box");
         }
-        // owner leaves, mismatch list and (sorted layout) local flags, on complete leaf lists
+        // owner leaves and mismatch list
         void owners(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, u32 n_local,
-                    u32 gblocks, u32 leaf_cap, u32 *lflag) {
+                    u32 gblocks, u32 leaf_cap) {
             k_owner<<<div_up((u64) gblocks * GRP_WAVES * OWN_LANES, 256), 256, 0, s>>>(
-                n_local, t.I, t.nodes.data(), nb.item_leaf.data(), nb.bstart.data(),
+                n_local, t.L, t.I, t.nodes.data(), nb.item_leaf.data(), nb.xstart.data(),
                 nb.counters.data() + 7, t.sort_index.data(), nb.ps.data(), nb.lap.data(),
                 nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(), leaf_cap,
-                nb.owner.data(), lflag, nb.mism.data(), nb.counters.data() + 5);
+                nb.owner.data(), nb.mism.data(), nb.counters.data() + 5);
         }
 
         // boxes of the member batches for the batch-level cull of stage 2, on sets whose tree
@@ -802,7 +838,7 @@ namespace shamx {
             if (!t.fine_ties && !(e && std::atoi(e) == 1)) return nullptr;
             nb.bbox.resize((size_t) gblocks * GRP_WAVES * 8);
             k_batch_boxes<<<gblocks, GRP_WAVES * WAVE, 0, s>>>(
-                t.I, t.nodes.data(), nb.item_leaf.data(), nb.bstart.data(),
+                t.L, t.I, t.nodes.data(), nb.item_leaf.data(), nb.xstart.data(),
                 nb.counters.data() + 7, nb.ps.data(), htol, Rker2, nb.bbox.data());
             return nb.bbox.data();
         }
@@ -826,12 +862,11 @@ namespace shamx {
             u32 rows      = SORTED ? t.n_obj : n_local;
             u32 *mism_len      = nb.counters.data() + 5;
             const u32 *n_items = nb.counters.data() + 7;
-            if (SORTED) fill_u32(s, nb.cnt.data(), 0, rows); // ghost rows stay empty
             const f64 *bb = batch_boxes(s, nb, t, gblocks, htol, Rker2);
             launch_group<false, SORTED, false>(s, gblocks, bb,
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
                 nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
-                nb.item_leaf.data(), nb.bstart.data(), n_items, htol, Rker2, nb.cnt.data(),
+                nb.item_leaf.data(), nb.xstart.data(), n_items, htol, Rker2, nb.cnt.data(),
                 nullptr, nullptr, 0, leaf_cap);
             k_part_neigh<false, SORTED, false><<<div_up(n_local, 128), 128, 0, s>>>(
                 n_local, nb.mism.data(), mism_len, I, t.nodes.data(), t.sort_index.data(),
@@ -854,7 +889,7 @@ namespace shamx {
             launch_group<true, SORTED, false>(s, gblocks, bb,
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
                 nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
-                nb.item_leaf.data(), nb.bstart.data(), n_items, htol, Rker2, nullptr,
+                nb.item_leaf.data(), nb.xstart.data(), n_items, htol, Rker2, nullptr,
                 nb.offset.data(), nb.ids.data(), 0, leaf_cap);
             k_part_neigh<true, SORTED, false><<<div_up(n_local, 128), 128, 0, s>>>(
                 n_local, nb.mism.data(), mism_len, I, t.nodes.data(), t.sort_index.data(),
@@ -874,6 +909,21 @@ namespace shamx {
         // rows start on 64-byte boundaries
         u32 grow_cap(u32 need) { return (need + need / 8 + 16 + 15) & ~15u; }
     } // namespace
+
+    void local_rows(hipStream_t s, u32 nm, u32 n, const u32 *sort_index, u32 *lpos, u32 *perm,
+                    u32 *moved, DevArray<u32> &tile_cnt) {
+        if (nm == 0) return;
+        const u32 nt = compact_tiles(nm);
+        tile_cnt.resize(nt);
+        compact_dispatch(nm, [&](auto items) {
+            constexpr int IT = decltype(items)::value;
+            if (nt > 1 && nm != n)
+                k_local_count<IT><<<nt, CT_BLK, 0, s>>>(nm, n, sort_index, tile_cnt.data());
+            k_local_rows<IT><<<nt, CT_BLK, 0, s>>>(nm, n, sort_index, tile_cnt.data(), nt, lpos,
+                                                   perm, moved);
+        });
+        SHAMX_HIP(hipGetLastError());
+    }
 
     void neigh_build(hipStream_t s, NeighBuffers &nb, TreeBuffers &t, u32 n_local,
                      const f64 *x, const f64 *y, const f64 *z, const f64 *h, f64 htol,
@@ -901,7 +951,9 @@ namespace shamx {
         nb.inv.resize(nm);
         nb.mism.resize(std::max<u32>(n_local, 1));
         k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, t.sort_index.data(), x, y, z,
-                                                      h, nb.ps.data(), nb.inv.data(), err);
+                                                      h, nb.ps.data(), nb.inv.data(),
+                                                      sorted_layout ? nb.cnt.data() : nullptr,
+                                                      err);
         const u32 gblocks = batch_items(s, nb, t);
 
         // leaf lists in two passes (count, scan, fill); returns once their length is known
@@ -925,24 +977,18 @@ namespace shamx {
                 nb.n_pairs = 0;
                 return;
             }
-            owners(s, nb, t, n_local, gblocks, 0, nullptr);
+            owners(s, nb, t, n_local, gblocks, 0);
             stage2_packed<false>(s, nb, t, n_local, gblocks, x, y, z, h, htol, Rker2, hc);
             nb.row_stride = 0;
             SHAMX_HIP(hipGetLastError());
             return;
         }
 
-        // sorted layout: with the owners, the local rows in sorted order
-        nb.lflag.resize(nm);
-        nb.lscan.resize(nm);
+        // sorted layout: the local rows in sorted order
         nb.lpos.resize(std::max<u32>(n_local, 1));
-        auto own_leaves = [&](u32 leaf_cap) {
-            owners(s, nb, t, n_local, gblocks, leaf_cap, nb.lflag.data());
-            exclusive_scan_u32(s, nb.lflag.data(), nb.lscan.data(), nm, nb.counters.data() + 6,
-                               nb.scratch.data());
-            k_local_scatter<<<div_up(nm, 256), 256, 0, s>>>(nm, nb.lflag.data(),
-                                                            nb.lscan.data(), nb.lpos.data());
-        };
+        if (nb.want_perm) nb.perm.resize(std::max<u32>(n_local, 1));
+        local_rows(s, nm, n_local, t.sort_index.data(), nb.lpos.data(),
+                   nb.want_perm ? nb.perm.data() : nullptr, nb.counters.data() + 3, nb.tile_cnt);
 
         // Both stages in one pass each, rows of fixed capacity, chosen from the previous build
         // (about four times the mean length, at most the longest row plus headroom).  Rows
@@ -1007,7 +1053,7 @@ namespace shamx {
             if ((u64) L * cl > 0xffffffffull) {
                 // u32 entry indices cannot address fixed-capacity leaf lists: two passes each
                 packed_leaves();
-                own_leaves(0);
+                owners(s, nb, t, n_local, gblocks, 0);
                 stage2_packed<true>(s, nb, t, n_local, gblocks, x, y, z, h, htol, Rker2, hc);
                 nb.leaf_stride = 0;
                 nb.row_stride  = 0;
@@ -1029,7 +1075,7 @@ namespace shamx {
                 if (hc[12]) resolve_leaves(cl, hc[12], hc[13]);
             }
             const u32 leaf_cap = resolve_first ? 0u : cl; // lists past cl are truncated
-            own_leaves(leaf_cap);
+            owners(s, nb, t, n_local, gblocks, leaf_cap);
             if (packed) {
                 // particle rows packed (count, scan, fill)
                 const u32 n_leaf_pairs = hc[10];
@@ -1045,11 +1091,10 @@ namespace shamx {
             }
             // stage 2: fixed-capacity particle rows
             nb.ids.resize(std::max<u64>((u64) nm * cp, 1));
-            fill_u32(s, nb.cnt.data(), 0, nm); // ghost rows stay empty
             launch_group<true, true, true>(s, gblocks, batch_boxes(s, nb, t, gblocks, htol, Rker2),
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
                 nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
-                nb.item_leaf.data(), nb.bstart.data(), nb.counters.data() + 7, htol, Rker2,
+                nb.item_leaf.data(), nb.xstart.data(), nb.counters.data() + 7, htol, Rker2,
                 nb.cnt.data(), nb.offset.data(), nb.ids.data(), cp, leaf_cap);
             k_part_neigh<true, true, true><<<div_up(n_local, 128), 128, 0, s>>>(
                 n_local, nb.mism.data(), mism_len, I, t.nodes.data(), t.sort_index.data(),
@@ -1094,6 +1139,7 @@ namespace shamx {
             nb.cap_part = choose(mxp, nb.n_pairs, n_local, nm);
             break;
         }
+        nb.moved = hc[3];
         SHAMX_HIP(hipGetLastError());
     }
 

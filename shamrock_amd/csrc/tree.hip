@@ -16,6 +16,7 @@
 //   [0..2] aabb min, [3..5] aabb max, [6] rint = max h * htol,
 //   [7]    internal: (left total id, right total id); leaf: (first, end) in sorted order
 // so a traversal step reads exactly one record.
+#include "compact.hpp"
 #include "launch.hpp"
 #include "tree_layout.hpp"
 
@@ -415,7 +416,6 @@ namespace shamx {
         template<bool FIRST>
         __device__ inline bool reduc_keep(u32 j, u32 n, u32 K, const u32 *__restrict m,
                                           const u32 *__restrict F) {
-            if (j >= K) return false;
             if constexpr (FIRST) {
                 return j == 0 || m[j - 1] != m[j];
             } else {
@@ -430,106 +430,29 @@ namespace shamx {
             }
         }
 
-        // One iteration is two launches over tiles of the list: the kept entries
-        // of every tile, then their compaction, a block adding the counts of the tiles before
-        // its own (a few cached loads per thread) and testing its entries again, which is
-        // cheaper than a pass over stored flags.  (Flags, a two-launch scan and a compaction
-        // were four launches per iteration, each a few microseconds at any size below a few
-        // hundred thousand.)  A list of one tile needs the second launch only.
-        // Tiles of 1024 entries up to 2^23 (2.46 M positions: 67 us for the four iterations
-        // against 114 us with tiles of 4096, whose 600 blocks leave the chip half empty, and
-        // about 130 us for the sixteen launches before), 4096 beyond, where adding the counts of
-        // the earlier tiles, quadratic in their number, would weigh more.
-        constexpr int RED_BLK       = 256;
-        constexpr u32 RED_SMALL_MAX = 1u << 23;
-        template<bool FIRST, int RED_ITEMS>
-        __global__ void __launch_bounds__(RED_BLK)
+        // one iteration: the kept entries' compaction (compact.hpp)
+        template<bool FIRST, int ITEMS>
+        __global__ void __launch_bounds__(CT_BLK)
             k_reduc_count(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
                           const u32 *__restrict F, u32 *__restrict tile_cnt) {
-            __shared__ u32 part[RED_BLK / WAVE];
             const u32 K = FIRST ? n : min(*K_dev, n);
-            const u32 t0 = blockIdx.x * (RED_BLK * RED_ITEMS);
-            u32 c = 0;
-            if (t0 < K) {
-#pragma unroll 4
-                for (int k = 0; k < RED_ITEMS; k++)
-                    c += (u32) __popcll(__ballot(
-                        reduc_keep<FIRST>(t0 + k * RED_BLK + threadIdx.x, n, K, m, F)));
-            }
-            if (__lane_id() == 0) part[threadIdx.x / WAVE] = c;
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                for (int w = 1; w < RED_BLK / WAVE; w++) c += part[w];
-                tile_cnt[blockIdx.x] = c;
-            }
+            tile_count<ITEMS>(K, tile_cnt, [&](u32 j) { return reduc_keep<FIRST>(j, n, K, m, F); });
         }
-        template<bool FIRST, int RED_ITEMS>
-        __global__ void __launch_bounds__(RED_BLK)
+        template<bool FIRST, int ITEMS>
+        __global__ void __launch_bounds__(CT_BLK)
             k_reduc_compact(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
                             const u32 *__restrict F, const u32 *__restrict tile_cnt, u32 nt,
                             u32 *__restrict F_out, u32 *__restrict K_out,
                             u32 *__restrict K_copy) {
-            constexpr int NW = RED_BLK / WAVE;
-            __shared__ u32 part[NW];
-            __shared__ u32 cnt[RED_ITEMS * NW]; // kept entries per 64 of the tile, then before it
-            const u32 K    = FIRST ? n : min(*K_dev, n);
-            const u32 t0   = blockIdx.x * (RED_BLK * RED_ITEMS);
-            const u32 lane = (u32) __lane_id(), wid = threadIdx.x / WAVE;
-            // kept entries of the earlier tiles; block 0 counts all of them for the total
-            u32 before = 0;
-            if (nt > 1) {
-                const u32 lim = blockIdx.x == 0 ? nt : blockIdx.x;
-#pragma unroll 4
-                for (u32 i = threadIdx.x; i < lim; i += RED_BLK) before += tile_cnt[i];
-                before = wave_reduce(before, [](u32 p, u32 q) { return p + q; });
-                if (lane == 0) part[wid] = before;
-                __syncthreads();
-                before = 0;
-                for (int w = 0; w < NW; w++) before += part[w];
-                if (blockIdx.x == 0) {
-                    if (threadIdx.x == 0) {
-                        *K_out = before;
-                        if (K_copy) *K_copy = before;
-                    }
-                    before = 0;
-                }
-            }
-            if (t0 >= K) { // block-uniform
-                if (nt == 1 && threadIdx.x == 0) {
-                    *K_out = 0;
-                    if (K_copy) *K_copy = 0;
-                }
-                return;
-            }
-            u64 bal[RED_ITEMS];
-#pragma unroll
-            for (int k = 0; k < RED_ITEMS; k++) {
-                bal[k] = __ballot(reduc_keep<FIRST>(t0 + k * RED_BLK + threadIdx.x, n, K, m, F));
-                if (lane == 0) cnt[k * NW + wid] = (u32) __popcll(bal[k]);
-            }
-            __syncthreads();
-            static_assert(RED_ITEMS * NW <= WAVE, "one wave scans the counts");
-            if (wid == 0) {
-                const u32 v = lane < RED_ITEMS * NW ? cnt[lane] : 0u;
-                u32 inc     = v;
-                for (int o = 1; o < WAVE; o <<= 1) {
-                    u32 t = __shfl_up(inc, o, WAVE);
-                    if ((int) lane >= o) inc += t;
-                }
-                if (lane < RED_ITEMS * NW) cnt[lane] = inc - v;
-                if (nt == 1 && lane == WAVE - 1) {
-                    *K_out = inc;
-                    if (K_copy) *K_copy = inc;
-                }
-            }
-            __syncthreads();
-            const u64 lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-#pragma unroll
-            for (int k = 0; k < RED_ITEMS; k++) {
-                if (!((bal[k] >> lane) & 1ull)) continue;
-                const u32 j = t0 + k * RED_BLK + threadIdx.x;
-                F_out[before + cnt[k * NW + wid] + (u32) __popcll(bal[k] & lt)] = FIRST ? j : F[j];
-            }
+            const u32 K = FIRST ? n : min(*K_dev, n);
+            tile_compact<ITEMS>(
+                K, tile_cnt, nt, false,
+                [&](u32 j) { return reduc_keep<FIRST>(j, n, K, m, F); },
+                [&](u32 p, u32 j) { F_out[p] = FIRST ? j : F[j]; },
+                [&](u32 c) {
+                    *K_out = c;
+                    if (K_copy) *K_copy = c;
+                });
         }
 
         // update_morton_buf tail (reduction_alg.cpp:274-295) + remap (:564-585)
@@ -951,8 +874,7 @@ namespace shamx {
         // leaf reduction (reduction_alg.cpp:413-456) on the compacted list of split positions:
         // each iteration tests the positions still kept and compacts them, so it costs the
         // number of kept positions, not n (the lengths stay on the device: no host round trip)
-        const bool small = n <= RED_SMALL_MAX;
-        const u32 nt     = div_up(n, RED_BLK * (small ? 4 : 16));
+        const u32 nt = compact_tiles(n);
         t.red_cnt.resize(nt);
         t.red_pos.resize(std::max<u32>(n, 1));
         u32 *distinct = t.counters.data() + 1; // distinct codes (positions where codes change)
@@ -961,16 +883,14 @@ namespace shamx {
         auto iterate = [&](auto first, const u32 *K_in, const u32 *F_in, u32 *F_out, u32 *K_out,
                            u32 *K_copy) {
             constexpr bool FIRST = decltype(first)::value;
-            auto go              = [&](auto items) {
+            compact_dispatch(n, [&](auto items) {
                 constexpr int IT = decltype(items)::value;
                 if (nt > 1)
-                    k_reduc_count<FIRST, IT><<<nt, RED_BLK, 0, s>>>(
+                    k_reduc_count<FIRST, IT><<<nt, CT_BLK, 0, s>>>(
                         n, K_in, t.sorted.data(), F_in, t.red_cnt.data());
-                k_reduc_compact<FIRST, IT><<<nt, RED_BLK, 0, s>>>(
+                k_reduc_compact<FIRST, IT><<<nt, CT_BLK, 0, s>>>(
                     n, K_in, t.sorted.data(), F_in, t.red_cnt.data(), nt, F_out, K_out, K_copy);
-            };
-            if (small) go(std::integral_constant<int, 4>{});
-            else go(std::integral_constant<int, 16>{});
+            });
         };
         u32 *F_in = reduction_level > 0 ? t.red_pos.data() : t.reduc_map.data();
         iterate(std::true_type{}, nullptr, nullptr, F_in, distinct,
