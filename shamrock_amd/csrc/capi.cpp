@@ -152,7 +152,7 @@ struct shamx_solver {
     DevArray<u32> ghost_src, gwork;
     DevArray<u8> ghost_oid;
     DevArray<unsigned char> gscratch;
-    DevArray<u64> red, part;
+    DevArray<u64> red, part, part_corr, part_mid;
     // host copies of the step's reductions and counts (pinned, so the reads of one decision
     // queue on the stream and share one synchronisation)
     PinnedWords<u64, 8> hostw;
@@ -213,12 +213,6 @@ struct shamx_solver {
         P.resize(c);
         cs.resize(c);
         cap = c;
-    }
-
-    f64 read_key(int slot) {
-        hostw.read_async(stream, red.data() + slot, 1);
-        SHAMX_HIP(hipStreamSynchronize(stream));
-        return ordered_to_f64(hostw[0]);
     }
 
     // sorted-layout CSR: local particles in sorted order, records and rows by sorted position
@@ -413,18 +407,15 @@ struct shamx_solver {
             G = 0;
             return;
         }
-        // interaction range max h * htol_up_coarse * R, from the max key on the device
-        fill_u64(stream, red.data(), ORDERED_NEG_INF, 1);
-        max_key_f64(stream, N, h.data(), red.data());
         f64 box6[6] = {cfg.box_min[0], cfg.box_min[1], cfg.box_min[2],
                        cfg.box_max[0], cfg.box_max[1], cfg.box_max[2]};
         u32 g = periodic_ghosts(stream, N, x.data(), y.data(), z.data(), h.data(), box6,
-                                red.data(), cfg.htol_up_coarse, Rkern, ghost_src, ghost_oid,
+                                cfg.htol_up_coarse, Rkern, ghost_src, ghost_oid,
                                 gwork, gscratch, cap - N, hostc.data());
         if (g > cap - N) {
             grow(N + g);
             g = periodic_ghosts(stream, N, x.data(), y.data(), z.data(), h.data(), box6,
-                                red.data(), cfg.htol_up_coarse, Rkern, ghost_src, ghost_oid,
+                                cfg.htol_up_coarse, Rkern, ghost_src, ghost_oid,
                                 gwork, gscratch, cap - N, hostc.data());
         }
         G = g;
@@ -461,9 +452,7 @@ struct shamx_solver {
             timer.end(stream, PH_NEIGH, b);
             need(cfg.gpart_mass != 0, "invalid gpart_mass 0, this configuration can not converge");
             b = timer.begin(stream);
-            fill_f64(stream, eps.data(), 100., N);
-            SHAMX_HIP(hipMemcpyAsync(h_old.data(), h.data(), N * sizeof(f64),
-                                     hipMemcpyDeviceToDevice, stream));
+            h_loop_start(stream, N, h.data(), h_old.data(), eps.data(), hloop);
             f64 max_eps = std::numeric_limits<f64>::max(), min_eps = 0;
             if (cfg.h_iter_per_subcycles > 0) {
                 HLoopResult hl = h_iterate_loop(
@@ -485,9 +474,8 @@ struct shamx_solver {
         int b = timer.begin(stream);
         // final h of the images and in the sorted records, then Omega fused with the force
         // list filter (h and positions stay fixed for the rest of the step)
-        FieldPtrs fh{{h.data()}, 1};
-        gather_ghosts(stream, N, G, ghost_src.data(), fh);
-        ps_refresh_h(stream, N + G, tree.sort_index.data(), h.data(), nb.ps.data());
+        ps_refresh_h(stream, N + G, N, tree.sort_index.data(), ghost_src.data(), h.data(),
+                     nb.ps.data());
         nb.fcnt.resize(std::max<u32>(N + G, 1));
         nb.fids.resize(std::max<size_t>(nb.ids.size(), 1)); // same row offsets as ids
         compute_omega(stream, cfg.kernel, N, csr(), nb.ps.data(), x.data(), y.data(), z.data(),
@@ -589,13 +577,12 @@ struct shamx_solver {
                                          "a bug, either you are using a dt that is too large");
             b = timer.begin(stream);
             if (cfg.keep_storage_order) record_pass_inputs(corr_iter);
-            FieldPtrs fp{{h.data(), u.data(), vx.data(), vy.data(), vz.data(), omega.data()}, 6};
-            gather_ghosts(stream, N, G, ghost_src.data(), fp);
             // EOS of the merged set fused with the sorted force records (a corrector rerun
             // rewrites only the velocity, u, P and c_s of the records)
             frec.resize(force_record_bytes(cfg.mixed_precision) * (size_t) (N + G));
-            pack_force(stream, cfg.kernel, N + G, tree.sort_index.data(), x.data(), y.data(),
-                       z.data(), h.data(), vx.data(), vy.data(), vz.data(), u.data(),
+            pack_force(stream, cfg.kernel, N + G, N, tree.sort_index.data(), ghost_src.data(),
+                       x.data(), y.data(), z.data(), h.data(), vx.data(), vy.data(), vz.data(),
+                       u.data(),
                        omega.data(), P.data(), cs.data(), frec.data(), cfg.gpart_mass,
                        EosArgs{cfg.eos_kind, cfg.gamma, cfg.eos_cs, cfg.eos_cs0, cfg.eos_q,
                                cfg.eos_r0},
@@ -634,16 +621,16 @@ struct shamx_solver {
                           z.data(), vx.data(), vy.data(), vz.data(), h.data(), omega.data(),
                           u.data(), P.data(), cs.data(), ax.data(), ay.data(), az.data(),
                           du.data(), ax_old.data(), ay_old.data(), az_old.data(), du_old.data(),
-                          vsig.data(), dtc.data(), fa, red.data() + 3, red.data() + 7, part);
+                          vsig.data(), dtc.data(), fa, nullptr, nullptr, part);
             timer.end(stream, PH_FORCE, b);
             last.n_force_evals++;
             b = timer.begin(stream);
             corrector(stream, N, dtc_ / 2, vx.data(), vy.data(), vz.data(), ax.data(), ay.data(),
                       az.data(), ax_old.data(), ay_old.data(), az_old.data(), u.data(), du.data(),
-                      du_old.data(), cfg.gpart_mass, red.data() + 4, part);
+                      du_old.data(), cfg.gpart_mass, nullptr, part_corr);
+            reduce_pass(stream, N, part, &part_corr, part_mid, red.data() + 3, hostw.data());
             timer.end(stream, PH_CORR, b);
             const u64 *k = hostw.data();
-            hostw.read_async(stream, red.data() + 3, 5);
             SHAMX_HIP(hipStreamSynchronize(stream));
             f64 dt_min         = ordered_to_f64(k[0]);
             last.n_interacting = k[4];
@@ -730,11 +717,10 @@ struct shamx_solver {
         }
         prestep(1, false);
         b = timer.begin(stream);
-        FieldPtrs fp{{h.data(), u.data(), vx.data(), vy.data(), vz.data(), omega.data()}, 6};
-        gather_ghosts(stream, N, G, ghost_src.data(), fp);
         frec.resize(force_record_bytes(cfg.mixed_precision) * (size_t) (N + G));
-        pack_force(stream, cfg.kernel, N + G, tree.sort_index.data(), x.data(), y.data(),
-                   z.data(), h.data(), vx.data(), vy.data(), vz.data(), u.data(), omega.data(),
+        pack_force(stream, cfg.kernel, N + G, N, tree.sort_index.data(), ghost_src.data(),
+                   x.data(), y.data(), z.data(), h.data(), vx.data(), vy.data(), vz.data(),
+                   u.data(), omega.data(),
                    P.data(), cs.data(), frec.data(), cfg.gpart_mass,
                    EosArgs{cfg.eos_kind, cfg.gamma, cfg.eos_cs, cfg.eos_cs0, cfg.eos_q,
                            cfg.eos_r0},
@@ -753,10 +739,10 @@ struct shamx_solver {
                       z.data(), vx.data(), vy.data(), vz.data(), h.data(), omega.data(),
                       u.data(), P.data(), cs.data(), ax.data(), ay.data(), az.data(), du.data(),
                       ax_old.data(), ay_old.data(), az_old.data(), du_old.data(), vsig.data(),
-                      dtc.data(), fa, red.data() + 3, red.data() + 7, part);
+                      dtc.data(), fa, nullptr, nullptr, part);
+        reduce_pass(stream, N, part, nullptr, part_mid, red.data() + 3, hostw.data());
         timer.end(stream, PH_FORCE, b);
         const u64 *k = hostw.data();
-        hostw.read_async(stream, red.data() + 3, 5);
         SHAMX_HIP(hipStreamSynchronize(stream));
         auto t1 = std::chrono::steady_clock::now();
         f64 ph[PH_N] = {0};
@@ -968,11 +954,10 @@ struct shamx_solver {
         for (int k = 0; k < 4; k++)
             SHAMX_HIP(hipMemcpyAsync(dst[k], t.data() + k * (size_t) N, N * sizeof(f64),
                                      hipMemcpyDeviceToDevice, stream));
-        FieldPtrs fp{{h.data(), u.data(), vx.data(), vy.data(), vz.data(), omega.data()}, 6};
-        gather_ghosts(stream, N, G, ghost_src.data(), fp);
         adj_frec.resize(force_record_bytes(0) * (size_t) (N + G));
-        pack_force(stream, cfg.kernel, N + G, tree.sort_index.data(), x.data(), y.data(),
-                   z.data(), h.data(), vx.data(), vy.data(), vz.data(), u.data(), omega.data(),
+        pack_force(stream, cfg.kernel, N + G, N, tree.sort_index.data(), ghost_src.data(),
+                   x.data(), y.data(), z.data(), h.data(), vx.data(), vy.data(), vz.data(),
+                   u.data(), omega.data(),
                    P.data(), cs.data(), adj_frec.data(), cfg.gpart_mass,
                    EosArgs{cfg.eos_kind, cfg.gamma, cfg.eos_cs, cfg.eos_cs0, cfg.eos_q,
                            cfg.eos_r0},

@@ -28,15 +28,17 @@ namespace shamx {
     size_t bbox_scratch_bytes(u32 n);
     void bbox_nextafter(hipStream_t s, u32 n, const f64 *x, const f64 *y, const f64 *z,
                         f64 *bbox6, void *scratch);
-    // 30-bit Morton codes (MortonCodeSet.cpp:87-99)
+    // 30-bit Morton codes (MortonCodeSet.cpp:87-99), and a second copy of them in keys
     void morton_codes(hipStream_t s, u32 n, const f64 *x, const f64 *y, const f64 *z,
-                      const f64 *bbox6, u32 *codes);
+                      const f64 *bbox6, u32 *codes, u32 *keys = nullptr);
     // stable LSD radix sort of (key, index) pairs; sorts keys[0..n) and returns the permutation
     // in vals (vals are generated as iota in the first pass unless vals_given: then the
-    // values travel with their keys).  key_bits <= 32.
+    // values travel with their keys).  key_bits <= 32.  err: zeroed device word for the error
+    // flags (default: one in the scratch).
     size_t radix_sort_scratch_bytes(u32 n);
     void radix_sort_pairs(hipStream_t s, u32 n, u32 key_bits, u32 *keys, u32 *vals,
-                          u32 *keys_alt, u32 *vals_alt, void *scratch, bool vals_given = false);
+                          u32 *keys_alt, u32 *vals_alt, void *scratch, bool vals_given = false,
+                          u32 *err = nullptr);
     // the same sort on buffers held in a static device array (no allocation), n at most
     // NOALLOC_SORT_MAX_KEYS; calls that overlap on one GPU share that array and race
     constexpr u32 NOALLOC_SORT_MAX_KEYS = 1u << 22;
@@ -166,14 +168,16 @@ namespace shamx {
     // eps values and sweep count equal those of one sweep per host read.
     struct HLoopBuffers {
         DevArray<u64> st, part;
-        PinnedWords<u64, 16> host; // host copy of st
-        DevArray<u32> sel_a, sel_b, flag, off;
-        DevArray<unsigned char> scan;
+        PinnedWords<u64, 16> host; // the results in st, written by the sweeps' reductions
+        DevArray<u32> sel_a, sel_b, tile_cnt;
+        u32 last_iters = 0; // sweeps of the last loop (how many the next one queues at first)
     };
     struct HLoopResult {
         u32 iterations = 0, host_reads = 0, compactions = 0;
         f64 max_eps = 0, min_eps = 0;
     };
+    // before the loop: h_old = h, eps = 100 and the loop state
+    void h_loop_start(hipStream_t s, u32 n, const f64 *h, f64 *h_old, f64 *eps, HLoopBuffers &b);
     HLoopResult h_iterate_loop(hipStream_t s, int kernel, u32 n, Csr c, const double4 *ps,
                                const f64 *h_old, f64 *h_new, f64 *eps, f64 mass,
                                f64 h_evol_max, f64 h_evol_iter_max, f64 epsilon_h,
@@ -184,8 +188,9 @@ namespace shamx {
     void compute_omega(hipStream_t s, int kernel, u32 n, Csr c, const double4 *ps, const f64 *x,
                        const f64 *y, const f64 *z, const f64 *h, f64 *omega, f64 mass,
                        u32 *fcnt, u32 *fids, int mixed = 0);
-    // ps[s].w = h[sort_index[s]] for s < nm
-    void ps_refresh_h(hipStream_t s, u32 nm, const u32 *sort_index, const f64 *h, double4 *ps);
+    // h of the images from their sources, ps[s].w = h[sort_index[s]] for s < nm
+    void ps_refresh_h(hipStream_t s, u32 nm, u32 n, const u32 *sort_index, const u32 *ghost_src,
+                      f64 *h, double4 *ps);
     struct EosArgs {
         int kind;
         f64 gamma, cs, cs0, q, r0;
@@ -205,12 +210,13 @@ namespace shamx {
     // bytes of one force record (128 FP64, 64 mixed)
     size_t force_record_bytes(int mixed);
     // EOS on nm merged particles fused with the force-record build; record s describes
-    // particle perm[s] (identity when null).  P and cs are written per particle id.
+    // particle perm[s].  P and cs are written per particle id; the images (ids from n on) take h,
+    // v, u and omega of their source, in the records and in their own slots.
     // refresh: the records of the same particles were built by the last call and only
     // v and u changed since (corrector reruns): only those fields, P and c_s are rewritten
-    void pack_force(hipStream_t s, int kernel, u32 nm, const u32 *perm, const f64 *x,
-                    const f64 *y, const f64 *z, const f64 *h, const f64 *vx, const f64 *vy,
-                    const f64 *vz, const f64 *u, const f64 *omega, f64 *P, f64 *cs, void *rec,
+    void pack_force(hipStream_t s, int kernel, u32 nm, u32 n, const u32 *perm,
+                    const u32 *ghost_src, const f64 *x, const f64 *y, const f64 *z, f64 *h,
+                    f64 *vx, f64 *vy, f64 *vz, f64 *u, f64 *omega, f64 *P, f64 *cs, void *rec,
                     f64 mass, EosArgs e, int mixed, bool refresh = false);
     // UpdateDerivs constant AV (+ a_old save, vsig, per-particle CFL dt reduced into the
     // dt_min key, interacting-pair count).  Neighbours come from the records rec (row-indexed)
@@ -232,8 +238,12 @@ namespace shamx {
                    const f64 *ay, const f64 *az, const f64 *ax_old, const f64 *ay_old,
                    const f64 *az_old, f64 *u, const f64 *du, const f64 *du_old, f64 mass,
                    u64 *red, DevArray<u64> &part);
-    // max over n values as an ordered key (device)
-    void max_key_f64(hipStream_t s, u32 n, const f64 *v, u64 *key);
+    // the reductions of one pass: compute_force's (dt_min key, pair count; called with a null
+    // dt_min_key) and, with corr_part, corrector's (called with a null red), in one or two
+    // launches, to out[0..5) = dt_min key, max |dv|^2 key, sum |v|^2, energy, pair count, and
+    // to the host's pinned words.  mid: work space.
+    void reduce_pass(hipStream_t s, u32 n, const DevArray<u64> &force_part,
+                     const DevArray<u64> *corr_part, DevArray<u64> &mid, u64 *out, u64 *host);
     // varying AV (Cullen & Dehnen 2010): div v, curl v, d(div v)/dt over the force rows of the
     // n local particles (sorted layout), the alpha update from the saved sound speed into
     // alpha_new (local), and alpha of every merged particle into the FP64 records.
@@ -263,19 +273,12 @@ namespace shamx {
     // periodic image selection (BasicSPHGhosts.cpp:260-579): returns G (synchronises) and
     // fills src ids + appends positions/h of the images after the n local entries (count_host:
     // one pinned word for the count).
-    // The interaction range is (hmax * f1) * f2 with hmax the ordered key at *hmax_key (device).
+    // The interaction range is (hmax * f1) * f2 with hmax the maximum of h.
     u32 periodic_ghosts(hipStream_t s, u32 n, f64 *x, f64 *y, f64 *z, f64 *h, const f64 *box6,
-                        const u64 *hmax_key, f64 f1, f64 f2, DevArray<u32> &ghost_src,
+                        f64 f1, f64 f2, DevArray<u32> &ghost_src,
                         DevArray<u8> &ghost_off_id, DevArray<u32> &work,
                         DevArray<unsigned char> &scratch, u32 cap, u32 *count_host);
-    // ghost field refresh: dst[n + g] = src[ghost_src[g]] (+ offset for positions)
-    struct FieldPtrs {
-        f64 *p[8];
-        int n;
-    };
-    void gather_ghosts(hipStream_t s, u32 n, u32 G, const u32 *ghost_src, FieldPtrs fields);
-    // dst[j] = src[perm[j]] (gather) and dst[perm[j]] = src[j] (scatter), j < n
-    // the same gather of up to GATHER_MAX fields in one launch
+    // dst[j] = src[perm[j]] of up to GATHER_MAX fields in one launch, j < n
     constexpr int GATHER_MAX = 8;
     struct GatherPtrs {
         const f64 *src[GATHER_MAX];
@@ -283,6 +286,7 @@ namespace shamx {
         int n;
     };
     void perm_gather_fields(hipStream_t s, u32 n, const u32 *perm, const GatherPtrs &g);
+    // dst[j] = src[perm[j]] (gather) and dst[perm[j]] = src[j] (scatter), j < n
     void perm_gather_f64(hipStream_t s, u32 n, const u32 *perm, const f64 *src, f64 *dst);
     void perm_scatter_f64(hipStream_t s, u32 n, const u32 *perm, const f64 *src, f64 *dst);
     void perm_gather_u32(hipStream_t s, u32 n, const u32 *perm, const u32 *src, u32 *dst);

@@ -13,6 +13,7 @@
 // FP64 expressions keep the reference operation order (see common.hpp).  The mixed variant of
 // the force loop computes r_ab in FP64, then the pair terms in FP32, and accumulates with
 // Kahan compensation.
+#include "compact.hpp"
 #include "launch.hpp"
 
 #include <cstdlib>
@@ -337,67 +338,110 @@ namespace shamx {
 
         // ---- the Newton loop on the device (LoopSmoothingLengthIter.cpp:28-80)
         // Loop state, u64 words: 0 stop, 1 sweeps done, 2/3 max/min eps key of the particles
-        // dropped from the sweep list, 4/5/6 max/min eps key and active count of the last
-        // sweep (over its list), 8/9 max/min eps key over all particles, 10 active count.
+        // dropped from the sweep list, 4/5 max/min eps key over all particles, 6 active count of
+        // the last sweep (over its list).
         enum : int {
-            HL_STOP = 0, HL_ITERS, HL_FROZEN_MAX, HL_FROZEN_MIN, HL_SWEEP_MAX, HL_SWEEP_MIN,
-            HL_SWEEP_ACT, HL_PAD, HL_MAX, HL_MIN, HL_ACT, HL_WORDS = 16
+            HL_STOP = 0, HL_ITERS, HL_FROZEN_MAX, HL_FROZEN_MIN, HL_MAX, HL_MIN, HL_ACT,
+            HL_WORDS = 16
         };
-        __global__ void k_h_loop_init(u64 *__restrict st) {
-            if (threadIdx.x < HL_WORDS) {
+        // start of a subcycle's loop: h_old = h, eps = 100, the loop state
+        __global__ void __launch_bounds__(BLK)
+            k_h_loop_start(u32 n, const f64 *__restrict h, f64 *__restrict h_old,
+                           f64 *__restrict eps, u64 *__restrict st) {
+            const u32 i = blockIdx.x * BLK + threadIdx.x;
+            if (i < HL_WORDS) { // the first block
                 u64 v = 0;
-                if (threadIdx.x == HL_FROZEN_MAX) v = ORDERED_NEG_INF;
-                if (threadIdx.x == HL_FROZEN_MIN) v = ORDERED_POS_INF;
-                st[threadIdx.x] = v;
+                if (i == HL_FROZEN_MAX) v = ORDERED_NEG_INF;
+                if (i == HL_FROZEN_MIN) v = ORDERED_POS_INF;
+                st[i] = v;
             }
+            if (i >= n) return;
+            h_old[i] = h[i];
+            eps[i]   = 100.;
         }
-        // after each sweep: count it and stop the loop once max eps < epsilon_h, the
-        // reference's break condition
-        __global__ void k_h_loop_ctl(u64 *__restrict st, f64 epsilon_h) {
-            if (threadIdx.x != 0 || st[HL_STOP]) return;
-            st[HL_ITERS] += 1;
-            u64 mx = umax64(st[HL_FROZEN_MAX], st[HL_SWEEP_MAX]);
-            u64 mn = umin64(st[HL_FROZEN_MIN], st[HL_SWEEP_MIN]);
-            st[HL_MAX] = mx;
-            st[HL_MIN] = mn;
-            st[HL_ACT] = st[HL_SWEEP_ACT];
-            if (ordered_to_f64(mx) < epsilon_h) st[HL_STOP] = 1;
+        // after each sweep: reduce its nb block partials (slots `stride` apart), count it and
+        // stop the loop once max eps < epsilon_h, the reference's break condition.  One block;
+        // the state also goes to the host's pinned words, which are read after the batch.
+        constexpr int HLE_BLK = 1024;
+        __global__ void __launch_bounds__(HLE_BLK)
+            k_h_loop_end(u32 nb, u64 stride, const u64 *__restrict part, u64 *__restrict st,
+                         f64 epsilon_h, u64 *__restrict host) {
+            __shared__ u64 lds[3][HLE_BLK / WAVE];
+            if (st[HL_STOP]) return; // a sweep queued after the loop has stopped
+            u64 mx = ORDERED_NEG_INF, mn = ORDERED_POS_INF, act = 0;
+            for (u32 i = threadIdx.x; i < nb; i += HLE_BLK) {
+                mx = umax64(mx, part[i]);
+                mn = umin64(mn, part[stride + i]);
+                act += part[2 * stride + i];
+            }
+            mx  = wave_reduce(mx, umax64);
+            mn  = wave_reduce(mn, umin64);
+            act = wave_reduce(act, [](u64 p, u64 q) { return p + q; });
+            if (__lane_id() == 0) {
+                lds[0][threadIdx.x / WAVE] = mx;
+                lds[1][threadIdx.x / WAVE] = mn;
+                lds[2][threadIdx.x / WAVE] = act;
+            }
+            __syncthreads();
+            if (threadIdx.x != 0) return;
+            for (int w = 1; w < HLE_BLK / WAVE; w++) {
+                mx = umax64(mx, lds[0][w]);
+                mn = umin64(mn, lds[1][w]);
+                act += lds[2][w];
+            }
+            mx = umax64(st[HL_FROZEN_MAX], mx);
+            mn = umin64(st[HL_FROZEN_MIN], mn);
+            const u64 it   = st[HL_ITERS] + 1;
+            const u64 stop = ordered_to_f64(mx) < epsilon_h ? 1u : 0u;
+            st[HL_ITERS]   = it;
+            st[HL_MAX]     = mx;
+            st[HL_MIN]     = mn;
+            st[HL_ACT]     = act;
+            st[HL_STOP]    = stop;
+            host[HL_ITERS] = it;
+            host[HL_MAX]   = mx;
+            host[HL_MIN]   = mn;
+            host[HL_ACT]   = act;
+            host[HL_STOP]  = stop;
         }
         // rows of the sweep list whose particle still iterates (eps > 1e-6: the sweep's own
-        // test); the eps of the rows dropped is final for the subcycle and goes into the
-        // frozen max / min
-        // (grid-stride over few blocks: one pair of same-address atomics per block)
-        __global__ void __launch_bounds__(BLK)
-            k_h_active_flags(u32 n, const u32 *__restrict sel, const u32 *__restrict outi,
-                             const f64 *__restrict eps, u32 *__restrict flag,
-                             u64 *__restrict st) {
+        // test), compacted as in compact.hpp (tiles of 4096: one pair of same-address atomics per
+        // block); the eps of the rows dropped is final for the subcycle and goes into the frozen
+        // max / min
+        constexpr int HA_ITEMS = 16;
+        __global__ void __launch_bounds__(CT_BLK)
+            k_h_active_count(u32 n, const u32 *__restrict sel, const u32 *__restrict outi,
+                             const f64 *__restrict eps, u32 *__restrict tile_cnt) {
+            tile_count<HA_ITEMS>(n, tile_cnt, [&](u32 j) {
+                const u32 row = sel ? sel[j] : j;
+                return eps[outi ? outi[row] : row] > 1e-6;
+            });
+        }
+        __global__ void __launch_bounds__(CT_BLK)
+            k_h_active_rows(u32 n, const u32 *__restrict sel, const u32 *__restrict outi,
+                            const f64 *__restrict eps, const u32 *__restrict tile_cnt, u32 nt,
+                            u32 *__restrict out, u64 *__restrict st) {
+            static_assert(CT_BLK == BLK, "block_reduce is written for BLK threads");
             __shared__ u64 lds[2][BLK / WAVE];
             u64 kmax = ORDERED_NEG_INF, kmin = ORDERED_POS_INF;
-            for (u32 j = blockIdx.x * BLK + threadIdx.x; j < n; j += gridDim.x * BLK) {
-                u32 row = sel ? sel[j] : j;
-                f64 e   = eps[outi ? outi[row] : row];
-                bool keep = e > 1e-6;
-                flag[j]   = keep ? 1u : 0u;
-                if (!keep) {
-                    u64 k = f64_to_ordered(e);
-                    kmax  = umax64(kmax, k);
-                    kmin  = umin64(kmin, k);
-                }
-            }
+            tile_compact<HA_ITEMS>(
+                n, tile_cnt, nt, false,
+                [&](u32 j) {
+                    const u32 row = sel ? sel[j] : j;
+                    const f64 e   = eps[outi ? outi[row] : row];
+                    if (e > 1e-6) return true;
+                    const u64 k = f64_to_ordered(e);
+                    kmax        = umax64(kmax, k);
+                    kmin        = umin64(kmin, k);
+                    return false;
+                },
+                [&](u32 p, u32 j) { out[p] = sel ? sel[j] : j; }, [](u32) {});
             kmax = block_reduce(kmax, umax64, lds[0]);
             kmin = block_reduce(kmin, umin64, lds[1]);
             if (threadIdx.x == 0) {
-                if (kmax != ORDERED_NEG_INF) atomicMax((unsigned long long *) &st[HL_FROZEN_MAX],
-                                                       (unsigned long long) kmax);
-                if (kmin != ORDERED_POS_INF) atomicMin((unsigned long long *) &st[HL_FROZEN_MIN],
-                                                       (unsigned long long) kmin);
+                if (kmax != ORDERED_NEG_INF) atomic_max_key(&st[HL_FROZEN_MAX], kmax);
+                if (kmin != ORDERED_POS_INF) atomic_min_key(&st[HL_FROZEN_MIN], kmin);
             }
-        }
-        __global__ void k_h_compact_rows(u32 n, const u32 *__restrict sel,
-                                         const u32 *__restrict flag, const u32 *__restrict off,
-                                         u32 *__restrict out) {
-            u32 j = blockIdx.x * blockDim.x + threadIdx.x;
-            if (j < n && flag[j]) out[off[j]] = sel ? sel[j] : j;
         }
 
         // ------------------------------------------------------------- omega
@@ -533,11 +577,16 @@ namespace shamx {
             }
         }
 
-        // ps[s].w = h[sort_index[s]] (final h into the sorted position records)
-        __global__ void k_ps_refresh_h(u32 nm, const u32 *__restrict sort_index,
-                                       const f64 *__restrict h, double4 *__restrict ps) {
+        // final h of the images (their source's) and in the sorted position records
+        __global__ void k_ps_refresh_h(u32 nm, u32 n, const u32 *__restrict sort_index,
+                                       const u32 *__restrict ghost_src, f64 *__restrict h,
+                                       double4 *__restrict ps) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
-            if (s < nm) ps[s].w = h[sort_index[s]];
+            if (s >= nm) return;
+            const u32 b  = sort_index[s];
+            const f64 hb = h[b < n ? b : ghost_src[b - n]];
+            if (b >= n) h[b] = hb;
+            ps[s].w = hb;
         }
 
         // ------------------------------------------------------------- eos
@@ -660,20 +709,24 @@ namespace shamx {
             }
         };
 
-        // EOS on the merged set fused with the record build: record s takes particle perm[s].
+        // EOS on the merged set fused with the record build: record s takes particle perm[s], an
+        // image the fields of its source (written to its own slots too).
         // REFRESH: rewrite only the fields that a corrector pass changes
         template<class K, bool MIXED, bool REFRESH = false>
-        __global__ void k_pack_force(u32 nm, const u32 *__restrict perm, const f64 *__restrict x,
+        __global__ void k_pack_force(u32 nm, u32 n, const u32 *__restrict perm,
+                                     const u32 *__restrict ghost_src, const f64 *__restrict x,
                                      const f64 *__restrict y, const f64 *__restrict z,
-                                     const f64 *__restrict h, const f64 *__restrict vx,
-                                     const f64 *__restrict vy, const f64 *__restrict vz,
-                                     const f64 *__restrict u, const f64 *__restrict omega,
-                                     f64 *__restrict P, f64 *__restrict cs, void *__restrict rec,
-                                     f64 mass, EosArgs e) {
+                                     f64 *__restrict h, f64 *__restrict vx, f64 *__restrict vy,
+                                     f64 *__restrict vz, f64 *__restrict u,
+                                     f64 *__restrict omega, f64 *__restrict P,
+                                     f64 *__restrict cs, void *__restrict rec, f64 mass,
+                                     EosArgs e) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
             if (s >= nm) return;
-            u32 b  = perm ? perm[s] : s;
-            f64 hb = h[b], ub = u[b], xb = 0, yb = 0, zb = 0;
+            const u32 b = perm[s], a = b < n ? b : ghost_src[b - n];
+            const f64 hb = h[a], ub = u[a], vxb = vx[a], vyb = vy[a], vzb = vz[a], ob = omega[a];
+            if (b >= n) h[b] = hb, u[b] = ub, vx[b] = vxb, vy[b] = vyb, vz[b] = vzb, omega[b] = ob;
+            f64 xb = 0, yb = 0, zb = 0;
             if (!REFRESH || e.kind == 2) xb = x[b], yb = y[b], zb = z[b];
             f64 rho = rho_h(mass, hb, (f64) K::hfactd);
             f64 p, c;
@@ -684,17 +737,17 @@ namespace shamx {
                 // corrector reruns: positions, h and omega are those of the full build, only
                 // v and u (and with u the EOS) changed; the other fields are already in place
                 FRec32 *r = (FRec32 *) rec + s;
-                r->vx = (f32) vx[b], r->vy = (f32) vy[b], r->vz = (f32) vz[b];
+                r->vx = (f32) vxb, r->vy = (f32) vyb, r->vz = (f32) vzb;
                 r->u = (f32) ub, r->P = (f32) p, r->cs = (f32) c;
             } else if constexpr (REFRESH) {
                 FRec *r = (FRec *) rec + s;
-                r->vx = vx[b], r->vy = vy[b], r->vz = vz[b], r->u = ub, r->P = p, r->cs = c;
+                r->vx = vxb, r->vy = vyb, r->vz = vzb, r->u = ub, r->P = p, r->cs = c;
             } else if constexpr (MIXED)
                 ((FRec32 *) rec)[s] =
-                    make_frec32<K>(xb, yb, zb, hb, vx[b], vy[b], vz[b], ub, p, c, omega[b], mass);
+                    make_frec32<K>(xb, yb, zb, hb, vxb, vyb, vzb, ub, p, c, ob, mass);
             else
                 ((FRec *) rec)[s] =
-                    make_frec<K>(xb, yb, zb, hb, vx[b], vy[b], vz[b], ub, p, c, omega[b], mass);
+                    make_frec<K>(xb, yb, zb, hb, vxb, vyb, vzb, ub, p, c, ob, mass);
         }
 
         struct ForceOut {
@@ -1316,6 +1369,37 @@ namespace shamx {
             }
         }
 
+        // Several reductions in one launch, a block per chunk (x) and reduction (y): red y of
+        // chunk x to mid[y * gridDim.x + x], or, as the last stage (mid null, one chunk), to
+        // out[slot] and the host's pinned word host[slot].  The chunks are k_finalize's, so a
+        // sum takes its terms in the same fixed order.
+        constexpr int RED_JOBS = 5;
+        struct RedJobs {
+            const u64 *p[RED_JOBS];
+            u32 n[RED_JOBS];
+            int op[RED_JOBS], slot[RED_JOBS];
+        };
+        __global__ void __launch_bounds__(FIN_BLK)
+            k_finalize_jobs(RedJobs jobs, u32 chunk, u64 *__restrict mid, u64 *__restrict out,
+                            u64 *__restrict host) {
+            __shared__ u64 lds[FIN_BLK / WAVE];
+            __shared__ u64 res;
+            const int y  = blockIdx.y;
+            u64 *o       = mid ? mid + (u64) y * gridDim.x : &res;
+            const u64 *p = jobs.p[y];
+            const u32 n  = jobs.n[y];
+            switch (jobs.op[y]) {
+            case RED_MAX_KEY: fin_block<RED_MAX_KEY>(p, n, chunk, o, lds); break;
+            case RED_MIN_KEY: fin_block<RED_MIN_KEY>(p, n, chunk, o, lds); break;
+            case RED_SUM_U64: fin_block<RED_SUM_U64>(p, n, chunk, o, lds); break;
+            default: fin_block<RED_SUM_F64>(p, n, chunk, o, lds); break;
+            }
+            if (!mid && threadIdx.x == 0) {
+                out[jobs.slot[y]]  = res;
+                host[jobs.slot[y]] = res;
+            }
+        }
+
         // ------------------------------------------------------------- integrators
         __device__ inline f64 pos_mod(f64 v, f64 bmin, f64 delt) {
             f64 r = v - bmin;
@@ -1427,15 +1511,16 @@ namespace shamx {
             if (threadIdx.x == 0) part[blockIdx.x] = key;
         }
 
-        // (one same-address atomic per block: a few hundred blocks)
+        // per-block maxima as ordered keys
+        constexpr u32 MAX_KEY_BLOCKS = 256;
         __global__ void __launch_bounds__(BLK) k_max_key(u32 n, const f64 *__restrict v,
-                                                         u64 *__restrict key) {
+                                                         u64 *__restrict part) {
             __shared__ u64 lds[BLK / WAVE];
             u64 k = ORDERED_NEG_INF;
             for (u32 i = blockIdx.x * BLK + threadIdx.x; i < n; i += gridDim.x * BLK)
                 k = umax64(k, f64_to_ordered(v[i]));
             k = block_reduce(k, umax64, lds);
-            if (threadIdx.x == 0) atomic_max_key(key, k);
+            if (threadIdx.x == 0) part[blockIdx.x] = k;
         }
 
         // ------------------------------------------------------------- periodic images
@@ -1446,17 +1531,23 @@ namespace shamx {
 
         // the 26 image offsets and cut volumes of the periodic box (BasicSPHGhosts.cpp:260-509),
         // offset o in (x, y, z) nesting order without (0, 0, 0), from the interaction range
-        // (hmax * f1) * f2 with hmax read from the device (no host round trip)
+        // (hmax * f1) * f2 with hmax the maximum of the nk block maxima (no host round trip); one
+        // block of MAX_KEY_BLOCKS threads
         struct Box6 {
             f64 v[6];
         };
-        __global__ void k_cut_boxes(Box6 box, const u64 *__restrict hmax_key, f64 f1, f64 f2,
-                                    CutBoxes *__restrict cb) {
+        __global__ void __launch_bounds__(BLK)
+            k_cut_boxes(Box6 box, const u64 *__restrict keys, u32 nk, f64 f1, f64 f2,
+                        CutBoxes *__restrict cb) {
+            static_assert(MAX_KEY_BLOCKS == BLK, "a key per thread");
+            __shared__ u64 lds[BLK / WAVE];
+            const u64 hmax_key =
+                block_reduce(threadIdx.x < nk ? keys[threadIdx.x] : ORDERED_NEG_INF, umax64, lds);
             const int o = threadIdx.x;
             if (o >= 26) return;
             const int q     = o < 13 ? o : o + 1;
             const int io[3] = {q / 9 - 1, (q / 3) % 3 - 1, q % 3 - 1};
-            const f64 int_range = (ordered_to_f64(*hmax_key) * f1) * f2;
+            const f64 int_range = (ordered_to_f64(hmax_key) * f1) * f2;
             bool nonempty = true;
             for (int k = 0; k < 3; k++) {
                 f64 bmin = box.v[k], bmax = box.v[3 + k];
@@ -1533,13 +1624,6 @@ namespace shamx {
                 z[dst]         = pz + cb.off[o][2];
                 h[dst]         = ph;
             }
-        }
-
-        __global__ void k_gather(u32 n, u32 G, const u32 *__restrict src, FieldPtrs fp) {
-            u32 g = blockIdx.x * blockDim.x + threadIdx.x;
-            if (g >= G) return;
-            u32 s = src[g];
-            for (int f = 0; f < fp.n; f++) fp.p[f][n + g] = fp.p[f][s];
         }
     } // namespace
 
@@ -1634,59 +1718,79 @@ namespace shamx {
                                u32 max_iter, int mixed, HLoopBuffers &b) {
         HLoopResult res{};
         if (n == 0 || max_iter == 0) return res;
-        b.st.resize(HL_WORDS);
-        k_h_loop_init<<<1, 64, 0, s>>>(b.st.data());
         const u32 *sel = c.sel;
         u32 n_act      = n;
-        u32 done = 0, batch = 1;
+        // as many sweeps before the first host read as the last loop took, when they were few
+        // (the two or three of a settled step), else one; then one, two, four, eight
+        u32 done = 0, grow = 1;
+        u32 batch = b.last_iters <= 4 ? std::max<u32>(b.last_iters, 1) : 1;
         static_assert(HL_WORDS <= decltype(b.host)::size(), "h-loop words exceed the host copy");
         u64 *host = b.host.data();
+        for (int k = 0; k < HL_WORDS; k++) host[k] = 0;
         while (done < max_iter) {
             u32 k = std::min(batch, max_iter - done);
+            // no row is left: the remaining sweeps change nothing but their count (they still
+            // count, as the reference's sweeps over converged particles do); one reduction of no
+            // partials leaves max / min to the frozen extrema
+            if (n_act == 0) k = 1;
             for (u32 i = 0; i < k; i++) {
                 Rows r{sel, c.outi, c.cnt, c.offset, c.ids};
                 h_sweep(s, kernel, n_act, r, ps, nullptr, nullptr, nullptr, h_old, h_new, eps,
                         mass, h_evol_max, h_evol_iter_max, mixed, b.part, b.st.data());
-                u32 nb = div_up((u64) n_act * pair_lanes(), BLK);
-                finalize(s, nb, b.part.data(),
-                         RedSpec{3, {RED_MAX_KEY, RED_MIN_KEY, RED_SUM_U64},
-                                 {HL_SWEEP_MAX, HL_SWEEP_MIN, HL_SWEEP_ACT}},
-                         b.st.data(), b.part.data() + 3 * (size_t) nb);
-                k_h_loop_ctl<<<1, 64, 0, s>>>(b.st.data(), epsilon_h);
+                u32 nb           = div_up((u64) n_act * pair_lanes(), BLK);
+                const u64 *parts = b.part.data();
+                u64 stride       = nb;
+                if (nb > FIN_CHUNK) {
+                    u64 *mid      = b.part.data() + 3 * (size_t) nb;
+                    const u32 nb2 = div_up(nb, FIN_CHUNK);
+                    k_finalize<<<nb2, FIN_BLK, 0, s>>>(
+                        nb, FIN_CHUNK, parts, nb,
+                        RedSpec{3, {RED_MAX_KEY, RED_MIN_KEY, RED_SUM_U64}, {0, 1, 2}}, mid, nb2);
+                    parts = mid, nb = nb2, stride = nb2;
+                }
+                k_h_loop_end<<<1, HLE_BLK, 0, s>>>(nb, stride, parts, b.st.data(), epsilon_h, host);
             }
             SHAMX_HIP(hipGetLastError());
-            b.host.read_async(s, b.st.data(), HL_WORDS);
             SHAMX_HIP(hipStreamSynchronize(s));
             done += k;
             res.host_reads++;
             if (host[HL_STOP]) break;
+            if (n_act == 0) {
+                host[HL_ITERS] = max_iter;
+                break;
+            }
             // the particles still iterating are few: sweep only their rows from now on
             u32 keep = (u32) host[HL_ACT];
             if (done < max_iter && (u64) keep * 4 < n_act) {
-                b.flag.resize(std::max<u32>(n_act, 1));
-                b.off.resize(std::max<u32>(n_act, 1));
                 DevArray<u32> &dst = (sel == b.sel_a.data()) ? b.sel_b : b.sel_a;
                 dst.resize(std::max<u32>(keep, 1));
-                b.scan.resize(std::max(b.scan.size(), scan_scratch_bytes(n_act)));
-                k_h_active_flags<<<std::min<u32>(256, div_up(n_act, BLK)), BLK, 0, s>>>(
-                    n_act, sel, c.outi, eps, b.flag.data(), b.st.data());
-                exclusive_scan_u32(s, b.flag.data(), b.off.data(), n_act, nullptr, b.scan.data());
-                k_h_compact_rows<<<div_up(n_act, 256), 256, 0, s>>>(n_act, sel, b.flag.data(),
-                                                                   b.off.data(), dst.data());
+                const u32 nt = div_up(n_act, CT_BLK * HA_ITEMS);
+                b.tile_cnt.resize(nt);
+                if (nt > 1)
+                    k_h_active_count<<<nt, CT_BLK, 0, s>>>(n_act, sel, c.outi, eps,
+                                                           b.tile_cnt.data());
+                k_h_active_rows<<<nt, CT_BLK, 0, s>>>(n_act, sel, c.outi, eps, b.tile_cnt.data(),
+                                                      nt, dst.data(), b.st.data());
                 SHAMX_HIP(hipGetLastError());
                 sel   = dst.data();
                 n_act = keep;
-                // (with no row left the remaining sweeps launch nothing; their reduction over
-                // no partials leaves max / min to the frozen extrema, and they still count,
-                // as the reference's sweeps over converged particles do)
                 res.compactions++;
             }
-            batch = std::min<u32>(2 * batch, 8);
+            batch = grow;
+            grow  = std::min<u32>(2 * grow, 8);
         }
         res.iterations = (u32) host[HL_ITERS];
+        b.last_iters   = res.iterations;
         res.max_eps    = ordered_to_f64(host[HL_MAX]);
         res.min_eps    = ordered_to_f64(host[HL_MIN]);
         return res;
+    }
+
+    void h_loop_start(hipStream_t s, u32 n, const f64 *h, f64 *h_old, f64 *eps, HLoopBuffers &b) {
+        b.st.resize(HL_WORDS);
+        k_h_loop_start<<<std::max<u32>(div_up(n, BLK), 1), BLK, 0, s>>>(n, h, h_old, eps,
+                                                                       b.st.data());
+        SHAMX_HIP(hipGetLastError());
     }
 
     void compute_omega(hipStream_t s, int kernel, u32 n, Csr c, const double4 *ps, const f64 *x,
@@ -1718,9 +1822,10 @@ namespace shamx {
         SHAMX_HIP(hipGetLastError());
     }
 
-    void ps_refresh_h(hipStream_t s, u32 nm, const u32 *sort_index, const f64 *h, double4 *ps) {
+    void ps_refresh_h(hipStream_t s, u32 nm, u32 n, const u32 *sort_index, const u32 *ghost_src,
+                      f64 *h, double4 *ps) {
         if (nm == 0) return;
-        k_ps_refresh_h<<<div_up(nm, 256), 256, 0, s>>>(nm, sort_index, h, ps);
+        k_ps_refresh_h<<<div_up(nm, 256), 256, 0, s>>>(nm, n, sort_index, ghost_src, h, ps);
         SHAMX_HIP(hipGetLastError());
     }
 
@@ -1736,25 +1841,25 @@ namespace shamx {
 
     size_t force_record_bytes(int mixed) { return mixed ? sizeof(FRec32) : sizeof(FRec); }
 
-    void pack_force(hipStream_t s, int kernel, u32 nm, const u32 *perm, const f64 *x,
-                    const f64 *y, const f64 *z, const f64 *h, const f64 *vx, const f64 *vy,
-                    const f64 *vz, const f64 *u, const f64 *omega, f64 *P, f64 *cs, void *rec,
+    void pack_force(hipStream_t s, int kernel, u32 nm, u32 n, const u32 *perm,
+                    const u32 *ghost_src, const f64 *x, const f64 *y, const f64 *z, f64 *h,
+                    f64 *vx, f64 *vy, f64 *vz, f64 *u, f64 *omega, f64 *P, f64 *cs, void *rec,
                     f64 mass, EosArgs e, int mixed, bool refresh) {
         if (nm == 0) return;
         dispatch_kernel(kernel, [&](auto K) {
             using KT = decltype(K);
             if (refresh && mixed)
                 k_pack_force<KT, true, true><<<div_up(nm, 256), 256, 0, s>>>(
-                    nm, perm, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
+                    nm, n, perm, ghost_src, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
             else if (refresh)
                 k_pack_force<KT, false, true><<<div_up(nm, 256), 256, 0, s>>>(
-                    nm, perm, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
+                    nm, n, perm, ghost_src, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
             else if (mixed)
                 k_pack_force<KT, true><<<div_up(nm, 256), 256, 0, s>>>(
-                    nm, perm, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
+                    nm, n, perm, ghost_src, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
             else
                 k_pack_force<KT, false><<<div_up(nm, 256), 256, 0, s>>>(
-                    nm, perm, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
+                    nm, n, perm, ghost_src, x, y, z, h, vx, vy, vz, u, omega, P, cs, rec, mass, e);
         });
         SHAMX_HIP(hipGetLastError());
     }
@@ -1796,6 +1901,7 @@ namespace shamx {
             });
         });
         SHAMX_HIP(hipGetLastError());
+        if (!dt_min_key) return; // reduced with the corrector's (reduce_pass)
         // dt_min and the pair count may live in different buffers: reduce each slot separately;
         // both calls use the room after the two slots in turn (stream order)
         u64 *mid = part.data() + 2 * (size_t) nb;
@@ -1823,9 +1929,36 @@ namespace shamx {
         k_corrector<<<nb, BLK, 0, s>>>(n, hdt, vx, vy, vz, ax, ay, az, ax_old, ay_old, az_old, u,
                                        du, du_old, mass, part.data());
         SHAMX_HIP(hipGetLastError());
+        if (!red) return; // reduced with the force loop's (reduce_pass)
         finalize(s, nb, part.data(),
                  RedSpec{3, {RED_MAX_KEY, RED_SUM_F64, RED_SUM_F64}, {0, 1, 2}}, red,
                  part.data() + 3 * (size_t) nb);
+    }
+
+    void reduce_pass(hipStream_t s, u32 n, const DevArray<u64> &force_part,
+                     const DevArray<u64> *corr_part, DevArray<u64> &mid, u64 *out, u64 *host) {
+        if (n == 0) return;
+        const u32 nf = div_up((u64) n * pair_lanes(), BLK), nc = div_up(n, BLK);
+        const u64 *f = force_part.data(), *c = corr_part ? corr_part->data() : nullptr;
+        RedJobs jobs{{f, f + nf, c, c + nc, c + 2 * (size_t) nc},
+                     {nf, nf, nc, nc, nc},
+                     {RED_MIN_KEY, RED_SUM_U64, RED_MAX_KEY, RED_SUM_F64, RED_SUM_F64},
+                     {0, 4, 1, 2, 3}};
+        const u32 nj = c ? 5 : 2, nmax = c ? std::max(nf, nc) : nf;
+        if (nmax > FIN_CHUNK) {
+            const u32 nch = div_up(nmax, FIN_CHUNK);
+            mid.resize((size_t) RED_JOBS * nch);
+            k_finalize_jobs<<<dim3(nch, nj), FIN_BLK, 0, s>>>(jobs, FIN_CHUNK, mid.data(), nullptr,
+                                                            nullptr);
+            for (u32 y = 0; y < nj; y++) {
+                jobs.p[y] = mid.data() + (size_t) y * nch;
+                jobs.n[y] = nch;
+            }
+            k_finalize_jobs<<<dim3(1, nj), FIN_BLK, 0, s>>>(jobs, nch, nullptr, out, host);
+        } else {
+            k_finalize_jobs<<<dim3(1, nj), FIN_BLK, 0, s>>>(jobs, nmax, nullptr, out, host);
+        }
+        SHAMX_HIP(hipGetLastError());
     }
 
     void wrap_positions(hipStream_t s, u32 n, f64 *x, f64 *y, f64 *z, const f64 *box6) {
@@ -1882,35 +2015,28 @@ namespace shamx {
                  part.data() + nb);
     }
 
-    void max_key_f64(hipStream_t s, u32 n, const f64 *v, u64 *key) {
-        if (n == 0) return;
-        u32 nb = std::min<u32>(div_up(n, BLK), 256);
-        k_max_key<<<nb, BLK, 0, s>>>(n, v, key);
-        SHAMX_HIP(hipGetLastError());
-    }
-
     // cut volumes are computed on the host exactly as find_interfaces does for one patch:
     // offset o = (xo, yo, zo) in lexicographic order without (0,0,0); interf volume =
     // sender box ∩ (receiver box expanded by int_range - offset); membership half-open.
     u32 periodic_ghosts(hipStream_t s, u32 n, f64 *x, f64 *y, f64 *z, f64 *h, const f64 *box6,
-                        const u64 *hmax_key, f64 f1, f64 f2, DevArray<u32> &ghost_src,
+                        f64 f1, f64 f2, DevArray<u32> &ghost_src,
                         DevArray<u8> &ghost_off_id, DevArray<u32> &work,
                         DevArray<unsigned char> &scratch, u32 cap, u32 *count_host) {
         Box6 box{{box6[0], box6[1], box6[2], box6[3], box6[4], box6[5]}};
         u32 nb = div_up(std::max<u32>(n, 1), BLK);
-        // work: [cutboxes (as u32 words)] [26*nb counts] [26*nb bases] [total]
-        size_t cb_words = (sizeof(CutBoxes) + 3) / 4;
-        work.resize(cb_words + 2 * (size_t) 26 * nb + 4);
-        u32 *w           = work.data();
-        CutBoxes *cbd    = (CutBoxes *) w;
-        u32 *counts      = w + cb_words;
+        // work: [block maxima of h] [cutboxes] (as u32 words) [26*nb counts] [26*nb bases]
+        const size_t key_words = 2 * MAX_KEY_BLOCKS, cb_words = (sizeof(CutBoxes) + 3) / 4;
+        work.resize(key_words + cb_words + 2 * (size_t) 26 * nb);
+        u64 *keys        = (u64 *) work.data();
+        CutBoxes *cbd    = (CutBoxes *) (work.data() + key_words);
+        u32 *counts      = work.data() + key_words + cb_words;
         u32 *bases       = counts + (size_t) 26 * nb;
-        u32 *total       = bases + (size_t) 26 * nb;
         scratch.resize(std::max<size_t>(scratch.size(), scan_scratch_bytes(26 * nb)));
-        k_cut_boxes<<<1, 32, 0, s>>>(box, hmax_key, f1, f2, cbd);
+        const u32 nk = std::min<u32>(nb, MAX_KEY_BLOCKS);
+        k_max_key<<<nk, BLK, 0, s>>>(n, h, keys);
+        k_cut_boxes<<<1, BLK, 0, s>>>(box, keys, nk, f1, f2, cbd);
         k_ghost_count<<<nb, BLK, 0, s>>>(n, x, y, z, cbd, counts, nb);
-        exclusive_scan_u32(s, counts, bases, 26 * nb, total, scratch.data());
-        SHAMX_HIP(hipMemcpyAsync(count_host, total, sizeof(u32), hipMemcpyDeviceToHost, s));
+        exclusive_scan_u32(s, counts, bases, 26 * nb, count_host, scratch.data());
         SHAMX_HIP(hipStreamSynchronize(s));
         const u32 G = *count_host;
         if (G > cap) return G; // caller grows the merged arrays and calls again
@@ -1968,12 +2094,6 @@ namespace shamx {
     void perm_gather_u32(hipStream_t s, u32 n, const u32 *perm, const u32 *src, u32 *dst) {
         if (n == 0) return;
         k_perm_gather<u32><<<div_up(n, 256), 256, 0, s>>>(n, perm, src, dst);
-        SHAMX_HIP(hipGetLastError());
-    }
-
-    void gather_ghosts(hipStream_t s, u32 n, u32 G, const u32 *ghost_src, FieldPtrs fields) {
-        if (G == 0) return;
-        k_gather<<<div_up(G, 256), 256, 0, s>>>(n, G, ghost_src, fields);
         SHAMX_HIP(hipGetLastError());
     }
 

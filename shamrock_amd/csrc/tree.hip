@@ -105,13 +105,15 @@ namespace shamx {
         }
         __global__ void k_morton(u32 n, const f64 *__restrict x, const f64 *__restrict y,
                                  const f64 *__restrict z, const f64 *__restrict bb,
-                                 u32 *__restrict codes) {
+                                 u32 *__restrict codes, u32 *__restrict keys) {
             u32 i = blockIdx.x * blockDim.x + threadIdx.x;
             if (i >= n) return;
             u32 gx = to_grid(x[i], bb[0], bb[3]);
             u32 gy = to_grid(y[i], bb[1], bb[4]);
             u32 gz = to_grid(z[i], bb[2], bb[5]);
-            codes[i] = expand_bits_10(gx) * 4 + expand_bits_10(gy) * 2 + expand_bits_10(gz);
+            const u32 c = expand_bits_10(gx) * 4 + expand_bits_10(gy) * 2 + expand_bits_10(gz);
+            codes[i]    = c;
+            if (keys) keys[i] = c; // the copy that the sort works on
         }
 
         // position inside its Morton cell, as a 30-bit Morton code of a 1024^3 sub-grid of the
@@ -443,7 +445,7 @@ namespace shamx {
             k_reduc_compact(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
                             const u32 *__restrict F, const u32 *__restrict tile_cnt, u32 nt,
                             u32 *__restrict F_out, u32 *__restrict K_out,
-                            u32 *__restrict K_copy) {
+                            u32 *__restrict counters, u32 *__restrict host) {
             const u32 K = FIRST ? n : min(*K_dev, n);
             tile_compact<ITEMS>(
                 K, tile_cnt, nt, false,
@@ -451,7 +453,14 @@ namespace shamx {
                 [&](u32 p, u32 j) { F_out[p] = FIRST ? j : F[j]; },
                 [&](u32 c) {
                     *K_out = c;
-                    if (K_copy) *K_copy = c;
+                    if (!host) return;
+                    // the last iteration: leaf count, distinct codes and the sorts' error words
+                    // to the host's pinned words
+                    counters[0] = c;
+                    host[0]     = c;
+                    host[1]     = counters[1];
+                    host[2]     = counters[2];
+                    host[3]     = counters[3];
                 });
         }
 
@@ -711,9 +720,9 @@ namespace shamx {
     }
 
     void morton_codes(hipStream_t s, u32 n, const f64 *x, const f64 *y, const f64 *z,
-                      const f64 *bbox6, u32 *codes) {
+                      const f64 *bbox6, u32 *codes, u32 *keys) {
         if (n == 0) return;
-        k_morton<<<div_up(n, 256), 256, 0, s>>>(n, x, y, z, bbox6, codes);
+        k_morton<<<div_up(n, 256), 256, 0, s>>>(n, x, y, z, bbox6, codes, keys);
         SHAMX_HIP(hipGetLastError());
     }
 
@@ -730,7 +739,8 @@ namespace shamx {
     size_t radix_sort_scratch_bytes(u32 n) { return rs_scratch_bytes(n); }
 
     void radix_sort_pairs(hipStream_t s, u32 n, u32 key_bits, u32 *keys, u32 *vals,
-                          u32 *keys_alt, u32 *vals_alt, void *scratch, bool vals_given) {
+                          u32 *keys_alt, u32 *vals_alt, void *scratch, bool vals_given,
+                          u32 *err) {
         if (n == 0) return;
         if (key_bits == 0 || key_bits > 32) throw std::invalid_argument("radix sort key_bits");
         if (n >= (1u << 30)) throw std::invalid_argument("radix sort: n must be below 2^30");
@@ -742,7 +752,7 @@ namespace shamx {
         u32 nt       = div_up(n, RS_BLOCK * (small ? RS_ITEMS_SMALL : RS_ITEMS));
         u32 *hist    = (u32 *) scratch;
         u32 *ctr     = hist + 4 * RS_BINS;
-        u32 *err     = ctr + 4;
+        if (!err) err = ctr + 4;
         u32 *status  = ctr + 8;
         // digit counts and tile counters start at zero; the status words of pass 0 are zeroed
         // by the histogram kernel, those of pass p + 1 by pass p's tiles
@@ -837,12 +847,8 @@ namespace shamx {
         fill_u32(s, t.counters.data(), 0, 8);
         t.big_listed = false;
         bbox_nextafter(s, n, x, y, z, t.bbox6.data(), t.scratch.data());
-        morton_codes(s, n, x, y, z, t.bbox6.data(), t.codes.data());
-        SHAMX_HIP(hipMemcpyAsync(t.sorted.data(), t.codes.data(), n * sizeof(u32),
-                                 hipMemcpyDeviceToDevice, s));
+        morton_codes(s, n, x, y, z, t.bbox6.data(), t.codes.data(), t.sorted.data());
     }
-
-    u32 *radix_sort_error_word(void *scratch) { return (u32 *) scratch + 4 * RS_BINS + 4; }
 
     void tree_stage_sort(hipStream_t s, TreeBuffers &t, const f64 *x, const f64 *y,
                          const f64 *z) {
@@ -853,20 +859,15 @@ namespace shamx {
             k_fine_key<<<div_up(n, 256), 256, 0, s>>>(n, x, y, z, t.bbox6.data(),
                                                        t.split_a.data());
             radix_sort_pairs(s, n, 30, t.split_a.data(), t.split_b.data(), t.keys_alt.data(),
-                             t.vals_alt.data(), t.scratch.data(), false);
-            SHAMX_HIP(hipMemcpyAsync(t.counters.data() + 3,
-                                     radix_sort_error_word(t.scratch.data()), sizeof(u32),
-                                     hipMemcpyDeviceToDevice, s));
+                             t.vals_alt.data(), t.scratch.data(), false, t.counters.data() + 3);
             k_gather_u32<<<div_up(n, 256), 256, 0, s>>>(n, t.codes.data(), t.split_b.data(),
                                                          t.sorted.data());
             SHAMX_HIP(hipMemcpyAsync(t.sort_index.data(), t.split_b.data(), n * sizeof(u32),
                                      hipMemcpyDeviceToDevice, s));
         }
         radix_sort_pairs(s, n, 30, t.sorted.data(), t.sort_index.data(), t.keys_alt.data(),
-                         t.vals_alt.data(), t.scratch.data(), t.fine_ties);
-        // keep the sort's error word before the scratch is reused by the scans
-        SHAMX_HIP(hipMemcpyAsync(t.counters.data() + 2, radix_sort_error_word(t.scratch.data()),
-                                 sizeof(u32), hipMemcpyDeviceToDevice, s));
+                         t.vals_alt.data(), t.scratch.data(), t.fine_ties,
+                         t.counters.data() + 2);
     }
 
     void tree_stage_karras(hipStream_t s, TreeBuffers &t, u32 reduction_level) {
@@ -880,8 +881,9 @@ namespace shamx {
         u32 *distinct = t.counters.data() + 1; // distinct codes (positions where codes change)
         u32 *L_dev    = t.counters.data() + 0;
         u32 *K_tmp[2] = {t.counters.data() + 8, t.counters.data() + 9};
+        u32 *hc = t.host.data();
         auto iterate = [&](auto first, const u32 *K_in, const u32 *F_in, u32 *F_out, u32 *K_out,
-                           u32 *K_copy) {
+                           bool last) {
             constexpr bool FIRST = decltype(first)::value;
             compact_dispatch(n, [&](auto items) {
                 constexpr int IT = decltype(items)::value;
@@ -889,24 +891,23 @@ namespace shamx {
                     k_reduc_count<FIRST, IT><<<nt, CT_BLK, 0, s>>>(
                         n, K_in, t.sorted.data(), F_in, t.red_cnt.data());
                 k_reduc_compact<FIRST, IT><<<nt, CT_BLK, 0, s>>>(
-                    n, K_in, t.sorted.data(), F_in, t.red_cnt.data(), nt, F_out, K_out, K_copy);
+                    n, K_in, t.sorted.data(), F_in, t.red_cnt.data(), nt, F_out, K_out,
+                    t.counters.data(), last ? hc : nullptr);
             });
         };
         u32 *F_in = reduction_level > 0 ? t.red_pos.data() : t.reduc_map.data();
-        iterate(std::true_type{}, nullptr, nullptr, F_in, distinct,
-                reduction_level == 0 ? L_dev : nullptr);
+        iterate(std::true_type{}, nullptr, nullptr, F_in, distinct, reduction_level == 0);
         const u32 *K_in = distinct;
         for (u32 it = 1; it <= reduction_level; it++) {
             const bool last = it == reduction_level;
             u32 *F_out = last ? t.reduc_map.data()
                               : (F_in == t.red_pos.data() ? t.split_b.data() : t.red_pos.data());
             u32 *K_out = last ? L_dev : K_tmp[it % 2];
-            iterate(std::false_type{}, K_in, F_in, F_out, K_out, nullptr);
+            iterate(std::false_type{}, K_in, F_in, F_out, K_out, last);
             F_in = F_out;
             K_in = K_out;
         }
-        u32 *hc = t.host.data();
-        t.host.read_async(s, t.counters.data(), 4);
+        SHAMX_HIP(hipGetLastError());
         SHAMX_HIP(hipStreamSynchronize(s));
         if (hc[2] | hc[3]) throw std::runtime_error("radix sort: look-back or scatter inconsistency");
         // the next builds order runs of equal codes spatially when codes repeat on average
