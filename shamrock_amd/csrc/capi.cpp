@@ -617,7 +617,7 @@ struct shamx_solver {
                 fa.ext_y = aye.data();
                 fa.ext_z = aze.data();
             }
-            compute_force(stream, cfg.kernel, N, csr_force(), frec.data(), x.data(), y.data(),
+            compute_force(stream, cfg.kernel, N, N + G, csr_force(), frec.data(), x.data(), y.data(),
                           z.data(), vx.data(), vy.data(), vz.data(), h.data(), omega.data(),
                           u.data(), P.data(), cs.data(), ax.data(), ay.data(), az.data(),
                           du.data(), ax_old.data(), ay_old.data(), az_old.data(), du_old.data(),
@@ -735,7 +735,7 @@ struct shamx_solver {
             fa.ext_y = aye.data();
             fa.ext_z = aze.data();
         }
-        compute_force(stream, cfg.kernel, N, csr_force(), frec.data(), x.data(), y.data(),
+        compute_force(stream, cfg.kernel, N, N + G, csr_force(), frec.data(), x.data(), y.data(),
                       z.data(), vx.data(), vy.data(), vz.data(), h.data(), omega.data(),
                       u.data(), P.data(), cs.data(), ax.data(), ay.data(), az.data(), du.data(),
                       ax_old.data(), ay_old.data(), az_old.data(), du_old.data(), vsig.data(),
@@ -1336,7 +1336,7 @@ int shamx_force(void *stream, int kernel, uint32_t n, const uint32_t *cnt, const
     return guarded([&] {
         hipStream_t s = (hipStream_t) stream;
         u64 *sl       = slots();
-        compute_force(s, kernel, n, Csr{cnt, offset, ids}, nullptr, x, y, z, vx, vy, vz, h,
+        compute_force(s, kernel, n, 0, Csr{cnt, offset, ids}, nullptr, x, y, z, vx, vy, vz, h,
                       omega, u, P, cs, ax, ay, az, du, ax_old, ay_old, az_old, du_old, vsig,
                       dt_cfl,
                       ForceArgs{gpart_mass, alpha_u, alpha_AV, beta_AV, C_cour, C_force, mixed},

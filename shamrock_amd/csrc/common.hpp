@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -74,26 +75,31 @@ namespace shamx {
             return T(0);
         }
     };
+    // v clamped at +0 from below (0 for a NaN).  The truncated powers of M6 and M8 take their
+    // bases through it instead of choosing among partial sums: a term past its knot is a zero,
+    // which leaves the sum of the others as it is (a sum of zeros is +0 in the order used), so
+    // the values are those of the sum that stops there, without its compares and selects.
+    template<class T>
+    __host__ __device__ inline T clamp0(T v) {
+        return fmax(v, T(0));
+    }
     struct M6 {
         static constexpr f64 Rkern = 3, hfactd = 1.0, norm_3d = 1 / (120 * PI);
         static constexpr int id = 1;
         template<class T>
         __host__ __device__ static T f(T q) {
-            T t1 = T(3) - q, t2 = T(2) - q, t3 = T(1) - q;
+            T t1 = clamp0(T(3) - q), t2 = clamp0(T(2) - q), t3 = clamp0(T(1) - q);
             T t1_2 = t1 * t1, t2_2 = t2 * t2, t3_2 = t3 * t3;
             t1 = t1 * t1_2 * t1_2;
             t2 = t2 * t2_2 * t2_2;
             t3 = t3 * t3_2 * t3_2;
             t2 *= T(-6);
             t3 *= T(15);
-            if (q < T(1)) return t1 + t2 + t3;
-            if (q < T(2)) return t1 + t2;
-            if (q < T(3)) return t1;
-            return T(0);
+            return t1 + t2 + t3;
         }
         template<class T>
         __host__ __device__ static T df(T q) {
-            T t1 = T(3) - q, t2 = T(2) - q, t3 = T(1) - q;
+            T t1 = clamp0(T(3) - q), t2 = clamp0(T(2) - q), t3 = clamp0(T(1) - q);
             T t1_2 = t1 * t1, t2_2 = t2 * t2, t3_2 = t3 * t3;
             t1 = t1_2 * t1_2;
             t2 = t2_2 * t2_2;
@@ -101,10 +107,7 @@ namespace shamx {
             t1 *= T(-5);
             t2 *= T(30);
             t3 *= T(-75);
-            if (q < T(1)) return t1 + t2 + t3;
-            if (q < T(2)) return t1 + t2;
-            if (q < T(3)) return t1;
-            return T(0);
+            return t1 + t2 + t3;
         }
     };
     template<class T>
@@ -122,28 +125,22 @@ namespace shamx {
         static constexpr int id = 2;
         template<class T>
         __host__ __device__ static T f(T q) {
-            T t1 = pow7(T(4) - q), t2 = pow7(T(3) - q), t3 = pow7(T(2) - q), t4 = pow7(T(1) - q);
+            T t1 = pow7(clamp0(T(4) - q)), t2 = pow7(clamp0(T(3) - q)), t3 = pow7(clamp0(T(2) - q)),
+              t4 = pow7(clamp0(T(1) - q));
             t2 *= T(-8.);
             t3 *= T(28.);
             t4 *= T(-56.);
-            if (q < T(1)) return t1 + t2 + t3 + t4;
-            if (q < T(2)) return t1 + t2 + t3;
-            if (q < T(3)) return t1 + t2;
-            if (q < T(4)) return t1;
-            return T(0);
+            return t1 + t2 + t3 + t4;
         }
         template<class T>
         __host__ __device__ static T df(T q) {
-            T t1 = pow6(T(4) - q), t2 = pow6(T(3) - q), t3 = pow6(T(2) - q), t4 = pow6(T(1) - q);
+            T t1 = pow6(clamp0(T(4) - q)), t2 = pow6(clamp0(T(3) - q)), t3 = pow6(clamp0(T(2) - q)),
+              t4 = pow6(clamp0(T(1) - q));
             t1 *= T(-7.);
             t2 *= T(56.);
             t3 *= T(-196.);
             t4 *= T(392.);
-            if (q < T(1)) return t1 + t2 + t3 + t4;
-            if (q < T(2)) return t1 + t2 + t3;
-            if (q < T(3)) return t1 + t2;
-            if (q < T(4)) return t1;
-            return T(0);
+            return t1 + t2 + t3 + t4;
         }
     };
     struct C2 {

@@ -220,8 +220,9 @@ namespace shamx {
                     f64 mass, EosArgs e, int mixed, bool refresh = false);
     // UpdateDerivs constant AV (+ a_old save, vsig, per-particle CFL dt reduced into the
     // dt_min key, interacting-pair count).  Neighbours come from the records rec (row-indexed)
-    // when given, else from the SoA arrays.
-    void compute_force(hipStream_t s, int kernel, u32 n, Csr c, const void *rec, const f64 *x,
+    // when given (nm of them, with the rows that interact: the Omega pass's force rows), else from
+    // the SoA arrays.
+    void compute_force(hipStream_t s, int kernel, u32 n, u32 nm, Csr c, const void *rec, const f64 *x,
                        const f64 *y, const f64 *z, const f64 *vx, const f64 *vy, const f64 *vz,
                        const f64 *h, const f64 *omega, const f64 *u, const f64 *P, const f64 *cs,
                        f64 *ax, f64 *ay, f64 *az, f64 *du, f64 *ax_old, f64 *ay_old,

@@ -957,6 +957,238 @@ namespace shamx {
             }
         }
 
+        // ------------------------------------------------------------- force (FP64, solver rows)
+        // sqrt(v) correctly rounded for zero, infinity and 2^-767 < v (below, without the scaling
+        // of a general sqrt, its last bits; squared distances and P / rho ratios of a run are far
+        // above), and a value within an ulp or two of 1 / sqrt(v): the hardware estimate, one
+        // Newton step for both, two residual corrections of the root
+        __device__ inline f64 sqrt_pair(f64 v, f64 &recip) {
+            const f64 r0 = __builtin_amdgcn_rsq(v);
+            f64 s = v * r0, g = 0.5 * r0;
+            const f64 e = __builtin_fma(-g, s, 0.5);
+            g           = __builtin_fma(g, e, g);
+            s           = __builtin_fma(s, e, s);
+            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
+            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
+            recip       = g + g;
+            return __builtin_amdgcn_class(v, 0x260) ? v : s; // +-0 and +inf: themselves
+        }
+
+        // piece of 16 bytes q (0..35) of a group's four records: byte offset inside its record,
+        // and the lane of the group whose record it is
+        constexpr int FR_PIECES = sizeof(FRec) / 16; // 9
+        constexpr int fr_lane(int q) { return q / FR_PIECES; }
+        // offsets v of the records of the group's lanes, taken by the lane that loads piece
+        // 4 I + lane of the group
+        template<int I>
+        __device__ inline u32 fr_pick(u32 v) {
+            constexpr int c = fr_lane(4 * I) | (fr_lane(4 * I + 1) << 2) |
+                              (fr_lane(4 * I + 2) << 4) | (fr_lane(4 * I + 3) << 6);
+            return (u32) __builtin_amdgcn_mov_dpp((int) v, c, 0xf, 0xf, true);
+        }
+
+        // UpdateDerivs.cpp:88-288 over the solver's force rows, which hold exactly the pairs that
+        // interact, fused with the CFL signal speed (Solver.cpp:2749-2783).  Same sums in the
+        // same order as k_force with four lanes per particle; what differs is how records come.
+        //
+        // A lane that gathers its own 144-byte record makes every load instruction of the wave
+        // touch 64 lines; the address units were busy 69 % of k_force's time and its waves
+        // waited on them.  Here the four lanes of a particle fetch their four records together,
+        // 64 contiguous bytes per instruction (nine instructions for the 36 pieces of 16 bytes),
+        // straight into LDS, where lane l's pieces lie on different banks from its neighbours':
+        // 16 lines and a bit per instruction.  A lane then reads its record from LDS at once, the
+        // next records are requested into the same room, and the pair is evaluated meanwhile.
+        // The loop runs for the longest row of the wave, so that all lanes can load.
+        // Beside that it issues fewer instructions per pair: the rows need no criterion and no pair
+        // count, one estimate serves |r_ab| and its reciprocal, the largest |v.r| stands for the
+        // largest signal speed.
+        // Sedov 128^3 (M6, 230 M pairs): 2.71 -> 2.35 ms per evaluation; line accesses 52 -> 23 per
+        // load instruction, address units busy 69 -> 56 % of the time, waves waiting 51 -> 40 %,
+        // 236 -> 215 VALU instructions per wave and pass at 62 % of the issue peak, which with
+        // three waves per SIMD (LDS: 12 KB per wave) is what bounds it now.  Plummer sphere of
+        // 4.2 M (M4) 3.30 -> 3.0 ms, HCP lattice of 1.09 M 0.79 -> 0.67 ms.  Two lanes per
+        // particle, which need no fold room and let four waves fit: Plummer 3.8 ms; one lane:
+        // 6.8 ms.
+        // WIDE: records past 4 GiB (29.8 M of them), 64-bit offsets.
+        template<class K, bool WIDE>
+        __global__ void __launch_bounds__(BLK)
+            k_force_rows(u32 n, Rows r, const FRec *__restrict rec, ForceOut o, ForceArgs fa,
+                         u64 *__restrict part) {
+            using KK        = Kern<K, f64>;
+            constexpr int G = 4, NP = FR_PIECES;
+            __shared__ u64 lds[2][BLK / WAVE];
+            // lane c of a group folds component c (x, y, z, du) over its four lanes' terms in
+            // lane order, see k_force
+            __shared__ f64 fold[BLK][6];
+            __shared__ __attribute__((aligned(16))) double2 room[BLK / WAVE][NP][WAVE];
+            const u32 j    = (xcd_block(blockIdx.x, gridDim.x) * BLK + threadIdx.x) / G;
+            const u32 lane = (u32) __lane_id(), lg = lane % G;
+            const u32 wid  = (u32) __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
+            const bool act = j < n;
+            const u32 row  = act ? r.sel[j] : 0u;
+            const u32 k0 = act ? r.off[row] : 0u, len = act ? r.cnt[row] : 0u;
+            const u32 longest = wave_reduce(len, [](u32 p, u32 q) { return p > q ? p : q; });
+            const u32 steps   = ((u32) __builtin_amdgcn_readfirstlane((int) longest) + G - 1) / G;
+            // entry of pass t of this lane; past the row's end its last entry, of an empty row
+            // the particle itself
+            auto id_at = [&](u32 t) -> u32 {
+                const u32 k = t * G + lg;
+                return len ? r.ids[k0 + min(k, len - 1)] : row;
+            };
+            u32 src[NP], dst[NP]; // piece to load: offset in its record; own piece: offset in room
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                const u32 m = lg + (u32) i; // own piece i is piece 9 lg + i = 8 lg + m
+                src[i]      = ((4 * (u32) i + lg) % NP) * 16;
+                dst[i]      = (2 * lg + m / 4) * (WAVE * 16) + (lane / G) * 64 + (m % 4) * 16;
+            }
+            const char *recs = (const char *) rec;
+            char *mine       = (char *) &room[wid][0][0];
+            auto request     = [&](u32 id) {
+                const u32 v = WIDE ? id : id * (u32) sizeof(FRec);
+                auto one = [&](auto ic) {
+                    constexpr int I = decltype(ic)::value;
+                    const u32 w     = fr_pick<I>(v);
+                    const char *at  = WIDE ? recs + (u64) w * sizeof(FRec) + src[I]
+                                           : recs + (w + src[I]);
+                    __builtin_amdgcn_global_load_lds(
+                        (const __attribute__((address_space(1))) void *) at,
+                        (__attribute__((address_space(3))) void *) (mine + I * WAVE * 16), 16, 0, 0);
+                };
+                one(std::integral_constant<int, 0>{});
+                one(std::integral_constant<int, 1>{});
+                one(std::integral_constant<int, 2>{});
+                one(std::integral_constant<int, 3>{});
+                one(std::integral_constant<int, 4>{});
+                one(std::integral_constant<int, 5>{});
+                one(std::integral_constant<int, 6>{});
+                one(std::integral_constant<int, 7>{});
+                one(std::integral_constant<int, 8>{});
+            };
+            const FRec A            = rec[row];
+            const f64 pmass         = fa.mass;
+            const f64 rho_a_inv     = 1. / A.rho;
+            // 1 / (omega_a rho_a): romega is rho_a omega_a, the same product
+            const f64 omega_a_rho_a_inv = 1 / A.romega;
+            const f64 c_du1             = omega_a_rho_a_inv * rho_a_inv;
+            const f64 acs_a = (fa.varying ? A.alpha : fa.alpha_AV) * A.cs;
+            const f64 h4_a  = A.h * A.h * A.h * A.h;
+            const bool fast = A.rh != 0;
+            f64 vdot_max = -1, facc = 0; // facc: this lane's component
+            fold[threadIdx.x][5] = 0.;
+            const f64(*grp)[6]   = fold + (threadIdx.x & ~3u);
+            const u32 sa = lg, sb = lg == 3 ? 4u : 5u;
+            u32 idn = 0;
+            if (steps) {
+                request(id_at(0));
+                idn = id_at(1);
+            }
+            for (u32 t = 0; t < steps; t++) {
+                __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt 0: this pass's records are in LDS
+                wave_lds_sync();
+                union {
+                    FRec B;
+                    double2 p[NP];
+                } u;
+#pragma unroll
+                for (int i = 0; i < NP; i++) u.p[i] = *(const double2 *) (mine + dst[i]);
+                __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt 0: read before the room is reused
+                wave_lds_sync();
+                if (t + 1 < steps) {
+                    request(idn);
+                    idn = id_at(t + 2);
+                }
+                const FRec &B = u.B;
+                f64 tx = 0, ty = 0, tz = 0, tu1 = 0, tu2 = 0;
+                if (t * G + lg < len) {
+                    const f64 dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+                    const f64 rab2 = dx * dx + dy * dy + dz * dz;
+                    f64 rc;
+                    const f64 rab = sqrt_pair(rab2, rc);
+                    // 1 / rab from 1e-9 on, 0 below: two corrections make the estimate the
+                    // correctly rounded reciprocal
+                    rc             = __builtin_fma(__builtin_fma(-rab, rc, 1.), rc, rc);
+                    rc             = __builtin_fma(__builtin_fma(-rab, rc, 1.), rc, rc);
+                    const f64 inv  = rab >= 1e-9 ? rc : 0.;
+                    // dW = norm f'(r / h) / h^4 (sphkernels.hpp:2329-2343) and
+                    // Fab_b / (rho_b omega_b) of the conductivity term, the divisions by way of
+                    // the particles' reciprocals
+                    f64 Fab_a, Fab_b, fb_rom;
+                    if (fast)
+                        Fab_a = div_rcp(KK::norm * K::df(div_rcp(rab, A.h, A.rh)), h4_a, A.rh4);
+                    else
+                        Fab_a = KK::dW(rab, A.h);
+                    if (B.rh != 0) {
+                        const f64 h4_b = B.h * B.h * B.h * B.h;
+                        Fab_b  = div_rcp(KK::norm * K::df(div_rcp(rab, B.h, B.rh)), h4_b, B.rh4);
+                        fb_rom = div_rcp(Fab_b, B.romega, B.rromega);
+                    } else {
+                        Fab_b  = KK::dW(rab, B.h);
+                        fb_rom = Fab_b / B.romega;
+                    }
+                    const f64 vabx = A.vx - B.vx, vaby = A.vy - B.vy, vabz = A.vz - B.vz;
+                    const f64 rux = dx * inv, ruy = dy * inv, ruz = dz * inv;
+                    const f64 v_ab_r_ab = vabx * rux + vaby * ruy + vabz * ruz;
+                    const f64 abs_v     = fabs(v_ab_r_ab);
+                    const f64 vsig_a = acs_a + fa.beta_AV * abs_v;
+                    const f64 vsig_b =
+                        (fa.varying ? B.alpha : fa.alpha_AV) * B.cs + fa.beta_AV * abs_v;
+                    const f64 rho_avg = (A.rho + B.rho) * 0.5;
+                    f64 unused;
+                    const f64 vsig_u = sqrt_pair(fabs(A.P - B.P) / rho_avg, unused);
+                    const f64 qa_ab  = fmax(-0.5 * A.rho * vsig_a * v_ab_r_ab, 0.);
+                    const f64 qb_ab  = fmax(-0.5 * B.rho * vsig_b * v_ab_r_ab, 0.);
+                    const f64 AV_P_a = A.P + qa_ab, AV_P_b = B.P + qb_ab;
+                    const f64 nax = rux * Fab_a, nay = ruy * Fab_a, naz = ruz * Fab_a;
+                    const f64 nbx = rux * Fab_b, nby = ruy * Fab_b, nbz = ruz * Fab_b;
+                    const f64 ia = AV_P_a * A.inv_sub;
+                    const f64 ib = AV_P_b * B.inv_sub;
+                    const f64 mm = -pmass;
+                    tx  = mm * (ia * nax + ib * nbx);
+                    ty  = mm * (ia * nay + ib * nby);
+                    tz  = mm * (ia * naz + ib * nbz);
+                    tu1 = AV_P_a * c_du1 * pmass * (vabx * nax + vaby * nay + vabz * naz);
+                    tu2 = pmass * fa.alpha_u * vsig_u * (A.u - B.u) * 0.5 *
+                          (Fab_a * omega_a_rho_a_inv + fb_rom);
+                    // CFL signal speed: r_ab / |r_ab|, alpha 1, beta 2 (cs + 2 |vdot| is monotone
+                    // in |vdot|, rounding included: the largest one gives the largest speed)
+                    const f64 r2x = div_rcp(dx, rab, inv), r2y = div_rcp(dy, rab, inv),
+                              r2z = div_rcp(dz, rab, inv);
+                    const f64 vdot = vabx * r2x + vaby * r2y + vabz * r2z;
+                    vdot_max       = fmax(vdot_max, fabs(vdot));
+                }
+                f64 *m = fold[threadIdx.x];
+                m[0]   = tx;
+                m[1]   = ty;
+                m[2]   = tz;
+                m[3]   = tu1;
+                m[4]   = tu2;
+                wave_lds_sync();
+#pragma unroll
+                for (int L = 0; L < G; L++) {
+                    facc = facc + grp[L][sa];
+                    facc = facc + grp[L][sb];
+                }
+                wave_lds_sync();
+            }
+            const f64 fx = facc, fy = group_lane<G, 1>(facc), fz = group_lane<G, 2>(facc),
+                      tdu = group_lane<G, 3>(facc);
+            vdot_max           = group_max<G>(vdot_max);
+            const f64 vsig_max = vdot_max < 0 ? 0. : 1.0 * A.cs + 2.0 * vdot_max;
+            u64 key = ORDERED_POS_INF, npair = 0;
+            if (act && lg == 0) {
+                const u32 a = r.outi[row];
+                key   = f64_to_ordered(force_store(o, a, fx, fy, fz, tdu, vsig_max, A.h, fa));
+                npair = len;
+            }
+            key   = block_reduce(key, umin64, lds[0]);
+            npair = block_reduce(npair, [](u64 p, u64 q) { return p + q; }, lds[1]);
+            if (threadIdx.x == 0) {
+                part[blockIdx.x]             = key;
+                part[gridDim.x + blockIdx.x] = npair;
+            }
+        }
+
         // ------------------------------------------------------------- force (mixed)
         // r_ab and the neighbour criterion in FP64, pair terms in FP32, Kahan-compensated
         // per-lane sums combined across the group in FP64
@@ -1864,7 +2096,7 @@ namespace shamx {
         SHAMX_HIP(hipGetLastError());
     }
 
-    void compute_force(hipStream_t s, int kernel, u32 n, Csr c, const void *rec, const f64 *x,
+    void compute_force(hipStream_t s, int kernel, u32 n, u32 nm, Csr c, const void *rec, const f64 *x,
                        const f64 *y, const f64 *z, const f64 *vx, const f64 *vy, const f64 *vz,
                        const f64 *h, const f64 *omega, const f64 *u, const f64 *P, const f64 *cs,
                        f64 *ax, f64 *ay, f64 *az, f64 *du, f64 *ax_old, f64 *ay_old,
@@ -1888,6 +2120,14 @@ namespace shamx {
                             n, r,
                             SoASrc<KT, FRec32>{x, y, z, vx, vy, vz, h, omega, u, P, cs, fa.mass},
                             h, o, fa, part.data());
+                } else if (rec && G == 4) {
+                    // (the force rows' ids are below nm)
+                    if ((u64) nm * sizeof(FRec) > 0xffffffffull)
+                        k_force_rows<KT, true><<<nb, BLK, 0, s>>>(n, r, (const FRec *) rec, o, fa,
+                                                                  part.data());
+                    else
+                        k_force_rows<KT, false><<<nb, BLK, 0, s>>>(n, r, (const FRec *) rec, o,
+                                                                   fa, part.data());
                 } else {
                     if (rec)
                         k_force<KT, G><<<nb, BLK, 0, s>>>(
