@@ -446,10 +446,19 @@ namespace shamx {
         // time; those farther from the members' bounding box than both the members' largest
         // cut radius and their own are dropped (they cannot pass the pair test: the box
         // distance bounds every member distance from below, kept with a 1e-12 margin so that
-        // rounding cannot drop a pair), and the rest are compacted into LDS in order (sorted
-        // index, position, cut radius).  The wave then tests P candidates x M members per
-        // instruction, lane = candidate * M + member, so the kept lanes of one member are in
-        // candidate order and its row is the compaction of a ballot restricted to its lanes.
+        // rounding cannot drop a pair), and the rest are queued in order.  64 queued ones at a time,
+        // a lane each, are tested against the members one after the other; a member's row grows
+        // by the lanes of its ballot.  A lane finds its candidate from a bit mask of the ranges'
+        // first candidates.  The queue keeps the lanes of the pair tests full whatever the
+        // members' number and the share of candidates dropped.  (With tests on candidate x member
+        // lanes right after each 64 candidates, many lanes idled, and each lane searched its range
+        // by bisection, six dependent LDS reads.)  It holds sorted positions alone: a queued
+        // particle is read again, a cache hit.  With its position kept in LDS as well the kernel
+        // had 4 waves per SIMD for 8 and spent 58 % of the time in waits.  Bound by these loads'
+        // latency and by the issue of about 20 instructions per member and 64 candidates; the next
+        // leaves and candidates are requested while the present ones are tested.
+        // Before, with the positions in LDS, now: 2.1M Sedov 1.63, 1.61, 1.38 ms; 4M Plummer
+        // 4.58, 4.42, 3.53 ms; 1M disc 0.89, 0.83, 0.68 ms.  (Two members per turn: no change.)
         // n_items: the batches beyond the leaves' first ones.
         // LIST: one wave per particle of list (item_leaf holds particle ids, n_items their
         // count): its whole row at offset[its sorted position], the path of rows longer than
@@ -458,22 +467,25 @@ namespace shamx {
         __global__ void __launch_bounds__(GRP_WAVES * WAVE)
             k_group_neigh(u32 n, u32 L, u32 I, const f64 *__restrict nodes,
                           const u32 *__restrict sort_index, const double4 *__restrict ps,
-                          const u32 *__restrict owner, const u32 *__restrict leaf_cnt,
-                          const u32 *__restrict leaf_offset, const u32 *__restrict leaf_ids,
-                          const u32 *__restrict item_leaf, const u32 *__restrict xstart,
-                          const u32 *__restrict n_items, f64 htol, f64 Rker2,
+                          const u32 *__restrict owner, const u32 *__restrict lap,
+                          const u32 *__restrict leaf_cnt, const u32 *__restrict leaf_offset,
+                          const u32 *__restrict leaf_ids, const u32 *__restrict item_leaf,
+                          const u32 *__restrict xstart, const u32 *__restrict n_items, f64 htol,
+                          f64 Rker2,
                           u32 *__restrict cnt, u32 *__restrict offset, u32 *__restrict ids,
                           u32 cap, u32 leaf_cap, const u32 *__restrict inv = nullptr,
                           const f64 *__restrict bbox = nullptr) {
-            __shared__ u32 rstart[GRP_WAVES][WAVE], rexcl[GRP_WAVES][WAVE];
+            constexpr u32 QN = 2 * WAVE;
+            __shared__ u32 queue[GRP_WAVES][QN];    // queued candidates: sorted positions
+            __shared__ double4 mpos[GRP_WAVES][WAVE]; // member x, y, z, cut radius^2
+            // the ranges of a pass: sorted position less index of the first candidate, that index
+            __shared__ uint2 rng[GRP_WAVES][WAVE];
+            __shared__ u32 first[GRP_WAVES][2]; // bit c: candidate c of a window starts a range
             // BCULL: the neighbour leaves of one pass (range, leaf, batches before it)
             __shared__ u32 lr0[GRP_WAVES][BCULL ? WAVE : 1], lr1[GRP_WAVES][BCULL ? WAVE : 1];
             __shared__ u32 lbs[GRP_WAVES][BCULL ? WAVE : 1], lbx[GRP_WAVES][BCULL ? WAVE : 1];
-            __shared__ double4 cpos[GRP_WAVES][WAVE]; // candidate x, y, z, cut radius^2
-            __shared__ u32 cid[GRP_WAVES][WAVE];      // candidate id written to the rows
-            __shared__ double4 mpos[GRP_WAVES][WAVE]; // member x, y, z, cut radius^2
-            __shared__ u32 mrow[GRP_WAVES][WAVE];     // member row start
-            const int lane = __lane_id(), wid = threadIdx.x / WAVE;
+            const int lane = __lane_id();
+            const u32 wid  = (u32) __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
             const u32 item = blockIdx.x * GRP_WAVES + wid;
             if (item >= (LIST ? 0u : L) + *n_items) return;
             u32 l, mb, m1;
@@ -483,7 +495,7 @@ namespace shamx {
                 mb           = inv[a0];
                 m1           = mb + 1;
             } else {
-                l = item_leaf[item];
+                l = item < L ? item : item_leaf[item];
                 u32 m0;
                 node_children(nodes, I + l, m0, m1);
                 mb = m0 + item_batch(item, l, L, xstart) * WAVE;
@@ -493,16 +505,20 @@ namespace shamx {
             // entries; the build is repeated then, but nothing may be read past the row
             const u32 k0 = leaf_offset[l],
                       k1 = k0 + (leaf_cap ? min(leaf_cnt[l], leaf_cap) : leaf_cnt[l]);
+            // the first neighbour leaves, requested before the members are looked at; in the loop
+            // below the next ones are requested a pass ahead
+            u32 nd_next     = k0 + lane < k1 ? leaf_ids[k0 + lane] : 0u;
+            const bool all  = lap[l] == 0; // the leaf owns all its particles (k_owner)
             u32 sm   = mb + lane;
             bool mem = false;
             u32 a    = 0;
             double4 pa{0, 0, 0, 0};
             if (sm < m1) {
-                a = sort_index[sm];
-                if (a < n && owner[a] == l) {
-                    mem       = true;
-                    double4 p = ps[sm];
-                    f64 ra    = p.w * htol;
+                a               = sort_index[sm];
+                const double4 p = ps[sm];
+                if (a < n && (all || owner[a] == l)) {
+                    mem    = true;
+                    f64 ra = p.w * htol;
                     pa        = make_double4(p.x, p.y, p.z, ra * ra * Rker2);
                 }
             }
@@ -512,9 +528,12 @@ namespace shamx {
             const u32 rank = (u32) __popcll(members & lt); // member index of this lane
             const u32 ia   = SORTED ? sm : a;
             const u32 row0 = STRIDE ? (mem ? ia * cap : 0u) : ((FILL && mem) ? offset[ia] : 0u);
-            if (mem) {
-                mpos[wid][rank] = pa;
-                mrow[wid][rank] = row0;
+            if (mem) mpos[wid][rank] = pa;
+            // lane m (< M): row start and length so far of the member of rank m
+            u32 mrow, mlen = 0;
+            {
+                // lane `rank` receives from the member lane of that rank
+                mrow = (u32) __builtin_amdgcn_ds_permute((int) (mem ? rank : 63u) * 4, (int) row0);
             }
             // the members' bounding box and largest cut radius^2
             constexpr f64 BIG = 1.7976931348623157e308;
@@ -524,75 +543,93 @@ namespace shamx {
             const f64 bly = wave_reduce(mem ? pa.y : BIG, fmn), bhy = wave_reduce(mem ? pa.y : -BIG, fmx);
             const f64 blz = wave_reduce(mem ? pa.z : BIG, fmn), bhz = wave_reduce(mem ? pa.z : -BIG, fmx);
             const f64 br2 = wave_reduce(mem ? pa.w : 0.0, fmx);
-            // lane = c * M + mi: P candidates per pass; lanes past P * M stay idle
-            const u32 P  = WAVE / M;
-            const u32 mi = (u32) lane % M, ci = (u32) lane / M;
-            const bool on = ci < P;
-            u64 mine = 0; // this member's lanes
-            for (u32 c = 0; c < P; c++) mine |= 1ull << (c * M + mi);
-            wave_lds_sync();
-            const double4 me = mpos[wid][on ? mi : 0];
-            const u32 mrow0  = mrow[wid][on ? mi : 0];
-            u32 cursor = mrow0, count = 0;
-            // the candidates of the ranges rstart / rexcl [0, nr), `total` in all: staged 64 at
-            // a time, tested against the members
-            auto candidates = [&](const u32 nr, const u32 total) {
-                for (u32 c0 = 0; c0 < total; c0 += WAVE) {
-                    // stage 64 candidates: lane j takes candidate c0 + j; the ones that can
-                    // reach a member are compacted to the front of cpos / cid
-                    u32 cn;
-                    {
-                        const u32 c = c0 + lane;
-                        // the range holding candidate c: largest j with rexcl[j] <= c
-                        // (a dropped range is empty and shares its rexcl with the next one, so
-                        // the largest such j is a range that holds c)
-                        u32 j = 0;
-                        for (u32 st = WAVE / 2; st > 0; st >>= 1) {
-                            u32 t = j + st;
-                            if (t < nr && rexcl[wid][t] <= c) j = t;
-                        }
-                        const bool valid = c < total;
-                        u32 sb    = valid ? rstart[wid][j] + (c - rexcl[wid][j]) : 0u;
-                        double4 q = ps[sb];
-                        f64 rb    = q.w * htol;
-                        f64 rb2   = rb * rb * Rker2;
-                        f64 ex = q.x < blx ? blx - q.x : (q.x > bhx ? q.x - bhx : 0.0);
-                        f64 ey = q.y < bly ? bly - q.y : (q.y > bhy ? q.y - bhy : 0.0);
-                        f64 ez = q.z < blz ? blz - q.z : (q.z > bhz ? q.z - bhz : 0.0);
-                        f64 d2 = (ex * ex + ey * ey + ez * ez) * (1.0 - 1e-12);
-                        const bool near = valid & !((d2 > br2) & (d2 > rb2));
-                        const u64 nm    = __ballot(near);
-                        const u32 pos   = (u32) __popcll(nm & lt);
-                        cn              = (u32) __popcll(nm);
-                        wave_lds_sync();
-                        if (near) {
-                            cpos[wid][pos] = make_double4(q.x, q.y, q.z, rb2);
-                            cid[wid][pos]  = FILL ? (SORTED ? sb : sort_index[sb]) : 0u;
-                        }
-                        wave_lds_sync();
+            auto at = [](u32 v, u32 l) { return (u32) __builtin_amdgcn_readlane((int) v, (int) l); };
+            // lanes of m below this one
+            auto below = [](u64 m) {
+                return (u32) __builtin_amdgcn_mbcnt_hi(
+                    (u32) (m >> 32), (u32) __builtin_amdgcn_mbcnt_lo((u32) m, 0u));
+            };
+            u32 qh = 0, qn = 0; // first queued candidate and their number (wave-uniform)
+            // the first nq (<= 64) queued candidates against the members
+            auto test = [&](u32 nq) {
+                const bool on = (u32) lane < nq;
+                const u32 sl  = (qh + (on ? (u32) lane : 0u)) % QN;
+                const u32 sb    = queue[wid][sl];
+                double4 q       = ps[sb];
+                const f64 rb    = q.w * htol;
+                q.w             = rb * rb * Rker2;
+                const u32 id    = FILL ? (SORTED ? sb : sort_index[sb]) : 0u;
+                for (u32 m = 0; m < M; m++) {
+                    const double4 me = mpos[wid][m];
+                    const f64 dx = me.x - q.x, dy = me.y - q.y, dz = me.z - q.z;
+                    const f64 rab2  = dx * dx + dy * dy + dz * dz;
+                    const bool keep = on & !((rab2 > me.w) & (rab2 > q.w));
+                    const u64 km    = __ballot(keep);
+                    const u32 len   = at(mlen, m);
+                    if (FILL && keep) {
+                        const u32 p = len + below(km);
+                        if (!STRIDE || p < cap) ids[at(mrow, m) + p] = id;
                     }
-                    for (u32 cb0 = 0; cb0 < cn; cb0 += P) {
-                        const u32 cl = cb0 + ci; // candidate of this lane
-                        bool keep    = false;
-                        if (on && cl < cn) {
-                            const double4 q = cpos[wid][cl];
-                            f64 dx = me.x - q.x, dy = me.y - q.y, dz = me.z - q.z;
-                            f64 rab2 = dx * dx + dy * dy + dz * dz;
-                            keep     = !((rab2 > me.w) & (rab2 > q.w));
-                        }
-                        const u64 km = __ballot(keep);
-                        const u64 kt = km & mine;
-                        if (FILL && keep) {
-                            u32 pos = cursor + (u32) __popcll(kt & lt);
-                            if (STRIDE) {
-                                if (pos < mrow0 + cap) ids[pos] = cid[wid][cl];
-                            } else {
-                                ids[pos] = cid[wid][cl];
-                            }
-                        }
-                        const u32 kc = (u32) __popcll(kt);
-                        cursor += kc;
-                        count += kc;
+                    mlen = (u32) lane == m ? len + (u32) __popcll(km) : mlen;
+                }
+                qh += nq;
+                qn -= nq;
+            };
+            // candidates of this lane's range [s0, s0 + sz) of sorted positions, the lanes' ranges
+            // in order: the near ones into the queue, tested when there are 64
+            auto candidates = [&](u32 s0, u32 sz) {
+                u32 inc = sz;
+                for (int o = 1; o < WAVE; o <<= 1) {
+                    u32 t = __shfl_up(inc, o, WAVE);
+                    if (lane >= o) inc += t;
+                }
+                const u32 total = at(inc, WAVE - 1);
+                if (total == 0) return;
+                const u64 some = __ballot(sz > 0);
+                const u32 nr   = (u32) __popcll(some);
+                wave_lds_sync();
+                if (sz) rng[wid][below(some)] = make_uint2(s0 - (inc - sz), inc - sz);
+                wave_lds_sync();
+                const u32 start = (u32) lane < nr ? rng[wid][lane].y : 0xffffffffu;
+                // the sorted position of candidate c0 + lane
+                auto find = [&](u32 c0) -> u32 {
+                    // ranges begun before this window, and those that begin in it
+                    const u32 before = (u32) __popcll(__ballot(start < c0));
+                    const u32 w      = start - c0;
+                    if (lane < 2) first[wid][lane] = 0;
+                    wave_lds_sync();
+                    if (w < (u32) WAVE && start != 0xffffffffu)
+                        atomicOr(&first[wid][w / 32], 1u << (w % 32));
+                    wave_lds_sync();
+                    const u64 fm = (u64) first[wid][0] | ((u64) first[wid][1] << 32);
+                    const u32 c  = c0 + lane;
+                    const u32 j  = before + below(fm) + (u32) ((fm >> lane) & 1ull) - 1;
+                    return c < total ? rng[wid][j].x + c : 0u;
+                };
+                u32 sb_next    = find(0);
+                double4 q_next = ps[sb_next];
+                for (u32 c0 = 0; c0 < total; c0 += WAVE) {
+                    const u32 sb     = sb_next;
+                    const double4 q  = q_next;
+                    const bool valid = c0 + lane < total;
+                    if (c0 + WAVE < total) { // the next candidates load while these are tested
+                        sb_next = find(c0 + WAVE);
+                        q_next  = ps[sb_next];
+                    }
+                    f64 rb    = q.w * htol;
+                    f64 rb2   = rb * rb * Rker2;
+                    f64 ex = q.x < blx ? blx - q.x : (q.x > bhx ? q.x - bhx : 0.0);
+                    f64 ey = q.y < bly ? bly - q.y : (q.y > bhy ? q.y - bhy : 0.0);
+                    f64 ez = q.z < blz ? blz - q.z : (q.z > bhz ? q.z - bhz : 0.0);
+                    f64 d2 = (ex * ex + ey * ey + ez * ez) * (1.0 - 1e-12);
+                    const bool near = valid & !((d2 > br2) & (d2 > rb2));
+                    const u64 nm    = __ballot(near);
+                    if (near) queue[wid][(qh + qn + below(nm)) % QN] = sb;
+                    qn += (u32) __popcll(nm);
+                    wave_lds_sync();
+                    if (qn >= (u32) WAVE) {
+                        test(WAVE);
+                        wave_lds_sync();
                     }
                 }
             };
@@ -600,9 +637,10 @@ namespace shamx {
                 // neighbour leaves in batches of up to 64: lane i loads the range of the i-th
                 // leaf of the batch; candidates are the concatenated ranges in order
                 u32 k  = kb + lane;
-                u32 r0 = 0, r1 = 0, nd = 0;
+                u32 r0 = 0, r1 = 0;
+                const u32 nd = nd_next;
+                nd_next      = k + WAVE < k1 ? leaf_ids[k + WAVE] : 0u;
                 if (k < k1) {
-                    nd = leaf_ids[k];
                     node_children(nodes, nd, r0, r1); // leaf: sorted range
                     // the whole range is dropped when none of its particles can reach a
                     // member: the leaf's box is farther from the members' box than both the
@@ -619,18 +657,7 @@ namespace shamx {
                 }
                 const u32 nr = min(k1 - kb, (u32) WAVE);
                 if constexpr (!BCULL) {
-                    u32 sz  = r1 - r0;
-                    u32 inc = sz;
-                    for (int o = 1; o < WAVE; o <<= 1) {
-                        u32 t = __shfl_up(inc, o, WAVE);
-                        if (lane >= o) inc += t;
-                    }
-                    const u32 total = __shfl(inc, WAVE - 1, WAVE);
-                    wave_lds_sync();
-                    rstart[wid][lane] = r0;
-                    rexcl[wid][lane]  = inc - sz;
-                    wave_lds_sync();
-                    candidates(nr, total);
+                    candidates(r0, r1 - r0);
                 } else {
                     // each range split into the member batches of its leaf (64 sorted
                     // positions from the leaf's start; bbox: their boxes and largest cut
@@ -669,27 +696,13 @@ namespace shamx {
                             const f64 d2  = (ex * ex + ey * ey + ez * ez) * (1.0 - 1e-12);
                             if (d2 > br2 && d2 > bx[6]) s1 = s0;
                         }
-                        const u32 sz = s1 - s0;
-                        u32 inc      = sz;
-                        for (int o = 1; o < WAVE; o <<= 1) {
-                            u32 t = __shfl_up(inc, o, WAVE);
-                            if (lane >= o) inc += t;
-                        }
-                        const u32 total = __shfl(inc, WAVE - 1, WAVE);
-                        wave_lds_sync();
-                        rstart[wid][lane] = s0;
-                        rexcl[wid][lane]  = inc - sz;
-                        wave_lds_sync();
-                        candidates(min(totb - t0, (u32) WAVE), total);
+                        candidates(s0, s1 - s0);
                     }
                 }
             }
-            // lane mi (< M) holds member mi's count; the member lane of rank mi writes it
-            wave_lds_sync();
-            if (on && ci == 0) mrow[wid][mi] = count;
-            wave_lds_sync();
+            if (qn) test(qn);
+            const u32 cm = __shfl(mlen, (int) rank, WAVE);
             if (mem) {
-                u32 cm = mrow[wid][rank];
                 if (!FILL || STRIDE) cnt[ia] = cm;
                 if (STRIDE) offset[ia] = row0;
             }
@@ -865,7 +878,7 @@ namespace shamx {
             const f64 *bb = batch_boxes(s, nb, t, gblocks, htol, Rker2);
             launch_group<false, SORTED, false>(s, gblocks, bb,
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
-                nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
+                nb.owner.data(), nb.lap.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
                 nb.item_leaf.data(), nb.xstart.data(), n_items, htol, Rker2, nb.cnt.data(),
                 nullptr, nullptr, 0, leaf_cap);
             k_part_neigh<false, SORTED, false><<<div_up(n_local, 128), 128, 0, s>>>(
@@ -888,7 +901,7 @@ namespace shamx {
             nb.ids.resize(std::max<u64>(nb.n_pairs, 1));
             launch_group<true, SORTED, false>(s, gblocks, bb,
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
-                nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
+                nb.owner.data(), nb.lap.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
                 nb.item_leaf.data(), nb.xstart.data(), n_items, htol, Rker2, nullptr,
                 nb.offset.data(), nb.ids.data(), 0, leaf_cap);
             k_part_neigh<true, SORTED, false><<<div_up(n_local, 128), 128, 0, s>>>(
@@ -1093,7 +1106,7 @@ namespace shamx {
             nb.ids.resize(std::max<u64>((u64) nm * cp, 1));
             launch_group<true, true, true>(s, gblocks, batch_boxes(s, nb, t, gblocks, htol, Rker2),
                 n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
-                nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
+                nb.owner.data(), nb.lap.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
                 nb.item_leaf.data(), nb.xstart.data(), nb.counters.data() + 7, htol, Rker2,
                 nb.cnt.data(), nb.offset.data(), nb.ids.data(), cp, leaf_cap);
             k_part_neigh<true, true, true><<<div_up(n_local, 128), 128, 0, s>>>(
@@ -1130,7 +1143,7 @@ namespace shamx {
                 k_group_neigh<true, true, false, true>
                     <<<div_up(hc[14], (u32) GRP_WAVES), GRP_WAVES * WAVE, 0, s>>>(
                         n_local, L, I, t.nodes.data(), t.sort_index.data(), nb.ps.data(),
-                        nb.owner.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(),
+                        nb.owner.data(), nb.lap.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(),
                         nb.leaf_ids.data(), nb.olist.data(), nullptr, nb.counters.data() + 14,
                         htol, Rker2, nullptr, nb.offset.data(), nb.ids.data(), 0, 0,
                         nb.inv.data());
