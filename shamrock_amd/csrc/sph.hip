@@ -160,6 +160,10 @@ namespace shamx {
             return v;
         }
 
+        __device__ inline u32 wave_id() {
+            return (u32) __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
+        }
+
         // rows of the neighbour CSR processed by a kernel: the j-th processed particle has row
         // sel[j] (identity when null) and particle id outi[row] (identity when null)
         struct Rows {
@@ -178,6 +182,112 @@ namespace shamx {
         struct PosSoA {
             const f64 *__restrict x, *__restrict y, *__restrict z;
             __device__ double3 pos(u32 b) const { return make_double3(x[b], y[b], z[b]); }
+        };
+
+        // sqrt(v) correctly rounded for zero, infinity and 2^-767 < v (below, without the scaling
+        // of a general sqrt, its last bits; squared distances and P / rho ratios of a run are far
+        // above), and a value within an ulp or two of 1 / sqrt(v): the hardware estimate, one
+        // Newton step for both, two residual corrections of the root
+        __device__ inline f64 sqrt_pair(f64 v, f64 &recip) {
+            const f64 r0 = __builtin_amdgcn_rsq(v);
+            f64 s = v * r0, g = 0.5 * r0;
+            const f64 e = __builtin_fma(-g, s, 0.5);
+            g           = __builtin_fma(g, e, g);
+            s           = __builtin_fma(s, e, s);
+            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
+            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
+            recip       = g + g;
+            return __builtin_amdgcn_class(v, 0x260) ? v : s; // +-0 and +inf: themselves
+        }
+
+        // Rows of sorted position records, four lanes per particle.  A lane that gathers its own
+        // 32-byte record makes each of its two loads touch 64 lines; here the lanes of a particle
+        // fetch their records together, two records per instruction (quad lanes 0, 1 the halves of
+        // one, 2, 3 of the next), straight into LDS, and each reads its own from there.
+        // U passes (of four entries) per turn: read them, request the next turn's, use them.
+        // All lanes of a wave take part until its longest row ends.
+        template<int U>
+        struct QuadPos {
+            static constexpr u32 ROOM = 2 * U * WAVE; // double2 per wave
+            const char *recs;
+            char *mine;
+            u32 own; // this lane's record of pass 0 in the room
+            const u32 *ids;
+            u32 k0, len, lg, none;
+            __device__ QuadPos(const double4 *ps, double2 *room, const u32 *ids, u32 k0, u32 len,
+                               u32 none)
+                : ids(ids), k0(k0), len(len), none(none) {
+                const u32 lane = (u32) __lane_id();
+                lg   = lane % 4;
+                recs = (const char *) ps + (lg % 2) * 16;
+                mine = (char *) room;
+                own  = (lg / 2) * (WAVE * 16) + (lane / 4) * 64 + (lg % 2) * 32;
+            }
+            // turns of the longest row of the wave: all lanes load in all of them
+            __device__ u32 turns() const {
+                const u32 m = wave_reduce(len, [](u32 p, u32 q) { return p > q ? p : q; });
+                return ((u32) __builtin_amdgcn_readfirstlane((int) m) + 4 * U - 1) / (4 * U);
+            }
+            // ids of turn t; past the row's end its last entry, of an empty row `none`
+            __device__ void load_ids(u32 t, u32 (&id)[U]) const {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const u32 k = (t * U + (u32) u) * 4 + lg;
+                    id[u]       = len ? ids[k0 + min(k, len - 1)] : none;
+                }
+            }
+            template<int C>
+            __device__ void one(u32 id, u32 at) const {
+                const u32 w = (u32) __builtin_amdgcn_mov_dpp((int) id, C, 0xf, 0xf, true);
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *) (recs +
+                                                                      (u64) w * sizeof(double4)),
+                    (__attribute__((address_space(3))) void *) (mine + at * WAVE * 16), 16, 0, 0);
+            }
+            __device__ void request(const u32 (&id)[U]) const {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    one<0x50>(id[u], 2 * u);     // quad_perm 0, 0, 1, 1
+                    one<0xfa>(id[u], 2 * u + 1); // 2, 2, 3, 3
+                }
+            }
+            // the requested records; the room is free again afterwards
+            __device__ void take(double4 (&q)[U]) const {
+                __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt 0
+                wave_lds_sync();
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    q[u] = *(const double4 *) (mine + u * 2 * WAVE * 16 + own);
+                __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt 0
+                wave_lds_sync();
+            }
+            // use(u-th pass's entry is in the row, its id, record) in list order per pass
+            template<class Use>
+            __device__ void sweep(Use &&use) const {
+                const u32 T = turns();
+                if (!T) return;
+                u32 id[U], idn[U];
+                load_ids(0, id);
+                request(id);
+                load_ids(1, idn);
+                for (u32 t = 0; t < T; t++) {
+                    double4 q[U];
+                    u32 cur[U];
+                    take(q);
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        cur[u] = id[u];
+                        id[u]  = idn[u];
+                    }
+                    if (t + 1 < T) {
+                        request(idn);
+                        load_ids(t + 2, idn);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        use((t * U + (u32) u) * 4 + lg < len, cur[u], q[u]);
+                }
+            }
         };
 
         __device__ inline void kahan_add(f32 &s, f32 &c, f32 v) {
@@ -235,7 +345,63 @@ namespace shamx {
             const bool work = act && e > 1e-6;
             const f64 Rkern = K::Rkern;
             f64 h_a = 0, rho_sum = 0, sumdWdh = 0;
-            if (work) {
+            constexpr bool QUAD = G == 4 && std::is_same<Src, PosRec>::value;
+            if constexpr (QUAD) {
+                // Passes per turn, the sweeps' cost with 1, 2, 4 (0.70 and 0.167 ms when each lane
+                // gathered its records): FP64, 2.1M Sedov 0.72, 0.62, 0.62 ms, 4M Plummer 0.325,
+                // 0.318, 0.345 ms on average; mixed, 1M disc 0.181, 0.157, 0.153 ms.  The address
+                // units, busy 69 % of the time before, bound it no longer; what does is the VALU
+                // work of a pair (FP64: ordered sums, square root) at the 5 waves per SIMD that
+                // its registers leave, and latency.  The same fetch slows Omega (1.56 to 1.76 ms),
+                // whose LDS ring and registers leave no room for it.
+                using QP = QuadPos<MIXED ? 4 : 2>;
+                __shared__ __attribute__((aligned(16))) double2 room[BLK / WAVE][QP::ROOM];
+                const u32 k0 = work ? r.off[row] : 0u, len = work ? r.cnt[row] : 0u;
+                const QP rows(src.ps, room[wave_id()], r.ids, k0, len, row);
+                if (work) h_a = h_new[a];
+                const double3 pa = src.pos(row);
+                const f64 dint   = h_a * h_a * Rkern * Rkern;
+                auto dist2 = [&](const double4 &q) {
+                    const f64 dx = pa.x - q.x, dy = pa.y - q.y, dz = pa.z - q.z;
+                    return dx * dx + dy * dy + dz * dz;
+                };
+                if constexpr (MIXED) {
+                    using KI = KernInv<K>;
+                    f32 ih   = (f32) (1. / h_a);
+                    f32 ih3  = ih * ih * ih, ih4 = ih3 * ih;
+                    f32 rs = 0, rc = 0, ds = 0, dc = 0;
+                    // each lane sums its own entries in order
+                    rows.sweep([&](bool in, u32, const double4 &q) {
+                        const f64 rab2 = dist2(q);
+                        if (!in || rab2 > dint) return;
+                        f32 rab = sqrt_approx((f32) rab2);
+                        kahan_add(rs, rc, KI::W(rab, ih, ih3));
+                        kahan_add(ds, dc, KI::dhW(rab, ih, ih4));
+                    });
+                    rho_sum = (f64) rs - (f64) rc;
+                    sumdWdh = (f64) ds - (f64) dc;
+                } else {
+                    const KernAt<K> ka(h_a);
+                    // terms folded in list order
+                    rows.sweep([&](bool in, u32, const double4 &q) {
+                        f64 tw = 0, th = 0;
+                        const f64 rab2 = dist2(q);
+                        if (in && !(rab2 > dint)) {
+                            f64 unused;
+                            const f64 rab = sqrt_pair(rab2, unused);
+                            if (ka.fast) {
+                                tw = mass * ka.template W<true>(rab);
+                                th = mass * ka.template dhW<true>(rab);
+                            } else {
+                                tw = mass * ka.template W<false>(rab);
+                                th = mass * ka.template dhW<false>(rab);
+                            }
+                        }
+                        rho_sum = ordered_fold<G>(rho_sum, tw);
+                        sumdWdh = ordered_fold<G>(sumdWdh, th);
+                    });
+                }
+            } else if (work) {
                 h_a         = h_new[a];
                 double3 pa  = src.pos(row);
                 f64 dint    = h_a * h_a * Rkern * Rkern;
@@ -958,22 +1124,6 @@ namespace shamx {
         }
 
         // ------------------------------------------------------------- force (FP64, solver rows)
-        // sqrt(v) correctly rounded for zero, infinity and 2^-767 < v (below, without the scaling
-        // of a general sqrt, its last bits; squared distances and P / rho ratios of a run are far
-        // above), and a value within an ulp or two of 1 / sqrt(v): the hardware estimate, one
-        // Newton step for both, two residual corrections of the root
-        __device__ inline f64 sqrt_pair(f64 v, f64 &recip) {
-            const f64 r0 = __builtin_amdgcn_rsq(v);
-            f64 s = v * r0, g = 0.5 * r0;
-            const f64 e = __builtin_fma(-g, s, 0.5);
-            g           = __builtin_fma(g, e, g);
-            s           = __builtin_fma(s, e, s);
-            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
-            s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
-            recip       = g + g;
-            return __builtin_amdgcn_class(v, 0x260) ? v : s; // +-0 and +inf: themselves
-        }
-
         // piece of 16 bytes q (0..35) of a group's four records: byte offset inside its record,
         // and the lane of the group whose record it is
         constexpr int FR_PIECES = sizeof(FRec) / 16; // 9
