@@ -200,28 +200,40 @@ namespace shamx {
             return __builtin_amdgcn_class(v, 0x260) ? v : s; // +-0 and +inf: themselves
         }
 
-        // Rows of sorted position records, four lanes per particle.  A lane that gathers its own
-        // 32-byte record makes each of its two loads touch 64 lines; here the lanes of a particle
-        // fetch their records together, two records per instruction (quad lanes 0, 1 the halves of
-        // one, 2, 3 of the next), straight into LDS, and each reads its own from there.
+        // Rows of sorted records of 32 or 64 bytes, four lanes per particle.  A lane that gathers
+        // its own record makes each of its loads touch 64 lines; here the lanes of a particle
+        // fetch their four records together, 64 contiguous bytes per instruction (two records or
+        // one), straight into LDS, and each reads its own from there.  Pieces of 16 bytes are
+        // turned by their record's number, so that the lanes that read at once meet different
+        // banks.
         // U passes (of four entries) per turn: read them, request the next turn's, use them.
         // All lanes of a wave take part until its longest row ends.
-        template<int U>
-        struct QuadPos {
-            static constexpr u32 ROOM = 2 * U * WAVE; // double2 per wave
+        template<class T, int U>
+        struct QuadRows {
+            static constexpr int NP   = sizeof(T) / 16;     // pieces of a record, loads of a pass
+            static constexpr u32 ROOM = (u32) U * NP * WAVE; // double2 per wave
+            static_assert(sizeof(T) == 32 || sizeof(T) == 64);
             const char *recs;
             char *mine;
-            u32 own; // this lane's record of pass 0 in the room
+            u32 piece[NP]; // offset in its record of the piece loaded by load c
+            u32 own[NP];   // offset in the room of pass 0 of this lane's own pieces
             const u32 *ids;
             u32 k0, len, lg, none;
-            __device__ QuadPos(const double4 *ps, double2 *room, const u32 *ids, u32 k0, u32 len,
-                               u32 none)
-                : ids(ids), k0(k0), len(len), none(none) {
+            // a record's pieces are turned by this much
+            static constexpr __device__ u32 turn(u32 rec) { return NP == 4 ? rec : rec / 2; }
+            __device__ QuadRows(const T *rec, double2 *room, const u32 *ids, u32 k0, u32 len,
+                                u32 none)
+                : recs((const char *) rec), mine((char *) room), ids(ids), k0(k0), len(len),
+                  none(none) {
                 const u32 lane = (u32) __lane_id();
-                lg   = lane % 4;
-                recs = (const char *) ps + (lg % 2) * 16;
-                mine = (char *) room;
-                own  = (lg / 2) * (WAVE * 16) + (lane / 4) * 64 + (lg % 2) * 32;
+                lg             = lane % 4;
+#pragma unroll
+                for (u32 c = 0; c < NP; c++) {
+                    const u32 q = 4 * c + lg;
+                    piece[c]    = (q - turn(q / NP)) % NP * 16;
+                    own[c]      = (lg * NP / 4) * (WAVE * 16) + (lane / 4) * 64 +
+                             ((lg * NP) % 4 + (c + turn(lg)) % NP) * 16;
+                }
             }
             // turns of the longest row of the wave: all lanes load in all of them
             __device__ u32 turns() const {
@@ -237,41 +249,56 @@ namespace shamx {
                 }
             }
             template<int C>
-            __device__ void one(u32 id, u32 at) const {
-                const u32 w = (u32) __builtin_amdgcn_mov_dpp((int) id, C, 0xf, 0xf, true);
+            __device__ void one(u32 id, int u) const {
+                constexpr int perm = (4 * C / NP) | ((4 * C + 1) / NP << 2) |
+                                     ((4 * C + 2) / NP << 4) | ((4 * C + 3) / NP << 6);
+                const u32 w = (u32) __builtin_amdgcn_mov_dpp((int) id, perm, 0xf, 0xf, true);
                 __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void *) (recs +
-                                                                      (u64) w * sizeof(double4)),
-                    (__attribute__((address_space(3))) void *) (mine + at * WAVE * 16), 16, 0, 0);
+                    (const __attribute__((address_space(1))) void *) (recs + (u64) w * sizeof(T) +
+                                                                      piece[C]),
+                    (__attribute__((address_space(3))) void *) (mine + (u * NP + C) * WAVE * 16),
+                    16, 0, 0);
             }
             __device__ void request(const u32 (&id)[U]) const {
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    one<0x50>(id[u], 2 * u);     // quad_perm 0, 0, 1, 1
-                    one<0xfa>(id[u], 2 * u + 1); // 2, 2, 3, 3
+                    one<0>(id[u], u);
+                    one<1>(id[u], u);
+                    if constexpr (NP == 4) {
+                        one<2>(id[u], u);
+                        one<3>(id[u], u);
+                    }
                 }
             }
             // the requested records; the room is free again afterwards
-            __device__ void take(double4 (&q)[U]) const {
+            __device__ void take(T (&q)[U]) const {
                 __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt 0
                 wave_lds_sync();
 #pragma unroll
-                for (int u = 0; u < U; u++)
-                    q[u] = *(const double4 *) (mine + u * 2 * WAVE * 16 + own);
+                for (int u = 0; u < U; u++) {
+                    union {
+                        T rec;
+                        double2 p[NP];
+                    } v;
+#pragma unroll
+                    for (int c = 0; c < NP; c++)
+                        v.p[c] = *(const double2 *) (mine + u * NP * WAVE * 16 + own[c]);
+                    q[u] = v.rec;
+                }
                 __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt 0
                 wave_lds_sync();
             }
             // use(u-th pass's entry is in the row, its id, record) in list order per pass
             template<class Use>
             __device__ void sweep(Use &&use) const {
-                const u32 T = turns();
-                if (!T) return;
+                const u32 nt = turns();
+                if (!nt) return;
                 u32 id[U], idn[U];
                 load_ids(0, id);
                 request(id);
                 load_ids(1, idn);
-                for (u32 t = 0; t < T; t++) {
-                    double4 q[U];
+                for (u32 t = 0; t < nt; t++) {
+                    T q[U];
                     u32 cur[U];
                     take(q);
 #pragma unroll
@@ -279,7 +306,7 @@ namespace shamx {
                         cur[u] = id[u];
                         id[u]  = idn[u];
                     }
-                    if (t + 1 < T) {
+                    if (t + 1 < nt) {
                         request(idn);
                         load_ids(t + 2, idn);
                     }
@@ -349,12 +376,13 @@ namespace shamx {
             if constexpr (QUAD) {
                 // Passes per turn, the sweeps' cost with 1, 2, 4 (0.70 and 0.167 ms when each lane
                 // gathered its records): FP64, 2.1M Sedov 0.72, 0.62, 0.62 ms, 4M Plummer 0.325,
-                // 0.318, 0.345 ms on average; mixed, 1M disc 0.181, 0.157, 0.153 ms.  The address
+                // 0.318, 0.345 ms on average; mixed, 1M disc 0.181, 0.157, 0.150 ms (1.03M Sedov
+                // 0.34 to 0.25 ms).  The address
                 // units, busy 69 % of the time before, bound it no longer; what does is the VALU
                 // work of a pair (FP64: ordered sums, square root) at the 5 waves per SIMD that
                 // its registers leave, and latency.  The same fetch slows Omega (1.56 to 1.76 ms),
                 // whose LDS ring and registers leave no room for it.
-                using QP = QuadPos<MIXED ? 4 : 2>;
+                using QP = QuadRows<double4, MIXED ? 4 : 2>;
                 __shared__ __attribute__((aligned(16))) double2 room[BLK / WAVE][QP::ROOM];
                 const u32 k0 = work ? r.off[row] : 0u, len = work ? r.cnt[row] : 0u;
                 const QP rows(src.ps, room[wave_id()], r.ids, k0, len, row);
@@ -1341,7 +1369,11 @@ namespace shamx {
 
         // ------------------------------------------------------------- force (mixed)
         // r_ab and the neighbour criterion in FP64, pair terms in FP32, Kahan-compensated
-        // per-lane sums combined across the group in FP64
+        // per-lane sums combined across the group in FP64.  With four lanes per particle the
+        // records come as in QuadRows, two passes per turn (8 KB of LDS per wave: four waves per
+        // SIMD, as many as its registers leave).  Per evaluation, each lane gathering its own
+        // records / one pass per turn / two: 1.03M Sedov (M6) 728 / 643 / 576 us, 1M disc (M4)
+        // 496 / 469 / 432 us, 39k box (M8) 84 / 82 / 78 us.  Bound by VALU issue and latency.
         template<class K, int G, class Src>
         __global__ void __launch_bounds__(BLK)
             k_force_mixed(u32 n, Rows r, Src src, const f64 *__restrict h64, ForceOut o,
@@ -1356,9 +1388,13 @@ namespace shamx {
             f32 sx = 0, cx = 0, sy = 0, cy = 0, sz = 0, cz = 0, su = 0, cu = 0, vsig_max = 0;
             u32 row = 0, a = 0;
             f64 h_a64 = 0;
-            if (act) {
-                row = r.sel ? r.sel[j] : j;
-                a   = r.outi ? r.outi[row] : row;
+            constexpr bool QUAD = G == 4 && std::is_same<Src, RecSrc<FRec32>>::value;
+            using QP            = QuadRows<FRec32, 2>;
+            __shared__ __attribute__((aligned(16))) double2 room[QUAD ? BLK / WAVE : 1]
+                                                                [QUAD ? QP::ROOM : 1];
+            if (QUAD || act) {
+                if (act) row = r.sel ? r.sel[j] : j;
+                a = r.outi ? r.outi[row] : row;
                 const FRec32 A = src.get(row);
                 h_a64 = h64[a];
                 const f32 pmass = (f32) fa.mass;
@@ -1370,7 +1406,7 @@ namespace shamx {
                           alpha_u = (f32) fa.alpha_u;
                 const f32 c_du1 = omega_a_rho_a_inv * rho_a_inv * pmass;
                 const f64 ca = h_a64 * h_a64 * Rker2;
-                u32 k0 = r.off[row], k1 = k0 + r.cnt[row];
+                const u32 k0 = act ? r.off[row] : 0u, k1 = k0 + (act ? r.cnt[row] : 0u);
                 auto pair = [&](const FRec32 &B) {
                     f64 dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
                     f64 rab2 = dx * dx + dy * dy + dz * dz;
@@ -1406,6 +1442,12 @@ namespace shamx {
                     kahan_add(su, cu, t1 + t2);
                     vsig_max = fmaxf(vsig_max, cs_a + 2.f * abs_v);
                 };
+                if constexpr (QUAD) {
+                    const QP rows(src.rec, room[wave_id()], r.ids, k0, k1 - k0, row);
+                    rows.sweep([&](bool in, u32, const FRec32 &B) {
+                        if (in) pair(B);
+                    });
+                } else
                 // two records in flight, used in turn (no register copies between entries);
                 // loads past the row end read its last entry again (a cached line)
                 if (k0 < k1) {
