@@ -145,7 +145,9 @@ int shamx_tree_get(shamx_ctx *ctx, void *stream, uint32_t *sorted, uint32_t *sor
                    uint8_t *rflag, uint32_t *endrange, double *aabb_min, double *aabb_max,
                    double *rint);
 /* replaces NeighbourCache::start_neighbors_cache_2stages (NeighbourCache.cpp:222-604) on the
- * tree in ctx: neighbours of the first n_local particles among all tree objects */
+ * tree in ctx: neighbours of the first n_local particles among all tree objects.  A particle's
+ * owner leaf is the last one whose box contains the position passed here; error when none does
+ * (NaN, or moved out of every box since the boxes were made) */
 int shamx_neigh_build(shamx_ctx *ctx, void *stream, uint32_t n_local, const double *x,
                       const double *y, const double *z, const double *h, double htol,
                       double Rkern);

@@ -285,51 +285,93 @@ namespace shamx {
             xstart[l] = x;
         }
 
+        // the last leaf whose box contains p (is_coord_in_range_incl_max, geometry_utils.hpp:74-81),
+        // L when none does: the tiers right to left, entering the cells that contain p
+        __device__ inline bool box_holds(const f64 *__restrict rec, const double4 &p) {
+            return (rec[0] <= p.x) & (p.x <= rec[3]) & (rec[1] <= p.y) & (p.y <= rec[4]) &
+                   (rec[2] <= p.z) & (p.z <= rec[5]);
+        }
+        __device__ inline u32 last_leaf_holding(u32 L, u32 I, const f64 *__restrict nodes,
+                                                const f64 *__restrict tiers, const Tiers &tt,
+                                                const double4 &p) {
+            u32 t = tt.top, c = tt.n[tt.top] - 1;
+            for (;;) {
+                const f64 *rec = t ? tiers + (u64) (tt.off[t] + c) * NODE_F64
+                                   : nodes + (u64) (I + c) * NODE_F64;
+                if (box_holds(rec, p)) {
+                    if (t == 0) return c;
+                    t--;
+                    c = min(c * 8 + 7, tt.n[t] - 1);
+                    continue;
+                }
+                while (t < tt.top && c % 8 == 0) { // the first of its cell: on from that cell
+                    t++;
+                    c /= 8;
+                }
+                if (c == 0) return L;
+                c--;
+            }
+        }
+
         // Owner leaf (:406-451) of every local particle, OWN_LANES lanes per member batch (64
-        // sorted positions of a leaf).  The particle's own leaf contains it, so its owner is the
-        // last leaf of the own leaf's list whose box contains it (a leaf that contains a
-        // particle of this one meets its box and is in its list); leaves whose box no later leaf
-        // meets (lap) own all their particles.  Particles owned by another leaf go to mism.
-        // leaf_cap: as in stage 2.
-        constexpr u32 OWN_LANES = 16;
+        // sorted positions of a leaf): the last leaf whose box contains it.  When its own leaf does,
+        // that is the last leaf of the own leaf's list whose box contains it (a leaf that contains
+        // a particle of this one meets its box and is in its list, unless a reach below zero
+        // shrinks the box); leaves whose box no later leaf meets (lap) own all their particles.  A
+        // particle that its leaf's box does not contain (the caller moved it since the boxes were
+        // made) is searched for in the tiers; in no box: err bit 2.  Particles owned by another leaf
+        // go to mism, and lap is set for the leaf that keeps them.  leaf_cap: as in stage 2.
+        // Bound by memory latency.  Lanes 8 / 16: 2.1M Sedov (6 particles per leaf) 31 / 49 us, 4M
+        // Plummer 83 / 75 us, 1M disc 22 / 31 us.
+        constexpr u32 OWN_LANES = 8;
         __global__ void __launch_bounds__(256)
             k_owner(u32 n, u32 L, u32 I, const f64 *__restrict nodes,
+                    const f64 *__restrict tiers, Tiers tt,
                     const u32 *__restrict item_leaf, const u32 *__restrict xstart,
                     const u32 *__restrict n_extra,
                     const u32 *__restrict sort_index, const double4 *__restrict ps,
-                    const u32 *__restrict lap, const u32 *__restrict leaf_cnt,
+                    u32 *lap, const u32 *__restrict leaf_cnt,
                     const u32 *__restrict leaf_offset, const u32 *__restrict leaf_ids,
-                    u32 leaf_cap, u32 *__restrict owner, u32 *__restrict mism, u32 *__restrict mism_len) {
+                    u32 leaf_cap, u32 *__restrict owner, u32 *__restrict mism,
+                    u32 *__restrict mism_len, u32 *__restrict err) {
             const u32 item = (blockIdx.x * 256 + threadIdx.x) / OWN_LANES;
             if (item >= L + *n_extra) return;
-            const u32 l = item_leaf[item];
+            const u32 l = item < L ? item : item_leaf[item];
             u32 m0, m1;
             node_children(nodes, I + l, m0, m1);
             m0 += item_batch(item, l, L, xstart) * WAVE;
             m1 = min(m1, m0 + WAVE);
+            // (another lane of this leaf may set lap meanwhile: the search then finds the same)
             const bool over = lap[l] != 0;
+            const f64 *box  = nodes + (u64) (I + l) * NODE_F64;
             for (u32 s = m0 + threadIdx.x % OWN_LANES; s < m1; s += OWN_LANES) {
-                const u32 a = sort_index[s];
+                const u32 a     = sort_index[s];
+                const double4 p = ps[s];
                 if (a >= n) continue;
                 u32 own = l;
-                if (over) {
-                    const double4 p = ps[s];
-                    const u32 k0    = leaf_offset[l];
+                if (!(box_holds(box, p) & (box[6] >= 0))) {
+                    own = last_leaf_holding(L, I, nodes, tiers, tt, p);
+                    if (own >= L) {
+                        atomicOr(err, 2u);
+                        own = l;
+                    }
+                } else if (over) {
+                    const u32 k0 = leaf_offset[l];
                     u32 k = k0 + (leaf_cap ? min(leaf_cnt[l], leaf_cap) : leaf_cnt[l]);
                     while (k > k0) {
                         const u32 nd = leaf_ids[--k];
                         if (nd <= I + l) break;
-                        const f64 *rec = nodes + (u64) nd * NODE_F64;
-                        // is_coord_in_range_incl_max (geometry_utils.hpp:74-81)
-                        if ((rec[0] <= p.x) & (p.x <= rec[3]) & (rec[1] <= p.y) &
-                            (p.y <= rec[4]) & (rec[2] <= p.z) & (p.z <= rec[5])) {
+                        if (box_holds(nodes + (u64) nd * NODE_F64, p)) {
                             own = nd - I;
                             break;
                         }
                     }
                 }
                 owner[a] = own;
-                if (own != l) mism[atomicAdd(mism_len, 1u)] = a;
+                if (own != l) {
+                    mism[atomicAdd(mism_len, 1u)] = a;
+                    lap[l]                        = 1;
+                }
             }
         }
 
@@ -383,21 +425,18 @@ namespace shamx {
         }
 
         // sorted copy of positions and h (AoS, 32 B per object) + inverse permutation
-        // (sorted layout: with the row counts set to zero, the rows of images stay empty; a local
-        // particle with a NaN coordinate is inside no leaf box: err bit 2)
-        __global__ void k_sorted_copy(u32 nm, u32 n, const u32 *__restrict sort_index,
+        // (sorted layout: with the row counts set to zero, the rows of images stay empty)
+        __global__ void k_sorted_copy(u32 nm, const u32 *__restrict sort_index,
                                       const f64 *__restrict x, const f64 *__restrict y,
                                       const f64 *__restrict z, const f64 *__restrict h,
                                       double4 *__restrict ps, u32 *__restrict inv,
-                                      u32 *__restrict cnt, u32 *__restrict err) {
+                                      u32 *__restrict cnt) {
             u32 s = blockIdx.x * blockDim.x + threadIdx.x;
             if (s >= nm) return;
-            u32 b           = sort_index[s];
-            const double4 q = make_double4(x[b], y[b], z[b], h[b]);
-            ps[s]           = q;
-            inv[b]          = s;
+            u32 b  = sort_index[s];
+            ps[s]  = make_double4(x[b], y[b], z[b], h[b]);
+            inv[b] = s;
             if (cnt) cnt[s] = 0;
-            if ((b < n) & ((q.x != q.x) | (q.y != q.y) | (q.z != q.z))) atomicOr(err, 2u);
         }
 
         // Sorted layout: the sorted positions of the local particles in order (lpos; perm: the
@@ -835,10 +874,11 @@ namespace shamx {
         void owners(hipStream_t s, NeighBuffers &nb, const TreeBuffers &t, u32 n_local,
                     u32 gblocks, u32 leaf_cap) {
             k_owner<<<div_up((u64) gblocks * GRP_WAVES * OWN_LANES, 256), 256, 0, s>>>(
-                n_local, t.L, t.I, t.nodes.data(), nb.item_leaf.data(), nb.xstart.data(),
-                nb.counters.data() + 7, t.sort_index.data(), nb.ps.data(), nb.lap.data(),
-                nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(), leaf_cap,
-                nb.owner.data(), nb.mism.data(), nb.counters.data() + 5);
+                n_local, t.L, t.I, t.nodes.data(), t.tiers.data(), t.tt, nb.item_leaf.data(),
+                nb.xstart.data(), nb.counters.data() + 7, t.sort_index.data(), nb.ps.data(),
+                nb.lap.data(), nb.leaf_cnt.data(), nb.leaf_offset.data(), nb.leaf_ids.data(),
+                leaf_cap, nb.owner.data(), nb.mism.data(), nb.counters.data() + 5,
+                nb.counters.data() + 4);
         }
 
         // boxes of the member batches for the batch-level cull of stage 2, on sets whose tree
@@ -954,7 +994,6 @@ namespace shamx {
         nb.owner.resize(std::max<u32>(n_local, 1));
         nb.cnt.resize(std::max<u32>(rows, 1));
         nb.offset.resize(std::max<u32>(rows, 1));
-        u32 *err = nb.counters.data() + 4;
         fill_u32(s, nb.counters.data(), 0, 16);
         f64 Rker2 = Rkern * Rkern;
         u32 *hc = nb.host.data(); // 16 pinned words: the reads queue on the stream
@@ -963,10 +1002,9 @@ namespace shamx {
         nb.ps.resize(nm);
         nb.inv.resize(nm);
         nb.mism.resize(std::max<u32>(n_local, 1));
-        k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, n_local, t.sort_index.data(), x, y, z,
-                                                      h, nb.ps.data(), nb.inv.data(),
-                                                      sorted_layout ? nb.cnt.data() : nullptr,
-                                                      err);
+        k_sorted_copy<<<div_up(nm, 256), 256, 0, s>>>(nm, t.sort_index.data(), x, y, z, h,
+                                                      nb.ps.data(), nb.inv.data(),
+                                                      sorted_layout ? nb.cnt.data() : nullptr);
         const u32 gblocks = batch_items(s, nb, t);
 
         // leaf lists in two passes (count, scan, fill); returns once their length is known
