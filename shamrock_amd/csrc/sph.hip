@@ -1352,7 +1352,8 @@ namespace shamx {
             const f64 fx = facc, fy = group_lane<G, 1>(facc), fz = group_lane<G, 2>(facc),
                       tdu = group_lane<G, 3>(facc);
             vdot_max           = group_max<G>(vdot_max);
-            const f64 vsig_max = vdot_max < 0 ? 0. : 1.0 * A.cs + 2.0 * vdot_max;
+            // (0 where the sound speed is NaN, as a maximum that starts at 0 passes over NaN)
+            const f64 vsig_max = vdot_max < 0 ? 0. : fmax(0., 1.0 * A.cs + 2.0 * vdot_max);
             u64 key = ORDERED_POS_INF, npair = 0;
             if (act && lg == 0) {
                 const u32 a = r.outi[row];

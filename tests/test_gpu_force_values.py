@@ -1,0 +1,51 @@
+"""The force loop over the solver's rows against the general loop (SHAMX_PAIR_LANES=2) at values
+where an operation of its own could round or propagate otherwise.  The two have the same operations
+in the same order, so every output must keep its bits."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+from shamrock_amd import setups  # noqa: E402
+from shamrock_amd.solver import GpuSolver  # noqa: E402
+
+OUT = ("ax", "ay", "az", "du", "h")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu_ready():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+
+
+def _pass(cfg, f, monkeypatch, lanes):
+    with monkeypatch.context() as m:
+        if lanes:
+            m.setenv("SHAMX_PAIR_LANES", lanes)
+        g = GpuSolver(cfg, f)
+        log = g.density_force()
+        out = {k: g.get(k) for k in OUT} | {"vsig": g.get_f64(12, g.n), "cs": g.transient()["cs"]}
+        g.close()
+    return log, out
+
+
+def _same(cfg, f, monkeypatch):
+    (la, a), (lb, b) = (_pass(cfg, f, monkeypatch, v) for v in (None, "2"))
+    for k in ("n_interacting", "next_dt"):
+        assert la[k] == lb[k], k
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+    return a
+
+
+@pytest.mark.parametrize("kernel", ["M4", "M6"])
+def test_sound_speed_that_is_no_number(kernel, monkeypatch):
+    """A negative internal energy gives a negative pressure and a NaN sound speed; such a particle
+    has no signal speed above the maximum's start, 0 (the maximum passes over a NaN)."""
+    print(f"[force_values] nan cs {kernel}", flush=True)
+    cfg, f = setups.random_box(9**3, seed=4, kernel=kernel)
+    f["u"][::13] *= -1
+    out = _same(cfg, f, monkeypatch)
+    assert np.isnan(out["cs"]).any() and (out["vsig"][::13] == 0).all()
