@@ -184,10 +184,13 @@ namespace shamx {
             __device__ double3 pos(u32 b) const { return make_double3(x[b], y[b], z[b]); }
         };
 
-        // sqrt(v) correctly rounded for zero, infinity and 2^-767 < v (below, without the scaling
-        // of a general sqrt, its last bits; squared distances and P / rho ratios of a run are far
-        // above), and a value within an ulp or two of 1 / sqrt(v): the hardware estimate, one
-        // Newton step for both, two residual corrections of the root
+        // sqrt(v) correctly rounded for zero, infinity and 2^-767 < v, and an estimate of 1 / sqrt(v).
+        // Goldschmidt's iteration on the hardware's estimate (one step for root and reciprocal),
+        // then two residual corrections of the root (Markstein, IBM J. Res. Dev. 34(1), 1990;
+        // tests/test_root_identity.py).  A general square root scales its operand first; without
+        // that a root below 2^-383 loses its last bits.  A distance there is far below 1e-9, where
+        // the direction of a pair is taken as 0, and does not show beside h in a kernel; a
+        // ratio |dP| / rho there does not show beside any other term.
         __device__ inline f64 sqrt_pair(f64 v, f64 &recip) {
             const f64 r0 = __builtin_amdgcn_rsq(v);
             f64 s = v * r0, g = 0.5 * r0;
@@ -198,6 +201,16 @@ namespace shamx {
             s           = __builtin_fma(__builtin_fma(-s, s, v), g, s);
             recip       = g + g;
             return __builtin_amdgcn_class(v, 0x260) ? v : s; // +-0 and +inf: themselves
+        }
+        // RN(1 / y) from an estimate r (sqrt_pair's for y = its root; any within 2^-40).  Of two
+        // Newton corrections the first gives one of the two neighbours of 1 / y and the second
+        // rounds correctly (Markstein, 1990), unless the significand of y is all ones: 1 / y then
+        // lies just above a midpoint, and from the neighbour below the second one hits that
+        // midpoint and rounds to even.  The first one is turned up by 2^-64, which is more than its
+        // own error: near a midpoint it gives the neighbour above, from which all are right.
+        __device__ inline f64 rcp_of(f64 y, f64 r) {
+            r = __builtin_fma(__builtin_fma(-y, r, 1.) + 0x1p-64, r, r);
+            return __builtin_fma(__builtin_fma(-y, r, 1.), r, r);
         }
 
         // Rows of sorted records of 32 or 64 bytes, four lanes per particle.  A lane that gathers
@@ -1283,10 +1296,8 @@ namespace shamx {
                     const f64 rab2 = dx * dx + dy * dy + dz * dz;
                     f64 rc;
                     const f64 rab = sqrt_pair(rab2, rc);
-                    // 1 / rab from 1e-9 on, 0 below: two corrections make the estimate the
-                    // correctly rounded reciprocal
-                    rc             = __builtin_fma(__builtin_fma(-rab, rc, 1.), rc, rc);
-                    rc             = __builtin_fma(__builtin_fma(-rab, rc, 1.), rc, rc);
+                    // 1 / rab from 1e-9 on, 0 below
+                    rc             = rcp_of(rab, rc);
                     const f64 inv  = rab >= 1e-9 ? rc : 0.;
                     // dW = norm f'(r / h) / h^4 (sphkernels.hpp:2329-2343) and
                     // Fab_b / (rho_b omega_b) of the conductivity term, the divisions by way of

@@ -49,3 +49,22 @@ def test_sound_speed_that_is_no_number(kernel, monkeypatch):
     f["u"][::13] *= -1
     out = _same(cfg, f, monkeypatch)
     assert np.isnan(out["cs"]).any() and (out["vsig"][::13] == 0).all()
+
+
+@pytest.mark.parametrize("kernel", ["M4", "C2"])
+@pytest.mark.parametrize("k", [0, -1, 5, -20])
+def test_distances_of_all_ones(k, kernel, monkeypatch):
+    """Two square layers at the distance 2^k (1 - 2^-53), whose significand is all ones: the one
+    divisor that Newton's correction of a reciprocal leaves one ulp off (Markstein, 1990)."""
+    print(f"[force_values] all ones 2^{k} {kernel}", flush=True)
+    s, m = 2.0**k, 24
+    i, j, l = np.meshgrid([0.0, 1 - 2.0**-53], np.arange(m), np.arange(m), indexing="ij")
+    n = i.size
+    rng = np.random.default_rng(k + 100)
+    cfg, _ = setups.random_box(8, kernel=kernel, periodic=False)
+    cfg = dict(cfg, gpart_mass=s**3)
+    f = {"x": s * i.ravel(), "y": s * 1.25 * j.ravel(), "z": s * 1.5 * l.ravel(),
+         "h": np.full(n, 1.2 * s), "u": 1 + rng.random(n)}
+    f |= {c: rng.normal(0, 0.5, n) for c in ("vx", "vy", "vz")}
+    assert np.sqrt(f["x"].max() ** 2) == s * (1 - 2.0**-53)
+    _same(cfg, f, monkeypatch)
