@@ -49,6 +49,11 @@ namespace shamx {
             return !((alo[0] > bhi[0]) | (blo[0] > ahi[0]) | (alo[1] > bhi[1]) |
                      (blo[1] > ahi[1]) | (alo[2] > bhi[2]) | (blo[2] > ahi[2]));
         }
+        // a box that its reach r, below zero, shrinks past a point meets none
+        __device__ inline void close_shrunk(f64 r, f64 *lo, f64 *hi) {
+            if (r < 0 && ((lo[0] > hi[0]) | (lo[1] > hi[1]) | (lo[2] > hi[2])))
+                lo[0] = __builtin_inf(), hi[0] = -__builtin_inf();
+        }
 
         // One wave finds the lists of eight consecutive leaves (the targets).  Per tier it keeps a
         // first-in first-out queue in LDS of the cells that pass the criterion of the targets'
@@ -113,6 +118,9 @@ namespace shamx {
                     for (int k = 0; k < 3; k++) {
                         wide.lo[k] = c.lo[k] - r;
                         wide.hi[k] = c.hi[k] + r;
+                    }
+                    close_shrunk(r, wide.lo, wide.hi);
+                    for (int k = 0; k < 3; k++) {
                         m[k]       = c.lo[k];
                         m[3 + k]   = c.hi[k];
                         m[6 + k]   = wide.lo[k];
@@ -171,8 +179,9 @@ namespace shamx {
                 if (lane == 0) qh += n, qn -= n;
                 const Cell b = cell_load(nodes + (u64) (I + g) * NODE_F64);
                 const f64 r  = b.r * Rkern;
-                const f64 xlo[3] = {b.lo[0] - r, b.lo[1] - r, b.lo[2] - r};
-                const f64 xhi[3] = {b.hi[0] + r, b.hi[1] + r, b.hi[2] + r};
+                f64 xlo[3] = {b.lo[0] - r, b.lo[1] - r, b.lo[2] - r};
+                f64 xhi[3] = {b.hi[0] + r, b.hi[1] + r, b.hi[2] + r};
+                close_shrunk(r, xlo, xhi);
                 const bool later =
                     OUT != LEAF_FILL &&
                     __ballot(on & (g > g0 + t0) & boxes_meet(ulo, uhi, b.lo, b.hi)) != 0;

@@ -1,8 +1,8 @@
 /* Checks the square root and reciprocal of the HIP pair loops (sqrt_pair and rcp_of in
  * shamrock_amd/csrc/sph.hip) against sqrt and 1 / y: seeds of 1 / sqrt(v) with relative errors up
  * to 2^-22, operands that are random, squares, near powers of two, and squares of significands of
- * all ones, exponents in [-767, 1000].  Prints the mismatches of the roots, of the reciprocals, and of reciprocals by plain Newton corrections whose operand is
- * not of all ones. */
+ * all ones, exponents in [-767, 1000].  Prints the mismatches of the roots, of the reciprocals, and
+ * of reciprocals by plain Newton corrections whose operand is not of all ones. */
 #include <math.h>
 #include <stdint.h>
 #include <stdio.h>

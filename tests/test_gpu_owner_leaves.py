@@ -101,3 +101,31 @@ def test_outside_every_box_is_refused(n, level):
         _build(ctx, n, level, t, m)
     _build(ctx, n, level, t, t)  # the context is usable afterwards
     lib().shamx_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("size", [0.1, 0.3, 0.6, 1.0])
+@pytest.mark.parametrize("n,level", [(64, 0), (600, 1), (5000, 2), (5000, 4)])
+def test_reach_below_zero(n, level, size):
+    """Negative smoothing lengths shrink a leaf's box by its reach, to nothing where the reach is
+    more than half an edge: such a box meets none (BBAA::cella_neigh_b, geometry_utils.hpp:125-135).
+    Owners don't depend on the reach."""
+    print(f"[owner_leaves] reach n={n} level={level} size={size}", flush=True)
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0, 1, (n, 3))
+    h = rng.uniform(0.8, 1.2, n) * 0.5 * n ** (-1 / 3)
+    h[pos[:, 0] > 0.3] *= -size
+    t = _dev(pos, h)
+    ctx = C.c_void_p()
+    check(lib().shamx_ctx_create(C.byref(ctx)))
+    _build(ctx, n, level, t, t)
+    I, lo, hi, order, first, cnt, off, ids, own, lcnt, loff, lids = _read(ctx, n)
+    lib().shamx_ctx_destroy(ctx)
+    r = np.array([h[order[a:b]].max() for a, b in zip(first[:lo.shape[0]], first[1:])])[:, None]
+    r = r * HTOL * R
+    meet = lambda p, q, u, v: np.all(np.maximum(p, u) <= np.minimum(q, v), axis=-1)
+    for g in range(0, lo.shape[0], max(1, lo.shape[0] // 400)):
+        want = np.flatnonzero(meet(lo[g], hi[g], lo - r, hi + r) |
+                              meet(lo[g] - r[g], hi[g] + r[g], lo, hi))
+        np.testing.assert_array_equal(lids[loff[g]:loff[g] + lcnt[g]], I + want, err_msg=str(g))
+    for a in range(0, n, max(1, n // 1000)):
+        assert own[a] == np.flatnonzero(np.all((lo <= pos[a]) & (pos[a] <= hi), axis=1))[-1]
