@@ -48,7 +48,9 @@ namespace shamx {
     }
     constexpr f64 F64_BIG = 1.7976931348623157e308;
     __device__ inline Cell cell_none() {
-        return Cell{{F64_BIG, F64_BIG, F64_BIG}, {-F64_BIG, -F64_BIG, -F64_BIG}, -F64_BIG};
+        // (a reach of -inf: a leaf whose lengths are all NaN has it, and keeps it in its cells)
+        return Cell{{F64_BIG, F64_BIG, F64_BIG}, {-F64_BIG, -F64_BIG, -F64_BIG},
+                    -__builtin_inf()};
     }
     __device__ inline void cell_merge(Cell &c, const Cell &o) {
         for (int k = 0; k < 3; k++) {

@@ -129,3 +129,23 @@ def test_reach_below_zero(n, level, size):
         np.testing.assert_array_equal(lids[loff[g]:loff[g] + lcnt[g]], I + want, err_msg=str(g))
     for a in range(0, n, max(1, n // 1000)):
         assert own[a] == np.flatnonzero(np.all((lo <= pos[a]) & (pos[a] <= hi), axis=1))[-1]
+
+
+@pytest.mark.parametrize("n", [2, 65, 600])
+def test_cells_without_a_length(n):
+    """Lengths that are all NaN: the largest of a leaf starts at the type's lowest value, which
+    htol > 1 takes to -inf, and so it stays for every cell above."""
+    print(f"[owner_leaves] nan h n={n}", flush=True)
+    pos = np.random.default_rng(n).uniform(0, 1, (n, 3))
+    t = _dev(pos, np.full(n, np.nan))
+    ctx = C.c_void_p()
+    s = torch.cuda.current_stream().cuda_stream
+    check(lib().shamx_ctx_create(C.byref(ctx)))
+    check(lib().shamx_tree_build(ctx, s, n, *[a.data_ptr() for a in t], 0, HTOL))
+    sz = (C.c_uint32 * 4)()
+    check(lib().shamx_tree_sizes(ctx, sz))
+    r = torch.zeros(sz[1] + sz[2], dtype=torch.float64, device="cuda")
+    check(lib().shamx_tree_get(ctx, s, *[None] * 10, r.data_ptr()))
+    torch.cuda.synchronize()
+    lib().shamx_ctx_destroy(ctx)
+    np.testing.assert_array_equal(r.cpu().numpy(), -np.inf)
