@@ -444,8 +444,8 @@ namespace shamx {
         __global__ void __launch_bounds__(CT_BLK)
             k_reduc_compact(u32 n, const u32 *__restrict K_dev, const u32 *__restrict m,
                             const u32 *__restrict F, const u32 *__restrict tile_cnt, u32 nt,
-                            u32 *__restrict F_out, u32 *__restrict K_out,
-                            u32 *__restrict counters, u32 *__restrict host) {
+                            u32 *__restrict F_out, u32 *K_out, u32 *counters,
+                            u32 *__restrict host) {
             const u32 K = FIRST ? n : min(*K_dev, n);
             tile_compact<ITEMS>(
                 K, tile_cnt, nt, false,
@@ -455,7 +455,7 @@ namespace shamx {
                     *K_out = c;
                     if (!host) return;
                     // the last iteration: leaf count, distinct codes and the sorts' error words
-                    // to the host's pinned words
+                    // to the host's pinned words (K_out is one of the counters)
                     counters[0] = c;
                     host[0]     = c;
                     host[1]     = counters[1];
