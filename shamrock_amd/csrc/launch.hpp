@@ -207,7 +207,7 @@ namespace shamx {
         // ExternalForces.cpp:324-360) before the CFL criterion; null when there is none
         const f64 *ext_x = nullptr, *ext_y = nullptr, *ext_z = nullptr;
     };
-    // bytes of one force record (128 FP64, 64 mixed)
+    // bytes of one force record (144 FP64, 64 mixed)
     size_t force_record_bytes(int mixed);
     // EOS on nm merged particles fused with the force-record build; record s describes
     // particle perm[s].  P and cs are written per particle id; the images (ids from n on) take h,

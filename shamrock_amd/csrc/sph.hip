@@ -2324,7 +2324,11 @@ namespace shamx {
                             n, r,
                             SoASrc<KT, FRec32>{x, y, z, vx, vy, vz, h, omega, u, P, cs, fa.mass},
                             h, o, fa, part.data());
-                } else if (rec && G == 4) {
+                } else if (!rec) {
+                    k_force<KT, G><<<nb, BLK, 0, s>>>(
+                        n, r, SoASrc<KT, FRec>{x, y, z, vx, vy, vz, h, omega, u, P, cs, fa.mass},
+                        o, fa, part.data());
+                } else if constexpr (G == 4) {
                     // (the force rows' ids are below nm)
                     if ((u64) nm * sizeof(FRec) > 0xffffffffull)
                         k_force_rows<KT, true><<<nb, BLK, 0, s>>>(n, r, (const FRec *) rec, o, fa,
@@ -2333,14 +2337,8 @@ namespace shamx {
                         k_force_rows<KT, false><<<nb, BLK, 0, s>>>(n, r, (const FRec *) rec, o,
                                                                    fa, part.data());
                 } else {
-                    if (rec)
-                        k_force<KT, G><<<nb, BLK, 0, s>>>(
-                            n, r, RecSrc<FRec>{(const FRec *) rec}, o, fa, part.data());
-                    else
-                        k_force<KT, G><<<nb, BLK, 0, s>>>(
-                            n, r,
-                            SoASrc<KT, FRec>{x, y, z, vx, vy, vz, h, omega, u, P, cs, fa.mass}, o,
-                            fa, part.data());
+                    k_force<KT, G><<<nb, BLK, 0, s>>>(n, r, RecSrc<FRec>{(const FRec *) rec}, o,
+                                                      fa, part.data());
                 }
             });
         });
