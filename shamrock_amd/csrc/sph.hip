@@ -2072,6 +2072,12 @@ namespace shamx {
             int v         = e ? std::atoi(e) : 4;
             return (v == 1 || v == 2 || v == 4 || v == 16) ? v : 4;
         }
+        // SHAMX_WIDE_OFFSETS=1 (read at every call, for tests): the force rows' 64-bit record
+        // offsets below 4 GiB of records too
+        bool wide_offsets_forced() {
+            const char *e = std::getenv("SHAMX_WIDE_OFFSETS");
+            return e && std::atoi(e) == 1;
+        }
         template<class F>
         void dispatch_lanes(F &&f) {
             switch (pair_lanes()) {
@@ -2330,7 +2336,7 @@ namespace shamx {
                         o, fa, part.data());
                 } else if constexpr (G == 4) {
                     // (the force rows' ids are below nm)
-                    if ((u64) nm * sizeof(FRec) > 0xffffffffull)
+                    if ((u64) nm * sizeof(FRec) > 0xffffffffull || wide_offsets_forced())
                         k_force_rows<KT, true><<<nb, BLK, 0, s>>>(n, r, (const FRec *) rec, o, fa,
                                                                   part.data());
                     else

@@ -68,3 +68,25 @@ def test_distances_of_all_ones(k, kernel, monkeypatch):
     f |= {c: rng.normal(0, 0.5, n) for c in ("vx", "vy", "vz")}
     assert np.sqrt(f["x"].max() ** 2) == s * (1 - 2.0**-53)
     _same(cfg, f, monkeypatch)
+
+
+@pytest.mark.parametrize("kernel,side,av", [("M4", 5, 0), ("M4", 16, 1), ("M6", 17, 0),
+                                            ("M8", 11, 0), ("C2", 12, 0), ("C4", 13, 0),
+                                            ("C6", 13, 0)])
+def test_wide_offsets(kernel, side, av, monkeypatch):
+    """The force rows' 64-bit record offsets (sets of more than 29.8 M merged particles by
+    themselves) against the 32-bit ones: whole steps, every kernel, same bits."""
+    print(f"[force_values] wide {kernel} {side} av={av}", flush=True)
+    cfg, f = setups.random_box(side**3, seed=side, kernel=kernel)
+    cfg = dict(cfg, av_kind=av)
+    out = []
+    for wide in ("0", "1"):
+        monkeypatch.setenv("SHAMX_WIDE_OFFSETS", wide)
+        g = GpuSolver(cfg, f)
+        logs = [g.evolve_once() for _ in range(2)]
+        out.append(({k: g.get(k) for k in (*OUT, "x", "vx", "u")},
+                    [(m["n_interacting"], m["next_dt"], m["energy"]) for m in logs]))
+        g.close()
+    assert out[0][1] == out[1][1]
+    for k in out[0][0]:
+        np.testing.assert_array_equal(out[0][0][k], out[1][0][k], err_msg=k)
