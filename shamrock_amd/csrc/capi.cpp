@@ -252,7 +252,8 @@ struct shamx_solver {
     }
 
     // permute every per-particle field of the local particles into the sorted order of the
-    // last tree build (one gather per field; the images are rebuilt by the step anyway)
+    // last tree build (GATHER_MAX fields per launch, each into a temporary that takes its place;
+    // the images are rebuilt by the step anyway)
     void reorder_storage() {
         const bool go = pending_reorder();
         reo_known     = false;

@@ -127,7 +127,8 @@ namespace shamx {
         DevArray<unsigned char> scratch;
     };
     // NeighbourCache::start_neighbors_cache_2stages (NeighbourCache.cpp:222-604).
-    // Synchronises twice to size the leaf list and the particle list.
+    // Reference layout: synchronises twice, to size the leaf lists and the rows.  Sorted layout:
+    // once, for the counts past the rows' capacity (twice where leaf lists are known to overflow).
     void neigh_build(hipStream_t s, NeighBuffers &nb, TreeBuffers &t, u32 n_local,
                      const f64 *x, const f64 *y, const f64 *z, const f64 *h, f64 htol,
                      f64 Rkern, bool sorted_layout);

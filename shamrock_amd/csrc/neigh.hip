@@ -2,14 +2,17 @@
 //
 // neigh.hip -- two-stage neighbour cache (NeighbourCache::start_neighbors_cache_2stages,
 // shammodels/sph/src/modules/NeighbourCache.cpp:222-604).
-//   stage 1: per leaf, the list of interacting leaves (tree walk, :276-404)
+//   stage 1: per leaf, the list of interacting leaves (:276-404), by a search over the tiers of the
+//            leaves
 //   owner  : per local particle, the LAST leaf in depth-first order whose box contains it
 //            (inclusive max, :406-451)
 //   stage 2: per local particle, candidates of the owner's neighbour leaves kept when
 //            r_ab^2 <= max(rint_a, rint_b)^2 R^2 with rint = h * htol (:465-590)
-// Each list is built with a count pass, an exclusive scan and a fill pass that walks the same
-// candidates in the same order, so lists (and their order) are deterministic and identical to
-// the reference algorithm.  Traversal: KarrasTreeTraverser.hpp:69-118 (left child first).
+// The solver's lists are written in one pass into rows of fixed capacity, longer ones again into
+// an overflow region; the phase entry's (and rows that u32 indices cannot address that way) in a
+// count pass, a scan and a fill pass.  Either way a list holds its entries in the order of the
+// reference's walk, left child first (KarrasTreeTraverser.hpp:69-118), which is that of the leaf
+// index: lists and their order are deterministic and the reference's.
 #include "compact.hpp"
 #include "launch.hpp"
 #include "tree_layout.hpp"
@@ -71,12 +74,12 @@ namespace shamx {
         // target 30, so a group of T with box volume V against V1 and V2 of its halves splits
         // when (80 + 30 T) V > (80 + 15 T) (V1 + V2).
         //
-        // Bound by instruction issue (Sedov 128^3: 4280 VALU and 2720 scalar instructions per
-        // wave, 54 % of the VALU issue peak, 13 % of wave time waiting).  It replaces a
-        // depth-first walk of the binary tree shared by 64 leaves per wave, a chain of about
-        // 1000 dependent record loads.  Per build: Sedov 128^3 (391 k leaves) 1.39 -> 0.60 ms,
-        // disc of 1 M particles 4.05 -> 0.78 ms, Plummer sphere of 4.2 M 1.53 -> 0.66 ms,
-        // M8 box of 39 k 1.20 -> 0.09 ms, 1,728 particles 0.39 -> 0.04 ms; without the
+        // Bound by instruction issue (first steps of Sedov 128^3: 3410 VALU and 2010 scalar
+        // instructions per wave, 60 % of the VALU issue peak, 16 % of wave time waiting).  It
+        // replaces a depth-first walk of the binary tree shared by 64 leaves per wave, a chain of
+        // about 1000 dependent record loads.  Per build: Sedov 128^3 (391 k leaves) 1.54 -> 0.62 ms,
+        // disc of 1 M particles 4.06 -> 0.78 ms, Plummer sphere of 4.2 M 1.54 -> 0.68 ms,
+        // M8 box of 39 k 1.21 -> 0.09 ms, 1,728 particles 0.39 -> 0.04 ms; without the
         // halving of loose groups the first three take 1.87, 5.8 and 9.4 ms.
         //
         // COUNT: list lengths only.  ROWS: leaf g's list at ids[g * cap], at most cap entries

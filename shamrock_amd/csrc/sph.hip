@@ -1193,13 +1193,13 @@ namespace shamx {
         // Beside that it issues fewer instructions per pair: the rows need no criterion and no pair
         // count, one estimate serves |r_ab| and its reciprocal, the largest |v.r| stands for the
         // largest signal speed.
-        // Sedov 128^3 (M6, 230 M pairs): 2.71 -> 2.35 ms per evaluation; line accesses 52 -> 23 per
-        // load instruction, address units busy 69 -> 56 % of the time, waves waiting 51 -> 40 %,
-        // 236 -> 215 VALU instructions per wave and pass at 62 % of the issue peak, which with
+        // Sedov 128^3 (M6, 258 M pairs): 2.67 -> 2.44 ms per evaluation; line accesses 54 -> 23 per
+        // load instruction, address units busy 72 -> 59 % of the time, waves waiting 53 -> 42 %,
+        // 251 -> 232 VALU instructions per wave and pass at 58 % of the issue peak, which with
         // three waves per SIMD (LDS: 12 KB per wave) is what bounds it now.  Plummer sphere of
-        // 4.2 M (M4) 3.30 -> 3.0 ms, HCP lattice of 1.09 M 0.79 -> 0.67 ms.  Two lanes per
-        // particle, which need no fold room and let four waves fit: Plummer 3.8 ms; one lane:
-        // 6.8 ms.
+        // 4.2 M (M4) 3.39 -> 3.21 ms, HCP lattice of 1.09 M 0.80 -> 0.70 ms; 1,728 particles, where
+        // nothing hides the way through LDS, 17 -> 19 us.  Two lanes per particle, which need no
+        // fold room and let four waves fit: Plummer 3.8 ms; one lane: 6.8 ms.
         // WIDE: records past 4 GiB (29.8 M of them), 64-bit offsets.
         template<class K, bool WIDE>
         __global__ void __launch_bounds__(BLK)
@@ -1384,8 +1384,8 @@ namespace shamx {
         // per-lane sums combined across the group in FP64.  With four lanes per particle the
         // records come as in QuadRows, two passes per turn (8 KB of LDS per wave: four waves per
         // SIMD, as many as its registers leave).  Per evaluation, each lane gathering its own
-        // records / one pass per turn / two: 1.03M Sedov (M6) 728 / 643 / 576 us, 1M disc (M4)
-        // 496 / 469 / 432 us, 39k box (M8) 84 / 82 / 78 us.  Bound by VALU issue and latency.
+        // records / one pass per turn / two: 1.03M Sedov (M6) 734 / 643 / 574 us, 1M disc (M4)
+        // 519 / 469 / 431 us, 39k box (M8) 91 / 82 / 79 us.  Bound by VALU issue and latency.
         template<class K, int G, class Src>
         __global__ void __launch_bounds__(BLK)
             k_force_mixed(u32 n, Rows r, Src src, const f64 *__restrict h64, ForceOut o,
@@ -1547,7 +1547,7 @@ namespace shamx {
         //
         // Bound by its LDS traffic (32 16-byte accesses per lane and pass: 256 of the about 350
         // cycles that 64 pairs take on a CU) beside about 190 VALU instructions per pair.  HCP
-        // lattice of 1.09 M particles (M4, 62 M pairs): 0.69 ms, against 1.97 + 2.31 ms for one
+        // lattice of 1.09 M particles (M4, 62 M pairs): 0.72 ms, against 1.97 + 2.30 ms for one
         // lane per particle with all sums in registers and plain divisions, one kernel for the
         // first-order operators and one for d(div v)/dt; Sod tube (M6, 11 M pairs) 0.19 against
         // 0.37 + 0.49 ms.
@@ -2463,7 +2463,7 @@ namespace shamx {
                  part.data() + nb);
     }
 
-    // cut volumes are computed on the host exactly as find_interfaces does for one patch:
+    // cut volumes are computed (k_cut_boxes) exactly as find_interfaces does for one patch:
     // offset o = (xo, yo, zo) in lexicographic order without (0,0,0); interf volume =
     // sender box ∩ (receiver box expanded by int_range - offset); membership half-open.
     u32 periodic_ghosts(hipStream_t s, u32 n, f64 *x, f64 *y, f64 *z, f64 *h, const f64 *box6,

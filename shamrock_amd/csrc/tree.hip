@@ -15,7 +15,7 @@
 // Node records: every cell (I internal cells then L leaves) owns one 64-byte record
 //   [0..2] aabb min, [3..5] aabb max, [6] rint = max h * htol,
 //   [7]    internal: (left total id, right total id); leaf: (first, end) in sorted order
-// so a traversal step reads exactly one record.
+// so a cell is one 64-byte read.
 #include "compact.hpp"
 #include "launch.hpp"
 #include "tree_layout.hpp"
@@ -677,8 +677,10 @@ namespace shamx {
         }
 
         // Box and largest rint of every internal cell: the cell covers the leaves between its
-        // index and endrange, which are at most 14 cells per tier (the ragged ends of the range,
-        // then its whole cells one tier up).  min and max are exact, so any merge order gives the
+        // index and endrange, which are at most 14 cells per tier below the top (the ragged ends of
+        // the range, then its whole cells one tier up) and up to the top's 64, read one after the
+        // other: the root, and any cell of a tree of 64 leaves, takes that long.  min and max are
+        // exact, so any merge order gives the
         // same doubles.  It replaces a merge up the binary tree, eight launches over bands of
         // four levels after a depth pass: Sedov
         // 128^3 (391 k cells) 33 us against 100 us, 1,728 particles 11 us against 33 us, and nine
