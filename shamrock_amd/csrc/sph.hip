@@ -390,11 +390,10 @@ namespace shamx {
                 // Passes per turn, the sweeps' cost with 1, 2, 4 (0.70 and 0.167 ms when each lane
                 // gathered its records): FP64, 2.1M Sedov 0.72, 0.62, 0.62 ms, 4M Plummer 0.325,
                 // 0.318, 0.345 ms on average; mixed, 1M disc 0.181, 0.157, 0.150 ms (1.03M Sedov
-                // 0.34 to 0.25 ms).  The address
-                // units, busy 69 % of the time before, bound it no longer; what does is the VALU
-                // work of a pair (FP64: ordered sums, square root) at the 5 waves per SIMD that
-                // its registers leave, and latency.  The same fetch slows Omega (1.56 to 1.76 ms),
-                // whose LDS ring and registers leave no room for it.
+                // 0.34 to 0.25 ms).  Line accesses per load instruction 29 to 20 (FP64).  Bound by
+                // the VALU work of a pair (FP64: ordered sums, square root; 81 % of the issue peak)
+                // and latency, the address units busy 60 % of the time.  The same fetch slows Omega
+                // (1.56 to 1.76 ms), whose LDS ring and registers leave no room for it.
                 using QP = QuadRows<double4, MIXED ? 4 : 2>;
                 __shared__ __attribute__((aligned(16))) double2 room[BLK / WAVE][QP::ROOM];
                 const u32 k0 = work ? r.off[row] : 0u, len = work ? r.cnt[row] : 0u;
@@ -1183,7 +1182,7 @@ namespace shamx {
         // same order as k_force with four lanes per particle; what differs is how records come.
         //
         // A lane that gathers its own 144-byte record makes every load instruction of the wave
-        // touch 64 lines; the address units were busy 69 % of k_force's time and its waves
+        // touch 64 lines; the address units were busy 72 % of k_force's time and its waves
         // waited on them.  Here the four lanes of a particle fetch their four records together,
         // 64 contiguous bytes per instruction (nine instructions for the 36 pieces of 16 bytes),
         // straight into LDS, where lane l's pieces lie on different banks from its neighbours':
